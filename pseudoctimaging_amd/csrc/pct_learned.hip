@@ -1385,53 +1385,43 @@ __device__ __forceinline__ void pruned_step(const float* __restrict__ lds, int b
     for (int b = 0; b < NBA; ++b) ba[b] = b ? opaque(base + b * C::PPB * C::PS) : base;
 #pragma unroll
     for (int b = 0; b < NBL; ++b) bl[b] = opaque(base + C::LOFF + b * C::PPB * C::PS);
-    float ex[BZ + 2][BX];
+    float c[BZ][BX], ct[BZ][BX];
+    squared_sums_xz<BX, BZ>(
+        tv,
+        [&](int pz, int i) {
+            return lds[ba[pz / C::PPB] + (pz % C::PPB) * C::PS + i * C::CW];
+        },
+        c);
 #pragma unroll
-    for (int pz = 0; pz < BZ + 2; ++pz) {
-        float d[BX + 2];
-        const int pp = ba[pz / C::PPB] + (pz % C::PPB) * C::PS;
+    for (int j = 0; j < BZ; ++j)
 #pragma unroll
-        for (int i = 0; i < BX + 2; ++i) {
-            const float df = tv[pz][i] - lds[pp + i * C::CW];
-            d[i] = df * df;
-        }
+        for (int i = 0; i < BX; ++i)
+            ct[j][i] = lds[bl[j / C::PPB] + (j % C::PPB) * C::PS + (i + 1) * C::CW];
+    issue_first();
 #pragma unroll
-        for (int i = 0; i < BX; i += 2) {
-            const float q = d[i + 1] + d[i + 2];
-            ex[pz][i] = d[i] + q;
-            ex[pz][i + 1] = q + d[i + 3];
-        }
-    }
+    for (int j = 0; j < BZ; ++j)
 #pragma unroll
-    for (int j = 0; j < BZ; j += 2) {
+        for (int i = 0; i < BX; ++i)
+            c[j][i] = lane_next(c[j][i]) + (lane_prev(c[j][i]) + c[j][i]);
+#pragma unroll
+    for (int j = 0; j < BZ; ++j)
+#pragma unroll
+        for (int i = 0; i < BX; ++i) c[j][i] = __builtin_amdgcn_exp2f(-c[j][i]);
+    issue_paired();
+#pragma unroll
+    for (int j = 0; j < BZ; ++j)
 #pragma unroll
         for (int i = 0; i < BX; ++i) {
-            const float q = ex[j + 1][i] + ex[j + 2][i];
-            const float e0 = ex[j][i] + q;
-            const float e1 = q + ex[j + 3][i];
-            const float s0 = lane_next(e0) + (lane_prev(e0) + e0);
-            const float s1 = lane_next(e1) + (lane_prev(e1) + e1);
-            const float w0 = __builtin_amdgcn_exp2f(-s0);
-            const float w1 = __builtin_amdgcn_exp2f(-s1);
-            const float l0 = lds[bl[j / C::PPB] + (j % C::PPB) * C::PS + (i + 1) * C::CW];
-            const float l1 =
-                lds[bl[(j + 1) / C::PPB] + ((j + 1) % C::PPB) * C::PS + (i + 1) * C::CW];
-            P[j][i] = fmaf(w0, l0, P[j][i]);
-            S[j][i] += w0;
-            P[j + 1][i] = fmaf(w1, l1, P[j + 1][i]);
-            S[j + 1][i] += w1;
-            Le[j][i] += l0;
-            Le[j + 1][i] += l1;
-            if (SAMPLE) {
-                Ws[j][i] += w0;
-                Ws[j + 1][i] += w1;
-            }
+            const float w = c[j][i], l = ct[j][i];
+            P[j][i] = fmaf(w, l, P[j][i]);
+            S[j][i] += w;
+            Le[j][i] += l;
+            if (SAMPLE) Ws[j][i] += w;
             if (SAMPLE && ERR && j == 0 && i == 0) {
-                m.wl = fmaf(w0, l0, m.wl);
-                m.l1 += l0;
+                m.wl = fmaf(w, l, m.wl);
+                m.l1 += l;
             }
         }
-    }
 }
 
 template <int W, int BX, int BZ, int NW, int HW>

@@ -26,6 +26,25 @@ __device__ __forceinline__ float lane_next(float v) {
         float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x130, 0xf, 0xf, false));
 }
 
+// Wave priority around the instructions that a SIMD issues alone.  The SIMD of
+// a gfx950 CU issues plain FP32 adds, multiplies and FMAs of two waves at a
+// time (2.1-2.4 cycles each measured, against 4.3 for one wave), but a DPP add
+// (4.1 cycles) or an exp (8.3) only on its own.  With equal priorities the
+// oldest wave always issues, the other waves each come to stand before such an
+// instruction, and nothing is left to pair with the oldest wave's FMAs: a
+// stream of 30 FMAs, 8 DPP adds and 4 exps measured 4.47 cycles an instruction
+// with four waves, as if nothing paired.  A wave that raises its priority for
+// its DPP adds and exps gets through them between the others' FMAs, and the
+// FMAs of all waves pair: 2.95 cycles.
+__device__ __forceinline__ void issue_first() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+}
+__device__ __forceinline__ void issue_paired() {
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+}
+
 // Work items are dispatched round-robin over the 8 XCDs; give each XCD a
 // contiguous run of items so that tiles that share halos share an L2.
 __device__ __forceinline__ int xcd_contiguous(int b, int n) {
@@ -110,6 +129,36 @@ __device__ __forceinline__ int opaque(int v) {
     return v;
 }
 
+// Sums over x and z of the squared differences of a lane's block: c[j][i] is
+// the sum over planes j .. j+2 and rows i .. i+2 of (tv - a)^2, a(pz, row) the
+// atlas value.  The multiply-adds are written out, so that every kernel that
+// weighs squared differences rounds alike.
+template <int BX, int BZ, class Atlas>
+__device__ __forceinline__ void squared_sums_xz(const float (&tv)[BZ + 2][BX + 2], Atlas a,
+                                                float (&c)[BZ][BX]) {
+    float ex[BZ + 2][BX];
+#pragma unroll
+    for (int pz = 0; pz < BZ + 2; ++pz) {
+        float d[BX + 2];
+#pragma unroll
+        for (int i = 0; i < BX + 2; ++i) d[i] = tv[pz][i] - a(pz, i);
+#pragma unroll
+        for (int i = 0; i < BX; i += 2) {
+            const float q = fmaf(d[i + 2], d[i + 2], d[i + 1] * d[i + 1]);
+            ex[pz][i] = fmaf(d[i], d[i], q);
+            ex[pz][i + 1] = fmaf(d[i + 3], d[i + 3], q);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < BZ; j += 2)
+#pragma unroll
+        for (int i = 0; i < BX; ++i) {
+            const float q = ex[j + 1][i] + ex[j + 2][i];
+            c[j][i] = ex[j][i] + q;
+            c[j + 1][i] = q + ex[j + 3][i];
+        }
+}
+
 // All 2 HW + 1 dx candidates of one dy with squared differences.  `base` is
 // the LDS element index of plane 0, row 0 of the lane's window for dx = 0.
 // Candidate dx reads MRI rows dx .. dx + BX + 1, so consecutive candidates
@@ -138,49 +187,48 @@ __device__ __forceinline__ void tiled_dx_sweep(const float* __restrict__ lds, in
         for (int pz = 0; pz < BZ + 2; ++pz)
             rows[r][pz] = lds[ba[pz / C::PPBS] + (pz % C::PPBS) * C::PS + r * C::CW];
     };
+    float ct[2 * HW + BX][BZ];   // CT of candidate dx, output i: row dx + i
+    auto load_ct = [&](int r) {
 #pragma unroll
-    for (int r = 0; r < BX + 1; ++r) load_row(r);
+        for (int j = 0; j < BZ; ++j)
+            ct[r][j] = lds[bl[j / C::PPBS] + (j % C::PPBS) * C::PS + (r + 1) * C::CW];
+    };
+    float w[BZ][BX];
+    auto accumulate = [&](int dx) {
 #pragma unroll
-    for (int dx = 0; dx <= 2 * HW; ++dx) {
-        load_row(dx + BX + 1);
-        float ex[BZ + 2][BX];
-#pragma unroll
-        for (int pz = 0; pz < BZ + 2; ++pz) {
-            float d[BX + 2];
-#pragma unroll
-            for (int i = 0; i < BX + 2; ++i) {
-                const float df = tv[pz][i] - rows[dx + i][pz];
-                d[i] = df * df;
-            }
-#pragma unroll
-            for (int i = 0; i < BX; i += 2) {
-                const float q = d[i + 1] + d[i + 2];
-                ex[pz][i] = d[i] + q;
-                ex[pz][i + 1] = q + d[i + 3];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < BZ; j += 2) {
+        for (int j = 0; j < BZ; ++j)
 #pragma unroll
             for (int i = 0; i < BX; ++i) {
-                const float q = ex[j + 1][i] + ex[j + 2][i];
-                const float e0 = ex[j][i] + q;
-                const float e1 = q + ex[j + 3][i];
-                const float s0 = lane_next(e0) + (lane_prev(e0) + e0);
-                const float s1 = lane_next(e1) + (lane_prev(e1) + e1);
-                const float w0 = __builtin_amdgcn_exp2f(-s0);
-                const float w1 = __builtin_amdgcn_exp2f(-s1);
-                const float l0 =
-                    lds[bl[j / C::PPBS] + (j % C::PPBS) * C::PS + (dx + i + 1) * C::CW];
-                const float l1 = lds[bl[(j + 1) / C::PPBS] + ((j + 1) % C::PPBS) * C::PS +
-                                     (dx + i + 1) * C::CW];
-                P[j][i] = fmaf(w0, l0, P[j][i]);
-                S[j][i] += w0;
-                P[j + 1][i] = fmaf(w1, l1, P[j + 1][i]);
-                S[j + 1][i] += w1;
+                P[j][i] = fmaf(w[j][i], ct[dx + i][j], P[j][i]);
+                S[j][i] += w[j][i];
             }
+    };
+#pragma unroll
+    for (int r = 0; r < BX + 2; ++r) load_row(r);
+#pragma unroll
+    for (int r = 0; r < BX; ++r) load_ct(r);
+#pragma unroll
+    for (int dx = 0; dx <= 2 * HW; ++dx) {
+        if (dx < 2 * HW) load_row(dx + BX + 2);
+        float c[BZ][BX];
+        squared_sums_xz<BX, BZ>(tv, [&](int pz, int i) { return rows[dx + i][pz]; }, c);
+        if (dx > 0) {
+            accumulate(dx - 1);
+            load_ct(dx + BX - 1);
         }
+        issue_first();
+#pragma unroll
+        for (int j = 0; j < BZ; ++j)
+#pragma unroll
+            for (int i = 0; i < BX; ++i)
+                c[j][i] = lane_next(c[j][i]) + (lane_prev(c[j][i]) + c[j][i]);
+#pragma unroll
+        for (int j = 0; j < BZ; ++j)
+#pragma unroll
+            for (int i = 0; i < BX; ++i) w[j][i] = __builtin_amdgcn_exp2f(-c[j][i]);
+        issue_paired();
     }
+    accumulate(2 * HW);
 }
 
 // Staging loads read clamped positions (always inside the volume) and
@@ -611,12 +659,30 @@ __device__ __forceinline__ void xterm_dx_sweep(const unsigned (&b)[XtCfg<C>::NBS
             rows[r][2 * k + 1] = v.y;
         }
     };
+    f32x2 le[2 * HW + BX][BZ];   // (L~, E) of candidate dx, output i: row dx + i
+    auto load_le = [&](int r) {
 #pragma unroll
-    for (int r = 0; r < BX + 1; ++r) load_row(r);
+        for (int j = 0; j < BZ; ++j) le[r][j] = pair_at_sweep<C>(b, X::MPAIRS + j, (r + 1) * C::CW);
+    };
+    float w[BZ][BX];
+    auto accumulate = [&](int dx) {
+#pragma unroll
+        for (int j = 0; j < BZ; ++j)
+#pragma unroll
+            for (int i = 0; i < BX; ++i) {
+                P[j][i] = fmaf(w[j][i], le[dx + i][j].x, P[j][i]);
+                S[j][i] = fmaf(w[j][i], le[dx + i][j].y, S[j][i]);
+            }
+    };
+#pragma unroll
+    for (int r = 0; r < BX + 2; ++r) load_row(r);
+#pragma unroll
+    for (int r = 0; r < BX; ++r) load_le(r);
 #pragma unroll
     for (int dx = 0; dx <= 2 * HW; ++dx) {
-        load_row(dx + BX + 1);
-        float ex[BZ + 2][BX];
+        // paired part: sums over x and z, and the sums of the candidate before
+        if (dx < 2 * HW) load_row(dx + BX + 2);
+        float c[BZ][BX], ex[BZ + 2][BX];
 #pragma unroll
         for (int pz = 0; pz < BZ + 2; ++pz) {
 #pragma unroll
@@ -627,26 +693,32 @@ __device__ __forceinline__ void xterm_dx_sweep(const unsigned (&b)[XtCfg<C>::NBS
                 ex[pz][i + 1] = fmaf(t2[pz][i + 3], rows[dx + i + 3][pz], q);
             }
         }
+        if (dx > 0) {
+            accumulate(dx - 1);
+            load_le(dx + BX - 1);
+        }
 #pragma unroll
-        for (int j = 0; j < BZ; j += 2) {
+        for (int j = 0; j < BZ; j += 2)
 #pragma unroll
             for (int i = 0; i < BX; ++i) {
                 const float q = ex[j + 1][i] + ex[j + 2][i];
-                const float e0 = ex[j][i] + q;
-                const float e1 = q + ex[j + 3][i];
-                const float c0 = lane_next(e0) + (lane_prev(e0) + e0);
-                const float c1 = lane_next(e1) + (lane_prev(e1) + e1);
-                const float w0 = __builtin_amdgcn_exp2f(c0);
-                const float w1 = __builtin_amdgcn_exp2f(c1);
-                const f32x2 g0 = pair_at_sweep<C>(b, X::MPAIRS + j, (dx + i + 1) * C::CW);
-                const f32x2 g1 = pair_at_sweep<C>(b, X::MPAIRS + j + 1, (dx + i + 1) * C::CW);
-                P[j][i] = fmaf(w0, g0.x, P[j][i]);
-                S[j][i] = fmaf(w0, g0.y, S[j][i]);
-                P[j + 1][i] = fmaf(w1, g1.x, P[j + 1][i]);
-                S[j + 1][i] = fmaf(w1, g1.y, S[j + 1][i]);
+                c[j][i] = ex[j][i] + q;
+                c[j + 1][i] = q + ex[j + 3][i];
             }
-        }
+        // exclusive part: sums over y and the weights
+        issue_first();
+#pragma unroll
+        for (int j = 0; j < BZ; ++j)
+#pragma unroll
+            for (int i = 0; i < BX; ++i)
+                c[j][i] = lane_next(c[j][i]) + (lane_prev(c[j][i]) + c[j][i]);
+#pragma unroll
+        for (int j = 0; j < BZ; ++j)
+#pragma unroll
+            for (int i = 0; i < BX; ++i) w[j][i] = __builtin_amdgcn_exp2f(c[j][i]);
+        issue_paired();
     }
+    accumulate(2 * HW);
 }
 
 // One candidate of a slab the cross-term form cannot take (restaged with
@@ -987,8 +1059,15 @@ __device__ __forceinline__ void tiled_item_xt(const TiledArgs& args, int item,
     }
 }
 
+// Waves per SIMD the registers are kept for.  The 2 x 2 blocks' sweep needs 137
+// registers with the next row's loads in flight; held to 128, four waves stay
+// resident (the spills lie outside the sweep): 15.4 ms against 15.9 with three
+// waves at 222x222x112, n=10, NH=11.  LDS holds the larger blocks to two.
+constexpr int xt_min_waves(int bx, int bz) { return bx * bz <= 4 ? 4 : 2; }
+
 template <int W, int BX, int BZ, int NW, int HW>
-__global__ __launch_bounds__(NW * 64) void fuse_tiled_xt(TiledArgs args) {
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(
+    xt_min_waves(BX, BZ)))) void fuse_tiled_xt(TiledArgs args) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int item = xcd_contiguous(blockIdx.x, args.n_items);
     if (args.only && !args.only[item]) return;   // uniform over the workgroup
