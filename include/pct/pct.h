@@ -380,9 +380,9 @@ void pct_to_hu(float* arr, size_t n);
 int pct_postprocess(int nh, int nx, int ny, int nz, float* arr);
 
 /* Device versions of pct_regularize and pct_postprocess on a device volume,
- * enqueued on `stream`; bit-identical results.  The NaN fill visits the NaN
- * voxels in the reference's scan order, one at a time (cost grows with the
- * NaN count, not the volume).  Uses the library workspace.  Volumes of
+ * enqueued on `stream`; bit-identical results.  The NaN fill takes the NaN
+ * voxels in an order that gives the reference's scan-order values, many at a
+ * time (cost grows with the NaN-holding regions' extents).  Uses the library workspace.  Volumes of
  * nx*ny*nz >= 2^31 - 1 voxels return PCT_ERR_TOO_LARGE. */
 int pct_regularize_dev(int nh, int nx, int ny, int nz, float* d_arr, pct_stream_t stream);
 int pct_postprocess_dev(int nh, int nx, int ny, int nz, float* d_arr, pct_stream_t stream);

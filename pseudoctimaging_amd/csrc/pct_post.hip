@@ -15,15 +15,16 @@
 // voxels in increasing t, all voxels of one t at once, therefore gives the
 // sequential sweep's values bit for bit.
 //
-// (1) The interior NaN voxels are listed (per-chunk counts, a scan, a
-// compaction per chunk); (2) one workgroup runs the sweeps: a counting sort
-// of the list by t, then the levels in increasing t with a barrier after
-// each non-empty one, one voxel per thread (the median by stable ranks, the
-// std::stable_sort of cpp:1035, signed zeros included).  Voxels whose median
-// is still NaN form the next sweep's list; sweeps stop when no NaN is left
-// or a sweep fills nothing.  Rounding and the rescale are elementwise.
+// The first sweep runs in tiles over the whole chip (fill_tiles_kernel).  It
+// leaves NaN only where a voxel has no value around it at its turn; those
+// voxels go through the later sweeps in one workgroup (nan_fill_levels_kernel:
+// a counting sort of the list by t, then the levels in increasing t with a
+// barrier after each non-empty one, one voxel per thread), until none is left
+// or a sweep fills nothing.  Medians follow the std::stable_sort of cpp:1035,
+// signed zeros included.  Rounding and the rescale are elementwise.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <cmath>
 
@@ -31,106 +32,6 @@
 #include "pct_tiled.h"
 
 namespace pct {
-
-// Interior NaN voxels of `arr` in scan order (z, x, y; y fastest) into
-// list[0..*count), in three passes over chunks of kListChunk interior
-// positions (one block each): count per chunk, exclusive scan of the counts,
-// then an ordered compaction of every chunk at its offset.
-constexpr int kListThreads = 256;
-constexpr int kListChunk = 4096;
-
-__device__ __forceinline__ int interior_id(long long t, int lo, int ix, int iy, int nx, int ny) {
-    const int y = lo + (int)(t % iy);
-    const int x = lo + (int)((t / iy) % ix);
-    const int z = lo + (int)(t / ((long long)iy * ix));
-    return (z * nx + x) * ny + y;
-}
-
-__global__ __launch_bounds__(kListThreads) void nan_count_kernel(const float* __restrict__ arr,
-                                                                 int nx, int ny, int lo, int ix,
-                                                                 int iy, long long total,
-                                                                 int* __restrict__ bcount) {
-    __shared__ int wsum[kListThreads / 64];
-    const long long c0 = (long long)blockIdx.x * kListChunk;
-    int cnt = 0;
-    for (int k = threadIdx.x; k < kListChunk; k += kListThreads) {
-        const long long t = c0 + k;
-        if (t < total && isnan(arr[interior_id(t, lo, ix, iy, nx, ny)])) ++cnt;
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o);
-    if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = cnt;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int tot = 0;
-        for (int w = 0; w < kListThreads / 64; ++w) tot += wsum[w];
-        bcount[blockIdx.x] = tot;
-    }
-}
-
-// Exclusive scan of nb block counts into boff; the total into *count.
-__global__ __launch_bounds__(1024) void nan_scan_kernel(const int* __restrict__ bcount, int nb,
-                                                        int* __restrict__ boff,
-                                                        int* __restrict__ count) {
-    __shared__ int wtot[16];
-    const int seg = (nb + 1023) / 1024;
-    const int b0 = threadIdx.x * seg, b1 = min(nb, b0 + seg);
-    int own = 0;
-    for (int b = b0; b < b1; ++b) own += bcount[b];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    int incl = own;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int v = __shfl_up(incl, o);
-        if (lane >= o) incl += v;
-    }
-    if (lane == 63) wtot[w] = incl;
-    __syncthreads();
-    int before = 0;
-    for (int j = 0; j < w; ++j) before += wtot[j];
-    int run = before + incl - own;   // exclusive prefix of this thread's segment
-    for (int b = b0; b < b1; ++b) {
-        boff[b] = run;
-        run += bcount[b];
-    }
-    if (threadIdx.x == 1023) {
-        int tot = 0;
-        for (int j = 0; j < 16; ++j) tot += wtot[j];
-        *count = tot;
-    }
-}
-
-__global__ __launch_bounds__(kListThreads) void nan_write_kernel(const float* __restrict__ arr,
-                                                                 int nx, int ny, int lo, int ix,
-                                                                 int iy, long long total,
-                                                                 const int* __restrict__ boff,
-                                                                 int* __restrict__ list) {
-    __shared__ int wcnt[kListThreads / 64];
-    const long long c0 = (long long)blockIdx.x * kListChunk;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    int base = boff[blockIdx.x];
-    for (int r = 0; r < kListChunk; r += kListThreads) {
-        const long long t = c0 + r + threadIdx.x;
-        int id = 0;
-        bool isn = false;
-        if (t < total) {
-            id = interior_id(t, lo, ix, iy, nx, ny);
-            isn = isnan(arr[id]);
-        }
-        const unsigned long long bal = __ballot(isn);
-        if (lane == 0) wcnt[w] = __popcll(bal);
-        __syncthreads();
-        int off = base, tot = 0;
-#pragma unroll
-        for (int j = 0; j < kListThreads / 64; ++j) {
-            if (j < w) off += wcnt[j];
-            tot += wcnt[j];
-        }
-        if (isn) list[off + __popcll(bal & ((1ull << lane) - 1ull))] = id;
-        __syncthreads();   // wcnt is rewritten next round
-        base += tot;
-    }
-}
 
 constexpr int kFillThreads = 1024;
 
@@ -238,6 +139,423 @@ __device__ __forceinline__ float neighbourhood_median(const float* arr, int id, 
     if (cnt % 2 == 0) return (float)(((double)a + (double)b) / 2);
     return b;
 }
+
+// ---------------------------------------------------------------------------
+// first sweep: tiles in dependency order
+// ---------------------------------------------------------------------------
+//
+// With interior coordinates (z, x, y) and the skewed ones
+//     Z = z,  X = x + z,  Y = y + x + 2 z     (t = Z + X + Y up to a constant)
+// every neighbour before a voxel in scan order has no larger Z, X and Y, and
+// every one after it no smaller.  The skewed space is cut into tiles of kTZ x
+// kTX x kTY; tile (i, j, k) may run once the tiles of (i - {0,1}, j - {0,1},
+// k - {0,1}) that hold NaN voxels are done: what it reads of earlier voxels is
+// then final, and no later voxel it reads has changed, since those tiles wait
+// for this one.  A workgroup takes the next tile from a list ordered by i + j +
+// k, waits for the tiles before it, copies the tile and its halo into LDS as
+// order-preserving integer keys, and runs the tile's levels of t with a
+// workgroup barrier after each.  A tile is handed out only after all tiles it
+// waits for, to workgroups that are already running, so every wait ends.
+//
+// What bounds it is the chain of levels a value travels through (1108 at
+// 222x222x112) and, per tile on that chain, one hand-over between workgroups
+// (flag, LDS copy).  Hence small tiles, eight lanes to a voxel (about 130
+// instructions to a median instead of 900 for one lane sorting 27 values), and
+// an LDS copy that starts before the wait with what no tile before it changes.
+// A level takes about 810 cycles, the copy after the wait 1900, the release
+// 1700.  222x222x112 with 4.2e6 NaN voxels: 48.2 ms for the one-workgroup sweep
+// (46 us a level), 1.63 ms here, 1.52 of it in fill_tiles_kernel.  Tiles of
+// {4, 8, 32} took 2.7 ms (before the early copy), {4, 8, 8} 2.04, {8, 8, 8}
+// 2.22, {4, 16, 8} 2.56; 512 workgroups 1.70.  Polling with acquire loads,
+// which invalidate the caches each time, took 4.6-6.2 ms.
+constexpr int kTZ = 4, kTX = 8, kTY = 16;
+constexpr int kTileLanes = 8;                              // lanes per voxel
+constexpr int kTileThreads = kTZ * kTX * kTileLanes;       // one voxel per (Z, X) and level
+constexpr int kTileLevels = kTZ + kTX + kTY - 2;
+constexpr int kSZ = kTZ + 2, kSX = kTX + 4, kSY = kTY + 8; // with the halo
+constexpr int kStage = kSZ * kSX * kSY;
+// the staged elements: the tile and its halo after it (known before the tiles
+// before it are done), then the halo before it
+constexpr int kAfter = (kSZ - 1) * (kSX - 2) * (kSY - 4), kBefore = kStage - kAfter;
+constexpr int kAfterLoads = (kAfter + kTileThreads - 1) / kTileThreads;
+constexpr int kBeforeLoads = (kBefore + kTileThreads - 1) / kTileThreads;
+constexpr int kTileWgs = 256;                              // workgroups that take tiles
+static_assert(kTileLevels <= 32, "one mask bit per level");
+static_assert(kTX % 4 == 0 && kTY >= 4 && kTX >= 2 && kTZ >= 1, "neighbours lie in adjacent tiles");
+
+// The tiles that can hold interior voxels.  Row i spans X from kTZ i, and
+// (i, j) spans Y from kTZ i + kTX j, so j and k are counted from there.
+struct FillTiles {
+    int nx, ny, nz, lo;   // volume, first interior coordinate
+    int iz, ix, iy;       // interior extents
+    int ni, nj, nk;       // tiles per axis of the compact numbering
+    int n_tiles, n_diag;  // n_diag: bound of i + j + k
+};
+
+__host__ __device__ __forceinline__ int tile_j0(int i) { return kTZ * i / kTX; }
+__host__ __device__ __forceinline__ int tile_k0(int i, int j) { return (kTZ * i + kTX * j) / kTY; }
+
+__device__ __forceinline__ void tile_coords(const FillTiles& f, int tile, int* i, int* j, int* k) {
+    const int kk = tile % f.nk, ij = tile / f.nk;
+    *i = ij / f.nj;
+    *j = tile_j0(*i) + ij % f.nj;
+    *k = tile_k0(*i, *j) + kk;
+}
+
+// Index of tile (i, j, k), or -1 where it holds no interior voxel.
+__device__ __forceinline__ int tile_index(const FillTiles& f, int i, int j, int k) {
+    if (i < 0) return -1;
+    const int jj = j - tile_j0(i);
+    if (jj < 0 || jj >= f.nj) return -1;
+    const int kk = k - tile_k0(i, j);
+    if (kk < 0 || kk >= f.nk) return -1;
+    return (i * f.nj + jj) * f.nk + kk;
+}
+
+// Counters and the diagonals' histogram of one fill.
+struct FillState {
+    int* next;        // tiles handed out
+    int* n_busy;      // tiles with NaN voxels
+    int* left;        // voxels still NaN after the first sweep
+    int* done;        // [n_tiles] 1: nothing (more) to do
+    int* order;       // [n_tiles] busy tiles by diagonal
+    int* diag;        // [n_diag + 1] tiles per diagonal, then their places
+};
+
+__global__ void fill_clear_kernel(FillState st, int n_diag) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t <= n_diag) st.diag[t] = 0;
+    if (t == 0) *st.next = *st.n_busy = *st.left = 0;
+}
+
+// One wave per tile: whether it holds an interior NaN voxel.
+constexpr int kScanWaves = 4;
+__global__ __launch_bounds__(kScanWaves * 64) void fill_scan_kernel(
+    const float* __restrict__ arr, FillTiles f, FillState st) {
+    const int lane = threadIdx.x & 63;
+    const int tile = blockIdx.x * kScanWaves + (threadIdx.x >> 6);
+    if (tile >= f.n_tiles) return;   // per wave; no barrier below
+    int i, j, k;
+    tile_coords(f, tile, &i, &j, &k);
+    constexpr int kLoads = kTZ * kTX * kTY / 64;
+    bool nan = false;
+#pragma unroll 8
+    for (int q = 0; q < kLoads; ++q) {
+        const int e = q * 64 + lane;
+        const int Z = kTZ * i + e / (kTX * kTY), X = kTX * j + (e / kTY) % kTX,
+                  Y = kTY * k + e % kTY;
+        const int z = Z, x = X - Z, y = Y - X - Z;
+        const bool in = z < f.iz && x >= 0 && x < f.ix && y >= 0 && y < f.iy;
+        const long long id =
+            ((long long)(f.lo + z) * f.nx + (f.lo + x)) * f.ny + (f.lo + y);
+        const float v = arr[in ? id : 0];
+        nan |= in && isnan(v);
+    }
+    const bool busy = __ballot(nan) != 0;
+    if (lane == 0) {
+        st.done[tile] = busy ? 0 : 1;
+        if (busy) atomicAdd(st.diag + (i + j + k), 1);
+    }
+}
+
+// Places of the diagonals in the order list (exclusive prefix of the counts).
+__global__ __launch_bounds__(1024) void fill_places_kernel(FillState st, int n_diag) {
+    __shared__ int wtot[16];
+    const int seg = (n_diag + 1023) / 1024;
+    const int b0 = min(n_diag, (int)threadIdx.x * seg), b1 = min(n_diag, b0 + seg);
+    int own = 0;
+    for (int b = b0; b < b1; ++b) own += st.diag[b];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int incl = own;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(incl, o);
+        if (lane >= o) incl += v;
+    }
+    if (lane == 63) wtot[w] = incl;
+    __syncthreads();
+    int before = 0;
+    for (int j = 0; j < w; ++j) before += wtot[j];
+    int run = before + incl - own;
+    for (int b = b0; b < b1; ++b) {
+        const int c = st.diag[b];
+        st.diag[b] = run;
+        run += c;
+    }
+    if (threadIdx.x == 1023) *st.n_busy = before + incl;
+}
+
+// Busy tiles into the list by diagonal (any order within one).
+__global__ void fill_order_kernel(FillTiles f, FillState st) {
+    const int tile = blockIdx.x * blockDim.x + threadIdx.x;
+    if (tile >= f.n_tiles || st.done[tile]) return;
+    int i, j, k;
+    tile_coords(f, tile, &i, &j, &k);
+    st.order[atomicAdd(st.diag + (i + j + k), 1)] = tile;
+}
+
+// Lane exchanges within the eight lanes of a voxel.
+template <int CTRL>
+__device__ __forceinline__ int lane_swap(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+constexpr int kSwap1 = 0xB1;    // lane ^ 1 (quad_perm 1, 0, 3, 2)
+constexpr int kSwap2 = 0x4E;    // lane ^ 2 (quad_perm 2, 3, 0, 1)
+constexpr int kSwap3 = 0x1B;    // lane ^ 3 (quad_perm 3, 2, 1, 0)
+constexpr int kSwap7 = 0x141;   // lane ^ 7 (row_half_mirror)
+
+// The value of the lane before (within a row of 16).
+__device__ __forceinline__ int lane_before(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
+}
+
+__device__ __forceinline__ int med3i(int a, int b, int c) {
+    return max(min(a, b), min(max(a, b), c));
+}
+
+__device__ __forceinline__ void order2(int& a, int& b) {
+    const int mn = min(a, b);
+    b = max(a, b);
+    a = mn;
+}
+
+// Each lane keeps the smaller (bound INT_MIN) or the larger (INT_MAX) of its
+// slots and another lane's: slot s against slot s, or against 3 - s (REV).
+template <int CTRL, bool REV>
+__device__ __forceinline__ void lane_split(int (&k)[4], int bound) {
+    int o[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) o[s] = lane_swap<CTRL>(k[REV ? 3 - s : s]);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) k[s] = med3i(k[s], o[s], bound);
+}
+
+// Sorts a lane's four slots when they form a bitonic sequence.
+__device__ __forceinline__ void bitonic4(int (&k)[4]) {
+    order2(k[0], k[2]);
+    order2(k[1], k[3]);
+    order2(k[0], k[1]);
+    order2(k[2], k[3]);
+}
+
+// Sorts the 32 keys of eight lanes: afterwards lane q holds ranks 4 q .. 4 q + 3.
+// b1, b2, b4: INT_MIN where bit 0, 1, 2 of the lane is 0, else INT_MAX.
+__device__ __forceinline__ void sort8x4(int (&k)[4], int b1, int b2, int b4) {
+    order2(k[0], k[1]);
+    order2(k[2], k[3]);
+    order2(k[0], k[2]);
+    order2(k[1], k[3]);
+    order2(k[1], k[2]);
+    lane_split<kSwap1, true>(k, b1);
+    bitonic4(k);
+    lane_split<kSwap3, true>(k, b2);
+    lane_split<kSwap1, false>(k, b1);
+    bitonic4(k);
+    lane_split<kSwap7, true>(k, b4);
+    lane_split<kSwap2, false>(k, b2);
+    lane_split<kSwap1, false>(k, b1);
+    bitonic4(k);
+}
+
+__global__ __launch_bounds__(kTileThreads) void fill_tiles_kernel(float* arr, FillTiles f,
+                                                                  FillState st, int* left_list) {
+    __shared__ int key[kStage];
+    __shared__ int s_ticket;
+    __shared__ unsigned s_levels;      // levels of the tile with NaN voxels
+    __shared__ int s_neg_zero;         // a -0 may occur in the tile
+    const int tid = threadIdx.x;
+    const int q = tid & (kTileLanes - 1), v = tid / kTileLanes;
+    const int vz = v / kTX, vx = v % kTX;
+    const int b1 = (q & 1) ? INT_MAX : INT_MIN, b2 = (q & 2) ? INT_MAX : INT_MIN,
+              b4 = (q & 4) ? INT_MAX : INT_MIN;
+    // LDS offsets of the lane's neighbours q, q + 8, ... of the 27 (the last
+    // slot of lanes 3 .. 7 is empty: none_if raises it to INT_MAX)
+    auto offset = [](int n) {
+        const int dz = n / 9 - 1, dx = (n / 3) % 3 - 1, dy = n % 3 - 1;
+        return (dz * kSX + (dx + dz)) * kSY + dy + dx + 2 * dz;
+    };
+    int off[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) off[s] = opaque(offset(min(q + 8 * s, 26)));
+    const int none_if = q < 3 ? INT_MIN : INT_MAX;
+    // the staged elements of the thread, as (sz, sx, sy) packed in bytes, -1
+    // for none; element (0, 0, 0) lies at Z - 1, X - 2, Y - 4 of the tile's origin
+    int after[kAfterLoads], before[kBeforeLoads];
+    auto pack = [](int sz, int sx, int sy) { return (sz << 16) | (sx << 8) | sy; };
+#pragma unroll
+    for (int l = 0; l < kAfterLoads; ++l) {
+        const int e = tid + l * kTileThreads;
+        constexpr int W = kSY - 4, H = kSX - 2;
+        after[l] = e < kAfter ? pack(1 + e / (H * W), 2 + (e / W) % H, 4 + e % W) : -1;
+    }
+#pragma unroll
+    for (int l = 0; l < kBeforeLoads; ++l) {
+        // plane sz = 0, then rows sx < 2, then columns sy < 4
+        int e = tid + l * kTileThreads;
+        int c = -1;
+        if (e < kSX * kSY) {
+            c = pack(0, e / kSY, e % kSY);
+        } else if ((e -= kSX * kSY) < (kSZ - 1) * 2 * kSY) {
+            c = pack(1 + e / (2 * kSY), (e / kSY) % 2, e % kSY);
+        } else if ((e -= (kSZ - 1) * 2 * kSY) < (kSZ - 1) * (kSX - 2) * 4) {
+            c = pack(1 + e / ((kSX - 2) * 4), 2 + (e / 4) % (kSX - 2), e % 4);
+        }
+        before[l] = c;
+    }
+    const int n_busy = *st.n_busy;
+    for (;;) {
+        __syncthreads();   // the previous tile is done with the shared state
+        if (tid == 0) {
+            s_ticket = atomicAdd(st.next, 1);
+            s_levels = 0;
+            s_neg_zero = 0;
+        }
+        __syncthreads();
+        const int ticket = __builtin_amdgcn_readfirstlane(s_ticket);
+        if (ticket >= n_busy) return;   // uniform; every tile has been handed out
+        const int tile = st.order[ticket];
+        int i, j, k;
+        tile_coords(f, tile, &i, &j, &k);
+        // volume coordinates of element (0, 0, 0)
+        const int Z0 = kTZ * i - 1, X0 = kTX * j - 2, Y0 = kTY * k - 4;
+        auto load = [&](int c, bool* in) {
+            const int Z = Z0 + (c >> 16), X = X0 + ((c >> 8) & 255), Y = Y0 + (c & 255);
+            const int z = f.lo + Z, x = f.lo + X - Z, y = f.lo + Y - X - Z;
+            *in = c >= 0 && (unsigned)z < (unsigned)f.nz && (unsigned)x < (unsigned)f.nx &&
+                  (unsigned)y < (unsigned)f.ny;
+            return arr[*in ? ((long long)z * f.nx + x) * f.ny + y : 0];
+        };
+        bool neg = false;
+        auto store = [&](int c, bool in, float v) {   // INT_MAX: NaN or outside the volume
+            const int kv = in && !isnan(v) ? float_key(v) : INT_MAX;
+            neg |= kv == -1;
+            if (c >= 0) key[((c >> 16) * kSX + ((c >> 8) & 255)) * kSY + (c & 255)] = kv;
+            return kv;
+        };
+        {
+            float raw[kAfterLoads];
+            bool in[kAfterLoads];
+#pragma unroll
+            for (int l = 0; l < kAfterLoads; ++l) raw[l] = load(after[l], &in[l]);
+            unsigned levels = 0;
+#pragma unroll
+            for (int l = 0; l < kAfterLoads; ++l) {
+                const int c = after[l];
+                const int kv = store(c, in[l], raw[l]);
+                const int zl = (c >> 16) - 1, xl = ((c >> 8) & 255) - 2, yl = (c & 255) - 4;
+                const int Z = kTZ * i + zl, X = kTX * j + xl, Y = kTY * k + yl;
+                const int x = X - Z, y = Y - X - Z;
+                if (in[l] && kv == INT_MAX && zl < kTZ && xl < kTX && yl < kTY && Z < f.iz &&
+                    x >= 0 && x < f.ix && y >= 0 && y < f.iy)
+                    levels |= 1u << (zl + xl + yl);
+            }
+            if (levels) atomicOr(&s_levels, levels);
+        }
+        if (tid >= 1 && tid < 8) {
+            const int p = tile_index(f, i - (tid & 1), j - ((tid >> 1) & 1), k - (tid >> 2));
+            if (p >= 0)
+                while (__hip_atomic_load(st.done + p, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT) == 0)
+                    __builtin_amdgcn_s_sleep(1);
+        }
+        // one acquire after the waits, by the wave that waited (an acquire in
+        // the loop would invalidate the caches at every poll)
+        if (tid < 64) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        __syncthreads();
+        {
+            float raw[kBeforeLoads];
+            bool in[kBeforeLoads];
+#pragma unroll
+            for (int l = 0; l < kBeforeLoads; ++l) raw[l] = load(before[l], &in[l]);
+#pragma unroll
+            for (int l = 0; l < kBeforeLoads; ++l) store(before[l], in[l], raw[l]);
+        }
+        if (neg) s_neg_zero = 1;
+        __syncthreads();
+
+        // the lane's voxel at level l is (vz, vx, l - vz - vx); y runs over
+        // the interior for local Y in [y_lo, y_hi)
+        const int Z = kTZ * i + vz, X = kTX * j + vx;
+        const int x = X - Z;
+        const bool row_in = Z < f.iz && x >= 0 && x < f.ix;
+        const int y_base = X + Z - kTY * k;   // local Y of interior y = 0
+        const int y_lo = max(0, y_base), y_hi = row_in ? min(kTY, y_base + f.iy) : 0;
+        const long long row_id =
+            ((long long)(f.lo + Z) * f.nx + (f.lo + x)) * f.ny + f.lo - y_base;
+        const int* const row_key = key + ((vz + 1) * kSX + vx + 2) * kSY + 4;
+        unsigned todo = (unsigned)__builtin_amdgcn_readfirstlane((int)s_levels);
+        while (todo) {   // uniform
+            const int l = __builtin_ctz(todo);
+            todo &= todo - 1;
+            const int yl = l - vz - vx;
+            const int* const at = row_key + min(max(yl, 0), kTY - 1);
+            const int centre = at[0];
+            int kk[4];
+#pragma unroll
+            for (int s = 0; s < 4; ++s) kk[s] = at[off[s]];
+            kk[3] = max(kk[3], none_if);
+            const bool valid = yl >= y_lo && yl < y_hi && centre == INT_MAX;
+            if (__ballot(valid)) {   // uniform over the wave
+                int cnt = 0;
+#pragma unroll
+                for (int s = 0; s < 4; ++s) cnt += kk[s] != INT_MAX ? 1 : 0;
+                cnt += lane_swap<kSwap1>(cnt);
+                cnt += lane_swap<kSwap2>(cnt);
+                cnt += lane_swap<kSwap7>(cnt);
+                sort8x4(kk, b1, b2, b4);
+                // the lane that holds rank cnt / 2 (slot hs) forms the median:
+                // the rank before it is its slot before, or the last of the
+                // lane before
+                const int hi = cnt >> 1, hs = hi & 3;
+                const int prev = lane_before(kk[3]);
+                const int kb = hs & 2 ? (hs & 1 ? kk[3] : kk[2]) : (hs & 1 ? kk[1] : kk[0]);
+                const int ka = hs & 2 ? (hs & 1 ? kk[2] : kk[1]) : (hs & 1 ? kk[0] : prev);
+                const float b = __int_as_float(float_key(__int_as_float(kb)));
+                const float a = __int_as_float(float_key(__int_as_float(ka)));
+                float res = (cnt & 1) ? b : (float)(((double)a + (double)b) / 2);
+                if (s_neg_zero) {   // -0 and +0 may meet: the stable ranks decide
+                    float ra = 0.f, rb = 0.f;
+#pragma unroll 1
+                    for (int m = 0; m < 27; ++m) {
+                        const int km = at[offset(m)];
+                        if (km == INT_MAX) continue;
+                        const float fm = __int_as_float(float_key(__int_as_float(km)));
+                        int rank = 0;
+#pragma unroll 1
+                        for (int n = 0; n < 27; ++n) {
+                            const int kn = at[offset(n)];
+                            const float fn = __int_as_float(float_key(__int_as_float(kn)));
+                            rank += kn != INT_MAX && (fn < fm || (fn == fm && n < m)) ? 1 : 0;
+                        }
+                        if (rank == hi) rb = fm;
+                        if (rank == hi - 1) ra = fm;
+                    }
+                    res = (cnt & 1) ? rb : (float)(((double)ra + (double)rb) / 2);
+                }
+                if (valid && q == (hi >> 2)) {
+                    if (cnt == 0) res = __builtin_nanf("");
+                    const long long id = row_id + yl;
+                    arr[id] = res;
+                    if (isnan(res)) {   // no value around it, or infinities of both signs
+                        left_list[atomicAdd(st.left, 1)] = (int)id;
+                    } else {
+                        const int rk = float_key(res);
+                        key[at - key] = rk;
+                        if (rk == -1) s_neg_zero = 1;
+                    }
+                }
+            }
+            __syncthreads();
+        }
+        __syncthreads();   // every wave's values come before the release
+        if (tid == 0)
+            __hip_atomic_store(st.done + tile, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// the other sweeps
+// ---------------------------------------------------------------------------
 
 // The sweeps of RegularizationStep over the listed voxels, in one workgroup.
 // hist has t_count + 1 ints; sorted and the lists hold `interior` ints.
@@ -368,41 +686,77 @@ static long long fill_levels(int nx, int ny, int nz) {
     return 4LL * (nz - 1) + 2LL * (nx - 1) + (ny - 1) + 1;
 }
 
-// Workspace of the NaN fill: a counter, three voxel lists (two sweeps' and
-// the sorted one), per-chunk counts and offsets, and the level histogram.
-static size_t fill_ws_bytes(long long interior, long long levels) {
-    const size_t list_bytes = ((size_t)interior * 4 + 255) & ~(size_t)255;
-    const long long nb = (interior + kListChunk - 1) / kListChunk;
-    const size_t block_bytes = ((size_t)nb * 4 + 255) & ~(size_t)255;
-    const size_t hist_bytes = ((size_t)(levels + 1) * 4 + 255) & ~(size_t)255;
-    return 256 + 3 * list_bytes + 2 * block_bytes + hist_bytes;
+// The fill's tiles (a volume below 2^31 voxels with interior voxels).
+static FillTiles fill_tiles(int nh, int nx, int ny, int nz) {
+    FillTiles f;
+    f.nx = nx;
+    f.ny = ny;
+    f.nz = nz;
+    f.lo = (nh - 1) / 2 + 1;
+    f.iz = nz - 2 * f.lo;
+    f.ix = nx - 2 * f.lo;
+    f.iy = ny - 2 * f.lo;
+    f.ni = (f.iz + kTZ - 1) / kTZ;
+    f.nj = (kTZ + f.ix - 2) / kTX + 2;
+    f.nk = (kTZ + kTX + f.iy - 3) / kTY + 2;
+    f.n_tiles = f.ni * f.nj * f.nk;
+    const int j_end = tile_j0(f.ni - 1) + f.nj;
+    f.n_diag = f.ni + j_end + tile_k0(f.ni - 1, j_end) + f.nk;
+    return f;
+}
+
+// Workspace of the NaN fill: counters, three voxel lists (two sweeps' and the
+// sorted one), the level histogram, the tiles' states and order, and the
+// diagonals' histogram.
+struct FillLayout {
+    size_t list, hist, done, order, diag, bytes;
+};
+static FillLayout fill_layout(int nh, int nx, int ny, int nz) {
+    auto align = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    const long long interior = fill_interior(nh, nx, ny, nz);
+    FillLayout w{};
+    w.list = align((size_t)interior * 4);
+    w.hist = 256 + 3 * w.list;
+    w.done = w.hist + align((size_t)(fill_levels(nx, ny, nz) + 1) * 4);
+    if (!interior) {
+        w.bytes = w.done;
+        return w;
+    }
+    const FillTiles f = fill_tiles(nh, nx, ny, nz);
+    w.order = w.done + align((size_t)f.n_tiles * 4);
+    w.diag = w.order + align((size_t)f.n_tiles * 4);
+    w.bytes = w.diag + align((size_t)(f.n_diag + 1) * 4);
+    return w;
 }
 
 static int enqueue_fill(int nh, int nx, int ny, int nz, float* d_arr, void* ws, hipStream_t s) {
-    const int lo = (nh - 1) / 2 + 1;
-    const long long ix = nx - 2 * lo, iy = ny - 2 * lo;
-    const long long interior = fill_interior(nh, nx, ny, nz);
-    if (interior == 0) return PCT_OK;
-    const size_t list_bytes = ((size_t)interior * 4 + 255) & ~(size_t)255;
-    const long long nb = (interior + kListChunk - 1) / kListChunk;
-    const size_t block_bytes = ((size_t)nb * 4 + 255) & ~(size_t)255;
+    if (fill_interior(nh, nx, ny, nz) == 0) return PCT_OK;
+    const FillLayout lay = fill_layout(nh, nx, ny, nz);
+    const FillTiles f = fill_tiles(nh, nx, ny, nz);
     char* w = static_cast<char*>(ws);
-    int* count = reinterpret_cast<int*>(w);
+    int* counters = reinterpret_cast<int*>(w);
     int* la = reinterpret_cast<int*>(w + 256);
-    int* lb = reinterpret_cast<int*>(w + 256 + list_bytes);
-    int* srt = reinterpret_cast<int*>(w + 256 + 2 * list_bytes);
-    int* bcount = reinterpret_cast<int*>(w + 256 + 3 * list_bytes);
-    int* boff = reinterpret_cast<int*>(w + 256 + 3 * list_bytes + block_bytes);
-    int* hist = reinterpret_cast<int*>(w + 256 + 3 * list_bytes + 2 * block_bytes);
-    const long long levels = fill_levels(nx, ny, nz);
-    const int ixi = (int)ix, iyi = (int)iy;
-    hipLaunchKernelGGL(nan_count_kernel, dim3((unsigned)nb), dim3(kListThreads), 0, s, d_arr, nx,
-                       ny, lo, ixi, iyi, interior, bcount);
-    hipLaunchKernelGGL(nan_scan_kernel, dim3(1), dim3(1024), 0, s, bcount, (int)nb, boff, count);
-    hipLaunchKernelGGL(nan_write_kernel, dim3((unsigned)nb), dim3(kListThreads), 0, s, d_arr, nx,
-                       ny, lo, ixi, iyi, interior, boff, la);
+    int* lb = reinterpret_cast<int*>(w + 256 + lay.list);
+    int* srt = reinterpret_cast<int*>(w + 256 + 2 * lay.list);
+    int* hist = reinterpret_cast<int*>(w + lay.hist);
+    FillState st;
+    st.next = counters;
+    st.n_busy = counters + 16;
+    st.left = counters + 32;
+    st.done = reinterpret_cast<int*>(w + lay.done);
+    st.order = reinterpret_cast<int*>(w + lay.order);
+    st.diag = reinterpret_cast<int*>(w + lay.diag);
+    hipLaunchKernelGGL(fill_clear_kernel, dim3((unsigned)(f.n_diag / 256 + 1)), dim3(256), 0, s,
+                       st, f.n_diag);
+    hipLaunchKernelGGL(fill_scan_kernel, dim3((unsigned)((f.n_tiles + kScanWaves - 1) / kScanWaves)),
+                       dim3(kScanWaves * 64), 0, s, d_arr, f, st);
+    hipLaunchKernelGGL(fill_places_kernel, dim3(1), dim3(1024), 0, s, st, f.n_diag);
+    hipLaunchKernelGGL(fill_order_kernel, dim3((unsigned)((f.n_tiles + 255) / 256)), dim3(256), 0,
+                       s, f, st);
+    hipLaunchKernelGGL(fill_tiles_kernel, dim3((unsigned)std::min(f.n_tiles, kTileWgs)),
+                       dim3(kTileThreads), 0, s, d_arr, f, st, la);
     hipLaunchKernelGGL(nan_fill_levels_kernel, dim3(1), dim3(kFillThreads), 0, s, d_arr, la, lb,
-                       srt, hist, count, nx, ny, (int)levels, (int*)nullptr);
+                       srt, hist, st.left, nx, ny, (int)fill_levels(nx, ny, nz), (int*)nullptr);
     return hipGetLastError() == hipSuccess ? PCT_OK : PCT_ERR_HIP;
 }
 
@@ -414,7 +768,7 @@ static int enqueue_fill_lib(int nh, int nx, int ny, int nz, float* d_arr, hipStr
     const long long interior = fill_interior(nh, nx, ny, nz);
     if (interior == 0) return PCT_OK;
     void* ws = nullptr;
-    rc = ensure_workspace(dev, fill_ws_bytes(interior, fill_levels(nx, ny, nz)), &ws);
+    rc = ensure_workspace(dev, fill_layout(nh, nx, ny, nz).bytes, &ws);
     if (rc) return rc;
     return enqueue_fill(nh, nx, ny, nz, d_arr, ws, s);
 }
@@ -427,7 +781,7 @@ static int enqueue_round_hu(int nx, int ny, int nz, float* d_arr, hipStream_t s)
 }
 
 size_t postprocess_ws_bytes(int nh, int nx, int ny, int nz) {
-    return fill_ws_bytes(fill_interior(nh, nx, ny, nz), fill_levels(nx, ny, nz));
+    return fill_layout(nh, nx, ny, nz).bytes;
 }
 
 int postprocess_dev_ws(int nh, int nx, int ny, int nz, float* d_arr, void* ws, hipStream_t s) {
