@@ -1,21 +1,24 @@
 // Training of the voxel embedding MLP on gfx950, FP32 throughout.
 //
-// One step over A anchors with K = NH^3 window offsets each:
-//   train_forward       one thread per voxel slot (A * (K+1) slots: the
-//                       anchor's target voxel, then the atlas voxel at every
-//                       offset): features, both hidden layers, embedding.
-//                       Activations go to a row-major [row][slot] buffer so
-//                       every store and later load is coalesced.
-//   train_loss          one workgroup per anchor: teacher SSD and student
-//                       distance for every offset, both log-softmaxes, the
-//                       KL term, and the gradient with respect to every
-//                       embedding of the anchor.
-//   train_backward      one thread per slot: gradients of both hidden layers.
-//   train_grad_partial  one workgroup per chunk of slots: every parameter's
-//                       gradient summed over the chunk (LDS-staged tiles).
-//   grad_reduce         partials summed in chunk order: the gradient does not
-//                       depend on scheduling.
-//   adam_step           Adam on the FP32 master parameters.
+// One step over A anchors with K = NH^3 window offsets each, V = A (K + 1)
+// voxel slots (the anchor's target voxel, then the atlas voxel at every
+// offset):
+//   train_forward    embeddings of all slots, 16 slots a wave at a time, every
+//                    layer on FP32 MFMA.
+//   train_loss       one workgroup per anchor: teacher SSD and student
+//                    distance for every offset, both log-softmaxes, the KL
+//                    term, and the gradient with respect to every embedding
+//                    of the anchor.
+//   train_backward   per 16 slots: the hidden layers again, their gradients,
+//                    and the products that make the parameter gradients,
+//                    summed in accumulators over the wave's slots, then over
+//                    the workgroup's waves in order.
+//   grad_reduce      the workgroups' sums in a fixed order: the gradient does
+//                    not depend on scheduling.
+//   adam_step        Adam on the FP32 master parameters.
+// Only embeddings and their gradients (16 floats a slot each) go through
+// memory: the hidden activations of 3.4e5 slots would be 0.4 GB a step, and
+// computing them twice costs 30 us of matrix time.
 // No counterpart in the reference program.
 #include <hip/hip_runtime.h>
 
@@ -30,21 +33,6 @@
 
 namespace pct {
 
-// Activation buffer rows (each row holds one value for every slot).
-constexpr int kRowX = 0;       // 30 features
-constexpr int kRowOne = 30;    // constant 1 (bias gradients)
-constexpr int kRowH1 = 31;     // 64 first hidden layer (after ReLU)
-constexpr int kRowH2 = 95;     // 64 second hidden layer (after ReLU)
-constexpr int kRowDE = 159;    // 16 d loss / d embedding
-constexpr int kRowDH2 = 175;   // 64 d loss / d second layer pre-activation
-constexpr int kRowDH1 = 239;   // 64 d loss / d first layer pre-activation
-constexpr int kRowsGrad = 303; // rows the gradient pass reads
-constexpr int kRowE = 303;     // 16 embedding
-constexpr int kRows = 319;
-
-constexpr int kTrainThreads = 256;
-constexpr int kGradTile = 32;  // slots per LDS tile of the gradient pass
-constexpr int kParamsPerThread = (kNetParams + kTrainThreads - 1) / kTrainThreads;
 constexpr int kMaxWindow = 15; // NH
 
 struct TrainArgs {
@@ -55,124 +43,252 @@ struct TrainArgs {
     const int* anchors;       // [A][4] z, x, y, atlas
     int n_anchors;
     int K;                    // NH^3
+    int inside;               // 1: every window lies inside the volume with a margin of 1, and
+                              // offsets to a neighbour fit 32 bits
     long long V;              // A * (K + 1)
     const float* params;      // device copy of the parameter vector
-    float* buf;               // [kRows][V]
+    float* emb;               // [V][16] embeddings
+    float* demb;              // [V][16] d loss / d embedding
     float* loss;              // [A]
     float mu, inv_sd;
     float teacher_t, tau;
 };
 
-__device__ __forceinline__ void slot_voxel(const TrainArgs& a, long long v, int* z, int* x, int* y,
-                                           const float** vol) {
-    const int i = (int)(v / (a.K + 1));
-    const int k = (int)(v - (long long)i * (a.K + 1));
-    const int* an = a.anchors + 4 * i;
-    *z = an[0];
-    *x = an[1];
-    *y = an[2];
-    *vol = a.img;
+// ---------------------------------------------------------------------------
+// MFMA layout
+// ---------------------------------------------------------------------------
+//
+// All products are v_mfma_f32_16x16x4_f32, D(16x16) += A(16x4) B(4x16): lane
+// (n = lane & 15, g = lane >> 4) holds A[n][g], B[g][n] and, in four registers
+// i, D[4 g + i][n].  The layers run transposed (units x slots): register i of
+// one layer's output tile, as it lies, is the B operand of a step whose four
+// contraction indices are 4 g + i, so the next layer takes it without moving
+// data, with its weights laid out to match.  The parameter gradients contract
+// over slots instead: the rows go through an LDS tile [row][slot], from which a
+// lane reads four slots 4 g + i of its row, operands of four steps.
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ v4f mfma4(float a, float b, v4f c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// The first layer's contraction index (step s, group g): a feature, 30 for the
+// constant 1 whose weight is the bias, 31 for nothing.  The central differences
+// sit in lanes that hold their two patch values.
+__device__ const unsigned char kFeatOf[4][8] = {{0, 1, 2, 3, 5, 6, 7, 8},
+                                                {9, 11, 13, 15, 17, 18, 19, 20},
+                                                {12, 14, 21, 23, 24, 25, 26, 29},
+                                                {4, 22, 10, 16, 27, 28, 30, 31}};
+constexpr int kFeatOne = 30, kFeatNone = 31;
+
+// Weight of feature f (0 .. 31 as above) to hidden unit m.
+__device__ __forceinline__ float first_weight(const float* __restrict__ p, int f, int m) {
+    return f < kFeat ? p[kOffW1 + f * kHid + m] : f == kFeatOne ? p[kOffB1 + m] : 0.f;
+}
+
+// Patch index of the lane's slot s (the centre where the slot holds none).
+__device__ __forceinline__ int patch_of(int g, int s) {
+    const int f = kFeatOf[g][s];
+    return f < 27 ? f : 13;
+}
+
+// Offsets of the lane's eight patch values from its voxel (used where a.inside).
+__device__ __forceinline__ void patch_offsets(const TrainArgs& a, int g, int (&off)[8]) {
+    const int plane = a.inside ? a.nx * a.ny : 0;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        const int p = patch_of(g, s);
+        off[s] = (p / 9 - 1) * plane + ((p / 3) % 3 - 1) * a.ny + (p % 3 - 1);
+    }
+}
+
+// The raw patch values of slot 16 tile + n, and whether the slot exists (a slot
+// past the end reads the first anchor's voxel).
+__device__ __forceinline__ void load_patch(const TrainArgs& a, long long tile, int n, int g,
+                                           const int (&off)[8], float (&raw)[8], bool* ok) {
+    const long long v0 = tile * 16;
+    long long i = v0 / (a.K + 1);
+    int k = (int)(v0 - i * (a.K + 1)) + n;
+    while (k > a.K) {
+        k -= a.K + 1;
+        ++i;
+    }
+    *ok = v0 + n < a.V;
+    if (!*ok) i = k = 0;
+    const int4 an = reinterpret_cast<const int4*>(a.anchors)[i];   // z, x, y, atlas
+    int z = an.x, x = an.y, y = an.z;
+    const float* __restrict__ vol = a.img;
     if (k > 0) {
         const int c = k - 1, nw = 2 * a.hw + 1;
-        *z += c / (nw * nw) - a.hw;
-        *x += (c / nw) % nw - a.hw;
-        *y += c % nw - a.hw;
-        *vol = a.atlas + (long long)an[3] * a.N;
+        z += c / (nw * nw) - a.hw;
+        x += (c / nw) % nw - a.hw;
+        y += c % nw - a.hw;
+        vol = a.atlas + (long long)an.w * a.N;
     }
-}
-
-__global__ __launch_bounds__(kTrainThreads) void train_forward(TrainArgs a) {
-    __shared__ float w[kNetParams];
-    for (int i = threadIdx.x; i < kNetParams; i += kTrainThreads) w[i] = a.params[i];
-    __syncthreads();
-    const long long v = (long long)blockIdx.x * kTrainThreads + threadIdx.x;
-    if (v >= a.V) return;
-    int z, x, y;
-    const float* vol;
-    slot_voxel(a, v, &z, &x, &y, &vol);
-    float* __restrict__ B = a.buf;
-    const long long V = a.V;
-    float f[kFeat];
+    if (a.inside) {   // uniform
+        const float* __restrict__ p = vol + ((long long)z * a.nx + x) * a.ny + y;
 #pragma unroll
-    for (int k = 0; k < kFeat; ++k) {
-        f[k] = feature(vol, a.nx, a.ny, a.nz, z, x, y, k, a.mu, a.inv_sd);
-        B[(kRowX + k) * V + v] = f[k];
-    }
-    B[kRowOne * V + v] = 1.f;
-    float h1[kHid];
+        for (int s = 0; s < 8; ++s) raw[s] = p[off[s]];
+    } else {
+        // g(u) = 0 outside the volume, where the raw value would be mu
 #pragma unroll
-    for (int m = 0; m < kHid; ++m) {
-        float acc = w[kOffB1 + m];
-#pragma unroll
-        for (int k = 0; k < kFeat; ++k) acc = fmaf(f[k], w[kOffW1 + k * kHid + m], acc);
-        h1[m] = fmaxf(acc, 0.f);
-        B[(kRowH1 + m) * V + v] = h1[m];
-    }
-    float e[kEmb];
-#pragma unroll
-    for (int j = 0; j < kEmb; ++j) e[j] = w[kOffB3 + j];
-#pragma unroll
-    for (int mc = 0; mc < kHid; mc += 16) {
-        float acc[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) acc[j] = w[kOffB2 + mc + j];
-#pragma unroll
-        for (int k = 0; k < kHid; ++k)
-#pragma unroll
-            for (int j = 0; j < 16; ++j)
-                acc[j] = fmaf(h1[k], w[kOffW2 + k * kHid + mc + j], acc[j]);
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const float h = fmaxf(acc[j], 0.f);
-            B[(kRowH2 + mc + j) * V + v] = h;
-#pragma unroll
-            for (int q = 0; q < kEmb; ++q) e[q] = fmaf(h, w[kOffW3 + (mc + j) * kEmb + q], e[q]);
+        for (int s = 0; s < 8; ++s) {
+            const int p = patch_of(g, s);
+            const int zz = z + p / 9 - 1, xx = x + (p / 3) % 3 - 1, yy = y + p % 3 - 1;
+            const bool in = zz >= 0 && zz < a.nz && xx >= 0 && xx < a.nx && yy >= 0 && yy < a.ny;
+            raw[s] = in ? vol[((long long)zz * a.nx + xx) * a.ny + yy] : a.mu;
         }
     }
-#pragma unroll
-    for (int j = 0; j < kEmb; ++j) B[(kRowE + j) * V + v] = e[j];
 }
 
-// Deterministic workgroup reductions (fixed pairing over kTrainThreads).
-__device__ __forceinline__ float block_sum(float v, float* red) {
-    red[threadIdx.x] = v;
-    __syncthreads();
-    for (int s = kTrainThreads / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-        __syncthreads();
+// The lane's eight first-layer inputs from its raw patch values.
+__device__ __forceinline__ void features(const TrainArgs& a, int g, bool ok,
+                                         const float (&raw)[8], float (&x)[8]) {
+#pragma unroll
+    for (int s = 0; s < 8; ++s) x[s] = (raw[s] - a.mu) * a.inv_sd;
+    const float d01 = 0.5f * (x[1] - x[0]), d23 = 0.5f * (x[3] - x[2]);
+    if (g == 2) x[7] = d01;
+    if (g == 3) {
+        x[4] = d01;
+        x[5] = d23;
+        x[6] = 1.f;
+        x[7] = 0.f;
     }
-    const float r = red[0];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) x[s] = ok ? x[s] : 0.f;
+}
+
+__device__ __forceinline__ v4f relu(v4f v) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = fmaxf(v[i], 0.f);
+    return v;
+}
+
+// ---------------------------------------------------------------------------
+// forward
+// ---------------------------------------------------------------------------
+
+// Bound by the matrix pipe: 112 products of 32 cycles for 16 slots, 31 us at
+// 3.4e5 slots (60 us measured, with the fragments' loads; 181 us with one thread
+// per slot and the hidden activations written out).  Each wave keeps the 112 weight fragments in registers and takes
+// a run of consecutive tiles; the next tile's patch loads are in flight during
+// the products.
+constexpr int kFwdWaves = 4;
+constexpr int kWaves = 2048;   // waves that share the tiles (two per SIMD)
+__global__ __launch_bounds__(kFwdWaves * 64, 2) void train_forward(TrainArgs a, long long tiles,
+                                                                   long long chunk) {
+    const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const long long t0 = ((long long)blockIdx.x * kFwdWaves + wv) * chunk;
+    const long long t1 = min(tiles, t0 + chunk);
+    if (t0 >= t1) return;   // per wave; no barrier below
+    const float* __restrict__ p = a.params;
+    float w1[4][8], w2[4][16], w3[16];
+    v4f b2[4], b3;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+#pragma unroll
+        for (int s = 0; s < 8; ++s) w1[m][s] = first_weight(p, kFeatOf[g][s], 16 * m + n);
+#pragma unroll
+        for (int q = 0; q < 16; ++q)
+            w2[m][q] = p[kOffW2 + (16 * (q >> 2) + 4 * g + (q & 3)) * kHid + 16 * m + n];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) b2[m][i] = p[kOffB2 + 16 * m + 4 * g + i];
+    }
+#pragma unroll
+    for (int q = 0; q < 16; ++q)
+        w3[q] = p[kOffW3 + (16 * (q >> 2) + 4 * g + (q & 3)) * kEmb + n];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) b3[i] = p[kOffB3 + 4 * g + i];
+    int off[8];
+    patch_offsets(a, g, off);
+    bool ok;
+    float raw[8];
+    load_patch(a, t0, n, g, off, raw, &ok);
+    for (long long t = t0; t < t1; ++t) {
+        float x[8];
+        features(a, g, ok, raw, x);
+        const bool ok_now = ok;
+        load_patch(a, min(t + 1, t1 - 1), n, g, off, raw, &ok);
+        v4f h1[4], h2[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) h1[m] = (v4f){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+#pragma unroll
+            for (int m = 0; m < 4; ++m) h1[m] = mfma4(w1[m][s], x[s], h1[m]);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            h1[m] = relu(h1[m]);
+            h2[m] = b2[m];
+        }
+#pragma unroll
+        for (int q = 0; q < 16; ++q)
+#pragma unroll
+            for (int m = 0; m < 4; ++m) h2[m] = mfma4(w2[m][q], h1[q >> 2][q & 3], h2[m]);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) h2[m] = relu(h2[m]);
+        v4f e[4] = {b3, (v4f){0.f, 0.f, 0.f, 0.f}, (v4f){0.f, 0.f, 0.f, 0.f},
+                    (v4f){0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int m = 0; m < 4; ++m) e[m] = mfma4(w3[4 * m + i], h2[m][i], e[m]);
+        if (ok_now)
+            *reinterpret_cast<v4f*>(a.emb + (t * 16 + n) * kEmb + 4 * g) =
+                (e[0] + e[1]) + (e[2] + e[3]);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// loss
+// ---------------------------------------------------------------------------
+
+constexpr int kLossThreads = 512;
+constexpr int kLossWaves = kLossThreads / 64;
+
+// Workgroup sum and maximum in a fixed order: within the waves, then over them.
+__device__ __forceinline__ float block_sum(float v, float* red) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    __syncthreads();   // red's last readers are done
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
+    float r = red[0];
+#pragma unroll
+    for (int w = 1; w < kLossWaves; ++w) r += red[w];
     return r;
 }
 __device__ __forceinline__ float block_max(float v, float* red) {
-    red[threadIdx.x] = v;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
     __syncthreads();
-    for (int s = kTrainThreads / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s) red[threadIdx.x] = fmaxf(red[threadIdx.x], red[threadIdx.x + s]);
-        __syncthreads();
-    }
-    const float r = red[0];
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
+    float r = red[0];
+#pragma unroll
+    for (int w = 1; w < kLossWaves; ++w) r = fmaxf(r, red[w]);
     return r;
 }
 
-__global__ __launch_bounds__(kTrainThreads) void train_loss(TrainArgs a) {
+__global__ __launch_bounds__(kLossThreads) void train_loss(TrainArgs a) {
     extern __shared__ float sh[];
-    float* lp = sh;                       // [K] teacher logits
-    float* lq = sh + a.K;                 // [K] student logits
-    float* red = sh + 2 * a.K;            // [kTrainThreads]
-    float* eT = red + kTrainThreads;      // [16]
-    float* tp = eT + kEmb;                // [27] target patch
+    float* lp = sh;                                 // [K] teacher logits
+    float* lq = sh + a.K;                           // [K] student logits
+    float* gsum = sh + 2 * a.K;                     // [kLossThreads][kEmb + 1]
+    __shared__ float red[kLossWaves];
+    __shared__ float eT[kEmb];
+    __shared__ float tp[27];                        // target patch
     const int i = blockIdx.x;
     const long long base = (long long)i * (a.K + 1);
-    const long long V = a.V;
-    float* __restrict__ B = a.buf;
+    const float* __restrict__ E = a.emb + base * kEmb;
+    float* __restrict__ D = a.demb + base * kEmb;
     const int* an = a.anchors + 4 * i;
     const int z = an[0], x = an[1], y = an[2];
     const float* __restrict__ A = a.atlas + (long long)an[3] * a.N;
     const long long plane = (long long)a.nx * a.ny;
-    if (threadIdx.x < kEmb) eT[threadIdx.x] = B[(kRowE + threadIdx.x) * V + base];
+    if (threadIdx.x < kEmb) eT[threadIdx.x] = E[threadIdx.x];
     if (threadIdx.x < 27) {
         const int p = threadIdx.x;
         tp[p] = a.img[(z + p / 9 - 1) * plane + (long long)(x + (p / 3) % 3 - 1) * a.ny +
@@ -181,19 +297,24 @@ __global__ __launch_bounds__(kTrainThreads) void train_loss(TrainArgs a) {
     __syncthreads();
     const int nw = 2 * a.hw + 1;
     float mp = -__builtin_huge_valf(), mq = -__builtin_huge_valf();
-    for (int c = threadIdx.x; c < a.K; c += kTrainThreads) {
-        const int zc = z + c / (nw * nw) - a.hw, xc = x + (c / nw) % nw - a.hw,
-                  yc = y + c % nw - a.hw;
+    for (int c = threadIdx.x; c < a.K; c += kLossThreads) {
+        // inside by a margin of 1 (only an even NH has offsets beyond it)
+        const int zc = min(max(z + c / (nw * nw) - a.hw, 1), a.nz - 2),
+                  xc = min(max(x + (c / nw) % nw - a.hw, 1), a.nx - 2),
+                  yc = min(max(y + c % nw - a.hw, 1), a.ny - 2);
+        const float* __restrict__ q = A + zc * plane + (long long)xc * a.ny + yc;
         float ssd = 0.f;
+#pragma unroll
         for (int p = 0; p < 27; ++p) {
-            const float d = tp[p] - A[(zc + p / 9 - 1) * plane +
-                                      (long long)(xc + (p / 3) % 3 - 1) * a.ny + (yc + p % 3 - 1)];
+            const float d = tp[p] - q[(p / 9 - 1) * plane + (long long)((p / 3) % 3 - 1) * a.ny +
+                                      (p % 3 - 1)];
             ssd = fmaf(d, d, ssd);
         }
+        const v4f* e = reinterpret_cast<const v4f*>(E + (long long)(1 + c) * kEmb);
         float dist = 0.f;
 #pragma unroll
         for (int j = 0; j < kEmb; ++j) {
-            const float d = eT[j] - B[(kRowE + j) * V + base + 1 + c];
+            const float d = eT[j] - e[j >> 2][j & 3];
             dist = fmaf(d, d, dist);
         }
         lp[c] = -ssd / a.teacher_t;
@@ -204,7 +325,7 @@ __global__ __launch_bounds__(kTrainThreads) void train_loss(TrainArgs a) {
     mp = block_max(mp, red);
     mq = block_max(mq, red);
     float zp = 0.f, zq = 0.f;
-    for (int c = threadIdx.x; c < a.K; c += kTrainThreads) {
+    for (int c = threadIdx.x; c < a.K; c += kLossThreads) {
         zp += expf(lp[c] - mp);
         zq += expf(lq[c] - mq);
     }
@@ -216,135 +337,319 @@ __global__ __launch_bounds__(kTrainThreads) void train_loss(TrainArgs a) {
     float gT[kEmb];
 #pragma unroll
     for (int j = 0; j < kEmb; ++j) gT[j] = 0.f;
-    for (int c = threadIdx.x; c < a.K; c += kTrainThreads) {
+    for (int c = threadIdx.x; c < a.K; c += kLossThreads) {
         const float lpn = lp[c] - lzp, lqn = lq[c] - lzq;
         const float p = expf(lpn), q = expf(lqn);
         kl = fmaf(p, lpn - lqn, kl);
         const float g = (p - q) * gscale;   // d loss / d dist_c
+        const v4f* e = reinterpret_cast<const v4f*>(E + (long long)(1 + c) * kEmb);
+        v4f* d = reinterpret_cast<v4f*>(D + (long long)(1 + c) * kEmb);
 #pragma unroll
-        for (int j = 0; j < kEmb; ++j) {
-            const long long idx = (kRowE + j) * V + base + 1 + c;
-            const float diff = eT[j] - B[idx];
-            gT[j] = fmaf(2.f * g, diff, gT[j]);
-            B[(kRowDE + j) * V + base + 1 + c] = -2.f * g * diff;
+        for (int q4 = 0; q4 < kEmb / 4; ++q4) {
+            const v4f ev = e[q4];
+            v4f dv;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float diff = eT[4 * q4 + j] - ev[j];
+                gT[4 * q4 + j] = fmaf(2.f * g, diff, gT[4 * q4 + j]);
+                dv[j] = -2.f * g * diff;
+            }
+            d[q4] = dv;
         }
     }
     kl = block_sum(kl, red);
+    // the target's gradient: thread (j, part) adds 16 of dimension j's terms,
+    // then the 32 parts
 #pragma unroll
-    for (int j = 0; j < kEmb; ++j) {
-        const float s = block_sum(gT[j], red);
-        if (threadIdx.x == 0) B[(kRowDE + j) * V + base] = s;
+    for (int j = 0; j < kEmb; ++j) gsum[threadIdx.x * (kEmb + 1) + j] = gT[j];
+    __syncthreads();
+    {
+        constexpr int kParts = kLossThreads / kEmb;
+        static_assert(kParts == 32, "one half wave per dimension");
+        const int j = threadIdx.x / kParts, part = threadIdx.x % kParts;
+        float sum = 0.f;
+#pragma unroll
+        for (int r = 0; r < kLossThreads / kParts; ++r)
+            sum += gsum[(part + r * kParts) * (kEmb + 1) + j];
+#pragma unroll
+        for (int o = kParts / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, kParts);
+        if (part == 0) D[j] = sum;
     }
     if (threadIdx.x == 0) a.loss[i] = kl / (float)a.n_anchors;
 }
 
-__global__ __launch_bounds__(kTrainThreads) void train_backward(TrainArgs a) {
-    __shared__ float w2[kHid * kHid];
-    __shared__ float w3[kHid * kEmb];
-    for (int i = threadIdx.x; i < kHid * kHid; i += kTrainThreads) w2[i] = a.params[kOffW2 + i];
-    for (int i = threadIdx.x; i < kHid * kEmb; i += kTrainThreads) w3[i] = a.params[kOffW3 + i];
+// ---------------------------------------------------------------------------
+// backward
+// ---------------------------------------------------------------------------
+
+// Bound by the matrix pipe: 288 products for 16 slots (96 for the hidden layers
+// again, 80 for their gradients, 112 for the parameters'), 80 us at 3.4e5
+// slots; the LDS reads of the fragments and rows take 60 % of that beside it.
+// 163 us measured, against 168 us for the activations' gradients and 487 us for
+// the parameters' from 0.4 GB of activations.  Eight waves share the weight
+// fragments in LDS (176 of them; the 112 registers of parameter-gradient
+// accumulators leave no room for them) and have an LDS tile each for the
+// transposed rows.
+constexpr int kBwdWaves = 8;
+constexpr int kRowX = 128;   // rows of the inputs in a wave's tile
+constexpr int kTileRows = kRowX + 32, kTileStride = 20;   // 16 slots, padded: no bank is hit twice
+constexpr int kFrag1 = 0, kFrag2 = 2048, kFrag3 = 6144, kFrag2T = 7168, kBias2 = 11264,
+              kFragEnd = 11328;
+constexpr int kBwdLds = (kFragEnd + kBwdWaves * kTileRows * kTileStride) * 4;
+static_assert(kNetParams <= kFragEnd, "the gradient's sum reuses the fragments' LDS");
+
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// D tile (16 rows from `row`) of 16 slots into the LDS tile.
+__device__ __forceinline__ void put_rows(float* tile, int row, int n, int g, v4f v) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) tile[(row + 4 * g + i) * kTileStride + n] = v[i];
+}
+// Operands of four steps over the 16 slots, rows from `row`.
+__device__ __forceinline__ v4f get_rows(const float* tile, int row, int n, int g) {
+    return *reinterpret_cast<const v4f*>(tile + (row + n) * kTileStride + 4 * g);
+}
+
+__global__ __launch_bounds__(kBwdWaves * 64, 2) void train_backward(TrainArgs a, long long tiles,
+                                                                    long long chunk,
+                                                                    float* partial) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    {
+        const float* __restrict__ p = a.params;
+        // fragment f of a section: float4 [f][lane], component i = step 4 f + i
+        for (int e = threadIdx.x; e < kFragEnd; e += kBwdWaves * 64) {
+            const int i = e & 3, l = (e >> 2) & 63, ln = l & 15, lg = l >> 4;
+            float w;
+            if (e < kFrag2) {
+                const int f = e >> 8, m = f >> 1, st = 4 * (f & 1) + i;
+                w = first_weight(p, kFeatOf[lg][st], 16 * m + ln);
+            } else if (e < kFrag3) {
+                const int f = (e - kFrag2) >> 8, m = f >> 2, kt = f & 3;
+                w = p[kOffW2 + (16 * kt + 4 * lg + i) * kHid + 16 * m + ln];
+            } else if (e < kFrag2T) {
+                const int m = (e - kFrag3) >> 8;
+                w = p[kOffW3 + (16 * m + ln) * kEmb + 4 * lg + i];
+            } else if (e >= kBias2) {
+                w = p[kOffB2 + e - kBias2];
+            } else {
+                const int f = (e - kFrag2T) >> 8, m = f >> 2, kt = f & 3;
+                w = p[kOffW2 + (16 * m + ln) * kHid + 16 * kt + 4 * lg + i];
+            }
+            lds[e] = w;
+        }
+    }
     __syncthreads();
-    const long long v = (long long)blockIdx.x * kTrainThreads + threadIdx.x;
-    if (v >= a.V) return;
-    float* __restrict__ B = a.buf;
-    const long long V = a.V;
-    float de[kEmb];
+    float* tile = lds + kFragEnd + wv * kTileRows * kTileStride;
+    auto frag = [&](int section, int f) {
+        return *reinterpret_cast<const v4f*>(lds + section + (f * 64 + lane) * 4);
+    };
+    const v4f zero = {0.f, 0.f, 0.f, 0.f};
+    v4f g1[2][4], g2[4][4], g3[4];   // gradients of W1 (and b1), W2, W3
+    float gb2[4], gb3 = 0.f;         // and of b2, b3: row 16 m + n, slots 4 g .. 4 g + 3
 #pragma unroll
-    for (int j = 0; j < kEmb; ++j) de[j] = B[(kRowDE + j) * V + v];
-    float dh2[kHid];
+    for (int m = 0; m < 4; ++m) {
+        g1[0][m] = g1[1][m] = g3[m] = zero;
+        gb2[m] = 0.f;
 #pragma unroll
-    for (int m = 0; m < kHid; ++m) {
-        float s = 0.f;
-#pragma unroll
-        for (int j = 0; j < kEmb; ++j) s = fmaf(w3[m * kEmb + j], de[j], s);
-        dh2[m] = B[(kRowH2 + m) * V + v] > 0.f ? s : 0.f;
-        B[(kRowDH2 + m) * V + v] = dh2[m];
+        for (int k = 0; k < 4; ++k) g2[k][m] = zero;
     }
-#pragma unroll 4
-    for (int k = 0; k < kHid; ++k) {
-        float s = 0.f;
+    int off[8];
+    patch_offsets(a, g, off);
+    const long long t0 = ((long long)blockIdx.x * kBwdWaves + wv) * chunk;
+    const long long t1 = min(tiles, t0 + chunk);
+    if (t0 < t1) {   // uniform over the wave; no workgroup barrier inside
+        bool ok;
+        float raw[8];
+        load_patch(a, t0, n, g, off, raw, &ok);
+        v4f de_next = ok ? *reinterpret_cast<const v4f*>(a.demb + (t0 * 16 + n) * kEmb + 4 * g)
+                         : zero;
+        for (long long t = t0; t < t1; ++t) {
+            float x[8];
+            features(a, g, ok, raw, x);
 #pragma unroll
-        for (int m = 0; m < kHid; ++m) s = fmaf(w2[k * kHid + m], dh2[m], s);
-        B[(kRowDH1 + k) * V + v] = B[(kRowH1 + k) * V + v] > 0.f ? s : 0.f;
-    }
-}
-
-// Rows whose product, summed over slots, is the gradient of parameter p
-// (ra = -1: no gradient).
-__device__ __forceinline__ void param_rows(int p, int* ra, int* rb) {
-    *ra = -1;
-    *rb = 0;
-    if (p < kOffB1) {
-        const int k = p / kHid, m = p % kHid;
-        if (k < kFeat) {
-            *ra = kRowX + k;
-            *rb = kRowDH1 + m;
+            for (int s = 0; s < 8; ++s) tile[(kRowX + 8 * g + s) * kTileStride + n] = x[s];
+            const v4f de = de_next;
+            const long long tn = min(t + 1, t1 - 1);
+            load_patch(a, tn, n, g, off, raw, &ok);
+            de_next = ok ? *reinterpret_cast<const v4f*>(a.demb + (tn * 16 + n) * kEmb + 4 * g)
+                         : zero;
+            v4f h1[4], h2[4];
+#pragma unroll
+            for (int m = 0; m < 4; ++m) h1[m] = zero;
+#pragma unroll
+            for (int f = 0; f < 2; ++f)
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    const v4f w = frag(kFrag1, 2 * m + f);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) h1[m] = mfma4(w[i], x[4 * f + i], h1[m]);
+                }
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                h1[m] = relu(h1[m]);
+                h2[m] = *reinterpret_cast<const v4f*>(lds + kBias2 + 16 * m + 4 * g);
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    const v4f w = frag(kFrag2, 4 * m + k);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) h2[m] = mfma4(w[i], h1[k][i], h2[m]);
+                }
+            // through the third layer and its input's ReLU
+            v4f d2[4];
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                h2[m] = relu(h2[m]);
+                const v4f w = frag(kFrag3, m);
+                d2[m] = zero;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) d2[m] = mfma4(w[i], de[i], d2[m]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) d2[m][i] = h2[m][i] > 0.f ? d2[m][i] : 0.f;
+            }
+            // W2: h1 (rows 0 .. 63) with d2 (rows 64 .. 127)
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                put_rows(tile, 16 * m, n, g, h1[m]);
+                put_rows(tile, 64 + 16 * m, n, g, d2[m]);
+            }
+            // through the second layer meanwhile
+            v4f d1[4];
+#pragma unroll
+            for (int m = 0; m < 4; ++m) d1[m] = zero;
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    const v4f w = frag(kFrag2T, 4 * m + k);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) d1[m] = mfma4(w[i], d2[k][i], d1[m]);
+                }
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) d1[m][i] = h1[m][i] > 0.f ? d1[m][i] : 0.f;
+            wave_lds_sync();
+            {
+                v4f rb[4];
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    rb[m] = get_rows(tile, 64 + 16 * m, n, g);
+                    gb2[m] += (rb[m][0] + rb[m][1]) + (rb[m][2] + rb[m][3]);
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const v4f ra = get_rows(tile, 16 * k, n, g);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int m = 0; m < 4; ++m) g2[k][m] = mfma4(ra[i], rb[m][i], g2[k][m]);
+                }
+            }
+            wave_lds_sync();
+            // W3: h2 (rows 0 .. 63) with de (rows 64 .. 79)
+#pragma unroll
+            for (int m = 0; m < 4; ++m) put_rows(tile, 16 * m, n, g, h2[m]);
+            put_rows(tile, 64, n, g, de);
+            wave_lds_sync();
+            {
+                const v4f rb = get_rows(tile, 64, n, g);
+                gb3 += (rb[0] + rb[1]) + (rb[2] + rb[3]);
+                v4f ra[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) ra[k] = get_rows(tile, 16 * k, n, g);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) g3[k] = mfma4(ra[k][i], rb[i], g3[k]);
+            }
+            wave_lds_sync();
+            // W1: x (row 8 g + s of its own rows) with d1 (rows 64 .. 127)
+#pragma unroll
+            for (int m = 0; m < 4; ++m) put_rows(tile, 64 + 16 * m, n, g, d1[m]);
+            wave_lds_sync();
+            {
+                v4f rb[4];
+#pragma unroll
+                for (int m = 0; m < 4; ++m) rb[m] = get_rows(tile, 64 + 16 * m, n, g);
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const v4f ra = get_rows(tile, kRowX + 16 * k, n, g);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int m = 0; m < 4; ++m) g1[k][m] = mfma4(ra[i], rb[m][i], g1[k][m]);
+                }
+            }
+            wave_lds_sync();   // the rows are rewritten next
         }
-    } else if (p < kOffW2) {
-        *ra = kRowOne;
-        *rb = kRowDH1 + (p - kOffB1);
-    } else if (p < kOffB2) {
-        const int q = p - kOffW2;
-        *ra = kRowH1 + q / kHid;
-        *rb = kRowDH2 + q % kHid;
-    } else if (p < kOffW3) {
-        *ra = kRowOne;
-        *rb = kRowDH2 + (p - kOffB2);
-    } else if (p < kOffB3) {
-        const int q = p - kOffW3;
-        *ra = kRowH2 + q / kEmb;
-        *rb = kRowDE + q % kEmb;
-    } else if (p < kNetParams) {
-        *ra = kRowOne;
-        *rb = kRowDE + (p - kOffB3);
     }
-}
-
-__global__ __launch_bounds__(kTrainThreads) void train_grad_partial(TrainArgs a, float* partial,
-                                                                    long long chunk) {
-    __shared__ float t[kRowsGrad][kGradTile + 1];
-    const long long v0 = (long long)blockIdx.x * chunk;
-    const long long v1 = min(a.V, v0 + chunk);
-    int ra[kParamsPerThread], rb[kParamsPerThread];
-    float acc[kParamsPerThread];
+    // biases: the sum over the four groups of slots
 #pragma unroll
-    for (int q = 0; q < kParamsPerThread; ++q) {
-        const int p = threadIdx.x + q * kTrainThreads;
-        param_rows(p < kNetParams ? p : kNetParams, &ra[q], &rb[q]);
-        acc[q] = 0.f;
+    for (int o = 32; o > 8; o >>= 1) {
+#pragma unroll
+        for (int m = 0; m < 4; ++m) gb2[m] += __shfl_xor(gb2[m], o);
+        gb3 += __shfl_xor(gb3, o);
     }
-    const float* __restrict__ B = a.buf;
-    for (long long vt = v0; vt < v1; vt += kGradTile) {
+    // the workgroup's gradient: its waves' sums in wave order
+    __syncthreads();
+    for (int e = threadIdx.x; e < kNetParams; e += kBwdWaves * 64) lds[e] = 0.f;
+    for (int w = 0; w < kBwdWaves; ++w) {
         __syncthreads();
-        for (int idx = threadIdx.x; idx < kRowsGrad * kGradTile; idx += kTrainThreads) {
-            const int row = idx / kGradTile, col = idx % kGradTile;
-            const long long vv = vt + col;
-            t[row][col] = vv < v1 ? B[row * a.V + vv] : 0.f;
-        }
-        __syncthreads();
+        if (wv != w) continue;   // uniform over the wave; the barriers are shared
 #pragma unroll
-        for (int q = 0; q < kParamsPerThread; ++q) {
-            if (ra[q] >= 0) {
-                float s = acc[q];
-                for (int col = 0; col < kGradTile; ++col) s = fmaf(t[ra[q]][col], t[rb[q]][col], s);
-                acc[q] = s;
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const int r = 16 * k + 4 * g + i, f = kFeatOf[r >> 3][r & 7];
+                    if (f != kFeatNone)
+                        lds[(f == kFeatOne ? kOffB1 : kOffW1 + f * kHid) + 16 * m + n] +=
+                            g1[k][m][i];
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    lds[kOffW2 + (16 * k + 4 * g + i) * kHid + 16 * m + n] += g2[k][m][i];
+                lds[kOffW3 + (16 * m + 4 * g + i) * kEmb + n] += g3[m][i];
             }
         }
-    }
+        if (g == 0) {
 #pragma unroll
-    for (int q = 0; q < kParamsPerThread; ++q) {
-        const int p = threadIdx.x + q * kTrainThreads;
-        if (p < kNetParams) partial[(long long)blockIdx.x * kNetParams + p] = acc[q];
+            for (int m = 0; m < 4; ++m) lds[kOffB2 + 16 * m + n] += gb2[m];
+            lds[kOffB3 + n] += gb3;
+        }
     }
+    __syncthreads();
+    for (int e = threadIdx.x; e < kNetParams; e += kBwdWaves * 64)
+        partial[(long long)blockIdx.x * kNetParams + e] = lds[e];
 }
 
-__global__ void grad_reduce(const float* __restrict__ partial, int nblk, float* __restrict__ grad) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= PCT_MLP_NPARAMS) return;
+// Sums the workgroups' gradients: thread (p, part) every fourth of them, then
+// the four parts.  Up to 256 partial vectors of 29 KB: 5 us, where one thread
+// per parameter over 666 of them, one dependent load after another, took 157.
+constexpr int kReduceParts = 4;
+__global__ __launch_bounds__(256) void grad_reduce(const float* __restrict__ partial, int nblk,
+                                                   float* __restrict__ grad) {
+    __shared__ float sh[kReduceParts][64];
+    const int c = threadIdx.x & 63, part = threadIdx.x >> 6;
+    const int p = blockIdx.x * 64 + c;
     float s = 0.f;
-    if (p < kNetParams)
-        for (int b = 0; b < nblk; ++b) s += partial[(long long)b * kNetParams + p];
-    grad[p] = s;
+    if (p < kNetParams) {
+#pragma unroll 8
+        for (int b = part; b < nblk; b += kReduceParts) s += partial[(long long)b * kNetParams + p];
+    }
+    sh[part][c] = s;
+    __syncthreads();
+    if (part == 0 && p < PCT_MLP_NPARAMS) grad[p] = (sh[0][c] + sh[1][c]) + (sh[2][c] + sh[3][c]);
 }
 
 __global__ void adam_step(float* __restrict__ params, float* __restrict__ m1,
@@ -360,12 +665,13 @@ __global__ void adam_step(float* __restrict__ params, float* __restrict__ m1,
     params[p] -= lr * (a / bc1) / (sqrtf(b / bc2) + 1e-8f);
 }
 
-// Device buffers of one training run, carved from the library workspace.
+// Device buffers of one training run, carved from the library workspace, and
+// the split of the slots' tiles over waves and workgroups.
 struct TrainPlan {
-    int K = 0, n_anchors = 0, nblk = 0;
-    long long V = 0, chunk = 0;
-    size_t o_params = 0, o_m1 = 0, o_m2 = 0, o_grad = 0, o_anchors = 0, o_buf = 0, o_loss = 0,
-           o_partial = 0, bytes = 0;
+    int K = 0, n_anchors = 0, nblk = 0, fwd_blk = 0;
+    long long V = 0, tiles = 0, chunk = 0;
+    size_t o_params = 0, o_m1 = 0, o_m2 = 0, o_grad = 0, o_anchors = 0, o_emb = 0, o_demb = 0,
+           o_loss = 0, o_partial = 0, bytes = 0;
 };
 
 static TrainPlan plan_training(int nh, int n_anchors) {
@@ -373,9 +679,11 @@ static TrainPlan plan_training(int nh, int n_anchors) {
     t.K = nh * nh * nh;
     t.n_anchors = n_anchors;
     t.V = (long long)n_anchors * (t.K + 1);
-    t.nblk = (int)std::min<long long>(1024, (t.V + 511) / 512);
-    t.chunk = (t.V + t.nblk - 1) / t.nblk;
-    t.chunk = (t.chunk + kGradTile - 1) / kGradTile * kGradTile;
+    t.tiles = (t.V + 15) / 16;
+    t.chunk = (t.tiles + kWaves - 1) / kWaves;
+    const long long waves = (t.tiles + t.chunk - 1) / t.chunk;
+    t.fwd_blk = (int)((waves + kFwdWaves - 1) / kFwdWaves);
+    t.nblk = (int)((waves + kBwdWaves - 1) / kBwdWaves);
     auto align = [](size_t v) { return (v + 255) & ~(size_t)255; };
     size_t off = 0;
     t.o_params = off; off = align(off + 4 * PCT_MLP_NPARAMS);
@@ -383,7 +691,8 @@ static TrainPlan plan_training(int nh, int n_anchors) {
     t.o_m2 = off; off = align(off + 4 * PCT_MLP_NPARAMS);
     t.o_grad = off; off = align(off + 4 * PCT_MLP_NPARAMS);
     t.o_anchors = off; off = align(off + 16 * (size_t)n_anchors);
-    t.o_buf = off; off = align(off + 4 * (size_t)kRows * t.V);
+    t.o_emb = off; off = align(off + 4 * (size_t)kEmb * t.V);
+    t.o_demb = off; off = align(off + 4 * (size_t)kEmb * t.V);
     t.o_loss = off; off = align(off + 4 * (size_t)n_anchors);
     t.o_partial = off; off = align(off + 4 * (size_t)t.nblk * kNetParams);
     t.bytes = off;
@@ -401,17 +710,28 @@ static int check_train_problem(const pct_problem* pb) {
 
 // Enqueues forward, loss, backward and the gradient into `grad` (device).
 static int enqueue_step(const TrainPlan& t, const TrainArgs& a, char* w, hipStream_t s) {
-    const unsigned vb = (unsigned)((t.V + kTrainThreads - 1) / kTrainThreads);
-    hipLaunchKernelGGL(train_forward, dim3(vb), dim3(kTrainThreads), 0, s, a);
-    const size_t loss_lds = sizeof(float) * (2 * (size_t)t.K + kTrainThreads + kEmb + 27);
-    hipLaunchKernelGGL(train_loss, dim3(t.n_anchors), dim3(kTrainThreads), loss_lds, s, a);
-    hipLaunchKernelGGL(train_backward, dim3(vb), dim3(kTrainThreads), 0, s, a);
-    float* partial = reinterpret_cast<float*>(w + t.o_partial);
-    hipLaunchKernelGGL(train_grad_partial, dim3(t.nblk), dim3(kTrainThreads), 0, s, a, partial,
+    hipLaunchKernelGGL(train_forward, dim3(t.fwd_blk), dim3(kFwdWaves * 64), 0, s, a, t.tiles,
                        t.chunk);
-    hipLaunchKernelGGL(grad_reduce, dim3((PCT_MLP_NPARAMS + 255) / 256), dim3(256), 0, s,
-                       partial, t.nblk, reinterpret_cast<float*>(w + t.o_grad));
+    const size_t loss_lds = sizeof(float) * (2 * (size_t)t.K + kLossThreads * (kEmb + 1));
+    hipLaunchKernelGGL(train_loss, dim3(t.n_anchors), dim3(kLossThreads), loss_lds, s, a);
+    float* partial = reinterpret_cast<float*>(w + t.o_partial);
+    hipLaunchKernelGGL(train_backward, dim3(t.nblk), dim3(kBwdWaves * 64), kBwdLds, s, a, t.tiles,
+                       t.chunk, partial);
+    hipLaunchKernelGGL(grad_reduce, dim3((PCT_MLP_NPARAMS + 63) / 64), dim3(256), 0, s, partial,
+                       t.nblk, reinterpret_cast<float*>(w + t.o_grad));
     return hipGetLastError() == hipSuccess ? PCT_OK : PCT_ERR_HIP;
+}
+
+// Lets the kernels with more than 64 KiB of LDS have it on the current device.
+static int allow_train_lds(const TrainPlan& t) {
+    const size_t loss_lds = sizeof(float) * (2 * (size_t)t.K + kLossThreads * (kEmb + 1));
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(train_backward),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kBwdLds) != hipSuccess ||
+        hipFuncSetAttribute(reinterpret_cast<const void*>(train_loss),
+                            hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)loss_lds) != hipSuccess)
+        return PCT_ERR_HIP;
+    return PCT_OK;
 }
 
 static TrainArgs make_train_args(const pct_problem* pb, const TrainPlan& t, const float* params,
@@ -428,9 +748,12 @@ static TrainArgs make_train_args(const pct_problem* pb, const TrainPlan& t, cons
     a.anchors = reinterpret_cast<const int*>(w + t.o_anchors);
     a.n_anchors = t.n_anchors;
     a.K = t.K;
+    // anchors lie hw + 1 inside; an even NH has more offsets than its window
+    a.inside = (pb->nh & 1) && (long long)pb->nx * pb->ny < (1LL << 30);
     a.V = t.V;
     a.params = reinterpret_cast<const float*>(w + t.o_params);
-    a.buf = reinterpret_cast<float*>(w + t.o_buf);
+    a.emb = reinterpret_cast<float*>(w + t.o_emb);
+    a.demb = reinterpret_cast<float*>(w + t.o_demb);
     a.loss = reinterpret_cast<float*>(w + t.o_loss);
     a.mu = params[kOffMu];
     a.inv_sd = params[kOffSd];
@@ -466,6 +789,8 @@ extern "C" int pct_mlp_loss_grad_dev(const pct_problem* pb, const float* params,
     const TrainPlan t = plan_training(pb->nh, n_anchors);
     void* ws = nullptr;
     rc = ensure_workspace(dev, t.bytes, &ws);
+    if (rc) return rc;
+    rc = allow_train_lds(t);
     if (rc) return rc;
     char* w = static_cast<char*>(ws);
     if (hipMemcpyAsync(w + t.o_params, params, 4 * PCT_MLP_NPARAMS, hipMemcpyHostToDevice, s) !=
@@ -504,6 +829,8 @@ extern "C" int pct_mlp_train_dev(const pct_problem* pb, float* params,
     const TrainPlan t = plan_training(pb->nh, opts->anchors);
     void* ws = nullptr;
     rc = ensure_workspace(dev, t.bytes, &ws);
+    if (rc) return rc;
+    rc = allow_train_lds(t);
     if (rc) return rc;
     char* w = static_cast<char*>(ws);
     float* d_params = reinterpret_cast<float*>(w + t.o_params);
