@@ -223,7 +223,7 @@ static bool plan_batch(const pct_subject* s, int n, const pct_batch_choice& ch, 
         if (!make_geometry(&s[i].pb, sid, std::min(grp, s[i].pb.n_atlas), &g)) return false;
         p->geo[i] = g;
         p->ws_off[i] = off;
-        off += tiled_ws_bytes(&s[i].pb, g.n_groups, sid);
+        off += tiled_ws_bytes(&s[i].pb, g.n_parts(), sid);
         item_cost[i] = g.group;
         if (g.n_items > 0) by_hw[hw].push_back(i);
     }
@@ -292,7 +292,7 @@ static int enqueue_batch(const pct_subject* s, const BatchPlan& p, const std::ve
             const int rc = launch_atlas_pairs(
                 &s[i].pb, s[i].d_atlas, s[i].d_atlas_label_norm, s[i].pb.n_atlas, t.scale,
                 reinterpret_cast<f32x2*>(base + p.ws_off[i] +
-                                         tiled_le_offset(&s[i].pb, p.geo[i].n_groups)),
+                                         tiled_le_offset(&s[i].pb, p.geo[i].n_parts())),
                 stream);
             if (rc) return rc;
         }
@@ -316,7 +316,7 @@ static int enqueue_batch(const pct_subject* s, const BatchPlan& p, const std::ve
                                        reinterpret_cast<float*>(base + p.ws_off[i]));
             if (is_xterm_shape(sid))
                 a.sub[k].le = reinterpret_cast<const f32x2*>(
-                    base + p.ws_off[i] + tiled_le_offset(&s[i].pb, p.geo[i].n_groups));
+                    base + p.ws_off[i] + tiled_le_offset(&s[i].pb, p.geo[i].n_parts()));
             a.n_items[k] = p.geo[i].n_items;
             ++k;
         }

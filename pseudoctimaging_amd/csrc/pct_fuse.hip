@@ -265,10 +265,11 @@ struct TiledEntry {
 template <int W, int BX, int BZ, int NW, int HW, int FORM>
 TiledEntry make_entry() {
     using C = TiledCfg<W, BX, BZ, NW, HW>;
-    if (FORM == 1)
+    if constexpr (FORM == 1)
         return TiledEntry{{W, BX, BZ, NW, 1}, HW, &fuse_tiled_xt<W, BX, BZ, NW, HW>,
                           XtCfg<C>::LDS_BYTES, 0};
-    return TiledEntry{{W, BX, BZ, NW, 0}, HW, &fuse_tiled<W, BX, BZ, NW, HW>, C::LDS_BYTES, 0};
+    else
+        return TiledEntry{{W, BX, BZ, NW, 0}, HW, &fuse_tiled<W, BX, BZ, NW, HW>, C::LDS_BYTES, 0};
 }
 
 template <int W, int BX, int BZ, int NW, int FORM = 0>
@@ -366,7 +367,7 @@ double problem_divisor(const pct_problem* pb) {
 
 static int interior(int n, int r) { return std::max(0, n - 2 * r); }
 
-bool make_geometry(const pct_problem* pb, int shape_id, int group, TileGeometry* g) {
+bool make_geometry(const pct_problem* pb, int shape_id, int group, TileGeometry* g, int split) {
     const int hw = (pb->nh - 1) / 2;
     const TiledEntry* e = find_entry(shape_id, hw);
     if (!e) return false;
@@ -384,7 +385,8 @@ bool make_geometry(const pct_problem* pb, int shape_id, int group, TileGeometry*
     g->n_tiles = (long long)g->tiles_y * g->tiles_x * g->tiles_z;
     g->group = std::max(1, std::min(group, pb->n_atlas));
     g->n_groups = (pb->n_atlas + g->group - 1) / g->group;
-    g->n_items = g->n_tiles * g->n_groups;
+    g->n_split = std::max(1, std::min(split, 2 * hw + 1));
+    g->n_items = g->n_tiles * g->n_parts();
     g->lds_bytes = e->lds_bytes;
     const int by_lds = kLdsPerCu / e->lds_bytes;
     const int by_waves = 32 / s.waves;  // 8 waves per SIMD slot budget, 4 SIMDs
@@ -596,14 +598,14 @@ bool is_xterm_shape(int shape_id) {
     return shape_id >= 0 && shape_id < (int)shapes().size() && shapes()[shape_id].form == 1;
 }
 
-size_t tiled_le_offset(const pct_problem* pb, int n_groups) {
+size_t tiled_le_offset(const pct_problem* pb, int n_parts) {
     const size_t N = (size_t)pb->nx * pb->ny * pb->nz;
-    return ((2 * (size_t)n_groups * N * sizeof(float)) + 255) & ~(size_t)255;
+    return ((2 * (size_t)n_parts * N * sizeof(float)) + 255) & ~(size_t)255;
 }
 
-size_t tiled_ws_bytes(const pct_problem* pb, int n_groups, int shape_id) {
+size_t tiled_ws_bytes(const pct_problem* pb, int n_parts, int shape_id) {
     const size_t N = (size_t)pb->nx * pb->ny * pb->nz;
-    size_t bytes = tiled_le_offset(pb, n_groups);
+    size_t bytes = tiled_le_offset(pb, n_parts);
     if (is_xterm_shape(shape_id))
         bytes += ((size_t)pb->n_atlas * N * sizeof(f32x2) + 255) & ~(size_t)255;
     return bytes;
@@ -644,7 +646,7 @@ int launch_finalize(const pct_problem* pb, const TileGeometry& g, const float* w
                     hipStream_t stream) {
     const long long N = (long long)pb->nx * pb->ny * pb->nz;
     const dim3 fb(256), fgrid((pb->ny + 255) / 256, pb->nx, pb->nz);
-    hipLaunchKernelGGL(fuse_finalize, fgrid, fb, 0, stream, ws, g.n_items > 0 ? g.n_groups : 0, N,
+    hipLaunchKernelGGL(fuse_finalize, fgrid, fb, 0, stream, ws, g.n_items > 0 ? g.n_parts() : 0, N,
                        pb->nx, pb->ny, pb->nz, g.r, out);
     return hipGetLastError() == hipSuccess ? PCT_OK : PCT_ERR_HIP;
 }
@@ -667,6 +669,7 @@ TiledArgs make_tiled_args(const pct_problem* pb, const TileGeometry& g, const fl
     a.n_items = (int)g.n_items;
     a.n_atlas = pb->n_atlas;
     a.group = g.group;
+    a.n_split = g.n_split;
     const double div = problem_divisor(pb);
     a.scale = (float)std::sqrt(1.4426950408889634 / div);
     a.only = nullptr;
@@ -730,11 +733,11 @@ static int launch_tiled(const pct_problem* pb, const float* img, const float* at
                         int shape_id, const TileGeometry& g, hipStream_t stream) {
     const TiledEntry* e = find_entry(shape_id, g.hw);
     if (!e) return PCT_ERR_UNSUPPORTED;
-    if (ws_bytes < tiled_ws_bytes(pb, g.n_groups, shape_id)) return PCT_ERR_INVALID;
+    if (ws_bytes < tiled_ws_bytes(pb, g.n_parts(), shape_id)) return PCT_ERR_INVALID;
     TiledArgs a = make_tiled_args(pb, g, img, atlas, label, static_cast<float*>(ws));
     if (is_xterm_shape(shape_id) && g.n_items > 0) {
         f32x2* le = reinterpret_cast<f32x2*>(static_cast<char*>(ws) +
-                                             tiled_le_offset(pb, g.n_groups));
+                                             tiled_le_offset(pb, g.n_parts()));
         const int rc = launch_atlas_pairs(pb, atlas, label, pb->n_atlas, a.scale, le, stream);
         if (rc) return rc;
         a.le = le;
@@ -831,7 +834,7 @@ extern "C" size_t pct_fuse_workspace_size(const pct_problem* pb, int choice) {
     int sid = 0, grp = 1;
     TileGeometry g;
     if (!choose(pb, &sid, &grp, nullptr, &g)) return 0;
-    return tiled_ws_bytes(pb, g.n_groups, sid);
+    return tiled_ws_bytes(pb, g.n_parts(), sid);
 }
 
 static int fuse_dev_impl(const pct_problem* pb, const float* img, const float* atlas,
@@ -848,7 +851,7 @@ static int fuse_dev_impl(const pct_problem* pb, const float* img, const float* a
     int sid = 0, grp = 1;
     TileGeometry g;
     if (!choose(pb, &sid, &grp, nullptr, &g)) return PCT_ERR_UNSUPPORTED;
-    const size_t need = tiled_ws_bytes(pb, g.n_groups, sid);
+    const size_t need = tiled_ws_bytes(pb, g.n_parts(), sid);
     if (own_ws) {
         rc = ensure_workspace(dev, need, &ws);
         if (rc) return rc;
@@ -946,7 +949,7 @@ extern "C" int pct_fuse_dev_noalloc(const pct_problem* pb, const float* d_img, c
     int sid = -1;
     TileGeometry g;
     if (!choose_noalloc(pb, &sid, &g)) return PCT_ERR_UNSUPPORTED;
-    const size_t need = tiled_ws_bytes(pb, g.n_groups, sid);
+    const size_t need = tiled_ws_bytes(pb, g.n_parts(), sid);
     if (need > kNoAllocScratchBytes) return PCT_ERR_TOO_LARGE;
     void* ws = nullptr;
     rc = scratch_address(dev, &ws);
@@ -1164,13 +1167,13 @@ static int fuse_host_impl(const pct_problem* pb, const float* img, const float* 
     void* ws = nullptr;
     {
         size_t need = post ? postprocess_ws_bytes(pb->nh, pb->nx, pb->ny, pb->nz) : 0;
-        if (tiled) need = std::max(need, tiled_ws_bytes(pb, g.n_groups, sid));
+        if (tiled) need = std::max(need, tiled_ws_bytes(pb, g.n_parts(), sid));
         if (!need) need = 256;
         rc = host_workspace(st, need, &ws);
     }
     f32x2* le = tiled && is_xterm_shape(sid)
                     ? reinterpret_cast<f32x2*>(static_cast<char*>(ws) +
-                                               tiled_le_offset(pb, g.n_groups))
+                                               tiled_le_offset(pb, g.n_parts()))
                     : nullptr;
     // cu:1687-1699: host->device copies
     if (!rc) rc = stage_h2d(st, st.img, img, N * 4, cs);
@@ -1191,9 +1194,9 @@ static int fuse_host_impl(const pct_problem* pb, const float* img, const float* 
             }
             // the items of groups g0 .. g1-1: pointers offset to the chunk
             TiledArgs a = make_tiled_args(pb, g, st.img, st.atlas + off, st.label + off,
-                                          static_cast<float*>(ws) + 2 * (size_t)g0 * N);
+                                          static_cast<float*>(ws) + 2 * (size_t)(g0 * g.n_split) * N);
             a.n_atlas = a1 - a0;
-            a.n_items = (int)(g.n_tiles * (g1 - g0));
+            a.n_items = (int)(g.n_tiles * (g1 - g0) * g.n_split);
             hipStream_t cstream = (c & 1) ? st.compute2 : s;
             if (le) {
                 // pairs of the chunk's atlases, computed as the single launch does
@@ -1344,7 +1347,7 @@ extern "C" int pct_autotune(const pct_problem* pb, const float* d_img, const flo
             TileGeometry g;
             if (!make_geometry(pb, sid, grp, &g)) continue;
             void* ws = nullptr;
-            const size_t need = tiled_ws_bytes(pb, g.n_groups, sid);
+            const size_t need = tiled_ws_bytes(pb, g.n_parts(), sid);
             rc = ensure_workspace(dev, need, &ws);
             if (rc) break;
             // warm-up

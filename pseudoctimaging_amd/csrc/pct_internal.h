@@ -25,10 +25,13 @@ struct TileShape {
 struct TileGeometry {
     int hw = 0, r = 0;
     int tiles_y = 0, tiles_x = 0, tiles_z = 0;
-    int group = 1, n_groups = 1;
+    int group = 1, n_groups = 1;   // atlases per group, groups
+    int n_split = 1;               // parts the window's dz are split into
     long long n_tiles = 0, n_items = 0;
     int lds_bytes = 0;
     int wg_per_cu = 0;
+    // partial sums per voxel: one per group and part of the window
+    int n_parts() const { return n_groups * n_split; }
 };
 
 // Problem validation shared by every entry point.

@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
 #include <vector>
 
 #include "pct_internal.h"
@@ -63,6 +64,8 @@ __device__ __forceinline__ float fused_value(float P, float S) {
 // tiled kernel
 // ---------------------------------------------------------------------------
 
+constexpr int kLdsPerCu = 160 * 1024;
+
 // Native two-float vector: its loads and stores stay single 64-bit accesses
 // (HIP's float2 struct is copied member by member).
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -71,7 +74,7 @@ struct TiledArgs {
     const float* img;
     const float* atlas;
     const float* label;
-    float* ws;        // [n_groups][2][N]
+    float* ws;        // [n_groups * n_split][2][N]
     long long N;      // nx*ny*nz
     int nx, ny, nz;
     int r;            // hw + 1
@@ -79,6 +82,7 @@ struct TiledArgs {
     int n_tiles;
     int n_items;
     int n_atlas, group;
+    int n_split;      // parts of the window's dz, each an item of its own
     float scale;      // sqrt(log2(e)/div)
     // optional item filter: when set, items whose byte is 0 are skipped
     const unsigned char* only;
@@ -111,12 +115,8 @@ struct TiledCfg {
     static_assert(PPB >= 1, "one plane must fit an LDS immediate window");
     static constexpr int NBA = (APLANES + PPB - 1) / PPB;   // base registers, MRI planes
     static constexpr int NBL = (LPLANES + PPB - 1) / PPB;   // base registers, CT planes
-    // the same for the dx sweep, whose immediates carry the row (up to
-    // 2 HW + BX + 1) and no dy
-    static constexpr int PPBS = (16383 - (2 * HW + BX + 1) * CW) / PS + 1;
-    static_assert(PPBS >= 1, "one plane must fit an LDS immediate window");
-    static constexpr int NBAS = (APLANES + PPBS - 1) / PPBS;
-    static constexpr int NBLS = (LPLANES + PPBS - 1) / PPBS;
+    // the dx sweep's immediates carry the row (up to 2 HW + BX + 1) alone
+    static_assert((2 * HW + BX + 1) * CW <= 16383, "rows must fit an LDS immediate");
     static_assert(64 % W == 0, "segment width must divide the wavefront");
     static_assert(BX % 2 == 0 && BZ % 2 == 0, "pairwise box sums need even blocks");
 };
@@ -129,6 +129,26 @@ __device__ __forceinline__ int opaque(int v) {
     return v;
 }
 
+// The four 3 x 3 window sums of the products u(z, x) v(z, x) over a 4 x 4 block:
+// the windows share the middle 2 x 2, and pairs of them an edge, so 20
+// multiply-adds and adds do where sums over x and then z take 22 (222x222x112,
+// n=10, NH=11: 15.7 against 16.15 ms).
+template <class U, class V>
+__device__ __forceinline__ void window_sums_2x2(U u, V v, float (&c)[2][2]) {
+    float core = u(1, 1) * v(1, 1);
+    core = fmaf(u(1, 2), v(1, 2), core);
+    core = fmaf(u(2, 1), v(2, 1), core);
+    core = fmaf(u(2, 2), v(2, 2), core);
+    const float top = fmaf(u(0, 2), v(0, 2), fmaf(u(0, 1), v(0, 1), core));
+    const float bottom = fmaf(u(3, 2), v(3, 2), fmaf(u(3, 1), v(3, 1), core));
+    const float left = fmaf(u(2, 0), v(2, 0), u(1, 0) * v(1, 0));
+    const float right = fmaf(u(2, 3), v(2, 3), u(1, 3) * v(1, 3));
+    c[0][0] = fmaf(u(0, 0), v(0, 0), top + left);
+    c[0][1] = fmaf(u(0, 3), v(0, 3), top + right);
+    c[1][0] = fmaf(u(3, 0), v(3, 0), bottom + left);
+    c[1][1] = fmaf(u(3, 3), v(3, 3), bottom + right);
+}
+
 // Sums over x and z of the squared differences of a lane's block: c[j][i] is
 // the sum over planes j .. j+2 and rows i .. i+2 of (tv - a)^2, a(pz, row) the
 // atlas value.  The multiply-adds are written out, so that every kernel that
@@ -136,6 +156,16 @@ __device__ __forceinline__ int opaque(int v) {
 template <int BX, int BZ, class Atlas>
 __device__ __forceinline__ void squared_sums_xz(const float (&tv)[BZ + 2][BX + 2], Atlas a,
                                                 float (&c)[BZ][BX]) {
+    if constexpr (BX == 2 && BZ == 2) {
+        float d[4][4];
+#pragma unroll
+        for (int pz = 0; pz < 4; ++pz)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) d[pz][i] = tv[pz][i] - a(pz, i);
+        window_sums_2x2([&](int pz, int i) { return d[pz][i]; },
+                        [&](int pz, int i) { return d[pz][i]; }, c);
+        return;
+    }
     float ex[BZ + 2][BX];
 #pragma unroll
     for (int pz = 0; pz < BZ + 2; ++pz) {
@@ -159,39 +189,63 @@ __device__ __forceinline__ void squared_sums_xz(const float (&tv)[BZ + 2][BX + 2
         }
 }
 
+// Where the slab's planes sit in LDS.  From one dz to the next the slab keeps
+// all but its first MRI and its first CT plane; the two new ones take their
+// places, so the plane a logical index names moves by one slot a step.  Element
+// offsets, uniform over the workgroup.
+template <class C>
+struct SlabSlots {
+    int mri[C::APLANES], ct[C::LPLANES];
+    __device__ __forceinline__ void reset() {
+#pragma unroll
+        for (int p = 0; p < C::APLANES; ++p) mri[p] = p * C::PS;
+#pragma unroll
+        for (int p = 0; p < C::LPLANES; ++p) ct[p] = C::LOFF + p * C::PS;
+    }
+    __device__ __forceinline__ void advance() {
+        const int m = mri[0], l = ct[0];
+#pragma unroll
+        for (int p = 0; p + 1 < C::APLANES; ++p) mri[p] = mri[p + 1];
+#pragma unroll
+        for (int p = 0; p + 1 < C::LPLANES; ++p) ct[p] = ct[p + 1];
+        mri[C::APLANES - 1] = m;
+        ct[C::LPLANES - 1] = l;
+    }
+};
+
 // All 2 HW + 1 dx candidates of one dy with squared differences.  `base` is
 // the LDS element index of plane 0, row 0 of the lane's window for dx = 0.
 // Candidate dx reads MRI rows dx .. dx + BX + 1, so consecutive candidates
 // share BX + 1 of their BX + 2 rows: the rows stay in registers and each
 // candidate after the first reads one new row (BZ + 2 reads instead of
-// (BZ + 2)(BX + 2)); CT rows are shared the same way.  The planes are
-// addressed from a few base registers hidden from the optimiser (`opaque`),
-// so each stays one register and the plane and row offsets ride in the
-// ds_read immediates.  Per candidate the lane squares its (BZ+2) x (BX+2)
+// (BZ + 2)(BX + 2)); CT rows are shared the same way.  Each plane is addressed
+// from a base register hidden from the optimiser (`opaque`), so that it stays
+// one register and the row offsets ride in the ds_read immediates.  Per candidate the lane squares its (BZ+2) x (BX+2)
 // differences, sums them pairwise over x and then z in registers and over y
 // across lanes (two DPP adds), and weighs with w = 2^-SSD' on MRI values
 // pre-scaled by sqrt(log2(e) / div).
 template <class C, int BX, int BZ, int HW>
 __device__ __forceinline__ void tiled_dx_sweep(const float* __restrict__ lds, int base,
+                                               const SlabSlots<C>& slots,
                                                const float (&tv)[BZ + 2][BX + 2],
                                                float (&P)[BZ][BX], float (&S)[BZ][BX]) {
-    int ba[C::NBAS], bl[C::NBLS];
+    int ba[BZ + 2], bl[BZ];
 #pragma unroll
-    for (int b = 0; b < C::NBAS; ++b) ba[b] = opaque(base + b * C::PPBS * C::PS);
+    for (int b = 0; b < BZ + 2; ++b) ba[b] = opaque(base + slots.mri[b]);
 #pragma unroll
-    for (int b = 0; b < C::NBLS; ++b) bl[b] = opaque(base + C::LOFF + b * C::PPBS * C::PS);
+    for (int b = 0; b < BZ; ++b) bl[b] = opaque(base + slots.ct[b]);
     constexpr int NR = BX + 2 + 2 * HW;
     float rows[NR][BZ + 2];
     auto load_row = [&](int r) {
 #pragma unroll
         for (int pz = 0; pz < BZ + 2; ++pz)
-            rows[r][pz] = lds[ba[pz / C::PPBS] + (pz % C::PPBS) * C::PS + r * C::CW];
+            rows[r][pz] = lds[ba[pz] + r * C::CW];
     };
     float ct[2 * HW + BX][BZ];   // CT of candidate dx, output i: row dx + i
     auto load_ct = [&](int r) {
 #pragma unroll
         for (int j = 0; j < BZ; ++j)
-            ct[r][j] = lds[bl[j / C::PPBS] + (j % C::PPBS) * C::PS + (r + 1) * C::CW];
+            ct[r][j] = lds[bl[j] + (r + 1) * C::CW];
     };
     float w[BZ][BX];
     auto accumulate = [&](int dx) {
@@ -252,60 +306,83 @@ __device__ __forceinline__ void lane_columns(int ys, int ny, int lane, int (&ycl
     }
 }
 
-// Copies the slab of one (atlas, dz) stage into LDS: plane p < APLANES holds
-// the atlas MRI at z = zdz-1+p (scaled), plane APLANES+j the atlas CT at
-// z = zdz+j; row rr is volume x = xs+rr, column c is volume y = ys+c; zero
-// outside the volume.  Each wave issues the loads of all its rows of two
-// planes before it writes any of them, so global latency is paid once per
-// pair of planes.
+// Copies two planes into LDS: plane q of `src[q]` at volume z = z[q], times
+// mul[q], to the element offset at[q]; row rr is volume x = xs+rr, column c is
+// volume y = ys+c; zero outside the volume.  Each wave issues the loads of all
+// its rows of both planes before it writes any of them, so global latency is
+// paid once per pair of planes.
 template <class C, int NW>
-__device__ __forceinline__ void stage_slab(float* __restrict__ lds, const float* __restrict__ A,
-                                           const float* __restrict__ L, float scale, int zdz,
-                                           int xs, int ys, int nx, int ny, int nz,
-                                           long long plane, int wv, int lane) {
-    constexpr int NP = C::APLANES + C::LPLANES;
+__device__ __forceinline__ void stage_two(float* __restrict__ lds, const float* const (&src)[2],
+                                          const float (&mul)[2], const int (&z)[2],
+                                          const int (&at)[2], int xs, int ys, int nx, int ny,
+                                          int nz, long long plane, int wv, int lane) {
     constexpr int RPW = (C::RX + NW - 1) / NW;   // rows per wave and plane
-    constexpr int PB = 2;                         // planes per batch
-    static_assert(NP % PB == 0, "plane batches must tile the slab");
+    // made anew for every call: kept over the sweeps, the addresses would cost
+    // 35 registers
+    wv = opaque(wv);
+    lane = opaque(lane);
     int ycl[C::COLCHUNKS];
     bool yin[C::COLCHUNKS];
     lane_columns<C>(ys, ny, lane, ycl, yin);
-#pragma unroll 1
-    for (int p0 = 0; p0 < NP; p0 += PB) {
-        float v[PB][RPW][C::COLCHUNKS];
+    float v[2][RPW][C::COLCHUNKS];
 #pragma unroll
-        for (int q = 0; q < PB; ++q) {
-            const int p = p0 + q;
-            const bool is_mri = p < C::APLANES;
-            const int zz = is_mri ? zdz - 1 + p : zdz + (p - C::APLANES);
-            const float* __restrict__ src = is_mri ? A : L;
-            const float mul = is_mri ? scale : 1.f;
-            const bool zok = zz >= 0 && zz < nz;
-            const float* __restrict__ sz = src + (long long)clampi(zz, nz) * plane;
+    for (int q = 0; q < 2; ++q) {
+        const bool zok = z[q] >= 0 && z[q] < nz;
+        const float* __restrict__ sz = src[q] + (long long)clampi(z[q], nz) * plane;
 #pragma unroll
-            for (int k = 0; k < RPW; ++k) {
-                const int rr = wv + k * NW;
-                const int xx = xs + rr;
-                const bool xok = zok && rr < C::RX && xx >= 0 && xx < nx;
-                const float* __restrict__ sr = sz + (long long)clampi(xx, nx) * ny;
+        for (int k = 0; k < RPW; ++k) {
+            const int rr = wv + k * NW;
+            const int xx = xs + rr;
+            const bool xok = zok && rr < C::RX && xx >= 0 && xx < nx;
+            const float* __restrict__ sr = sz + (long long)clampi(xx, nx) * ny;
 #pragma unroll
-                for (int cc = 0; cc < C::COLCHUNKS; ++cc) {
-                    const float raw = sr[ycl[cc]];
-                    v[q][k][cc] = (xok && yin[cc]) ? raw * mul : 0.f;
-                }
+            for (int cc = 0; cc < C::COLCHUNKS; ++cc) {
+                const float raw = sr[ycl[cc]];
+                v[q][k][cc] = (xok && yin[cc]) ? raw * mul[q] : 0.f;
             }
         }
+    }
 #pragma unroll
-        for (int q = 0; q < PB; ++q)
+    for (int q = 0; q < 2; ++q)
 #pragma unroll
-            for (int k = 0; k < RPW; ++k) {
-                const int rr = wv + k * NW;
+        for (int k = 0; k < RPW; ++k) {
+            const int rr = wv + k * NW;
 #pragma unroll
-                for (int cc = 0; cc < C::COLCHUNKS; ++cc) {
-                    const int c = lane + cc * 64;
-                    if (rr < C::RX && c < C::CW) lds[(p0 + q) * C::PS + rr * C::CW + c] = v[q][k][cc];
-                }
+            for (int cc = 0; cc < C::COLCHUNKS; ++cc) {
+                const int c = lane + cc * 64;
+                if (rr < C::RX && c < C::CW) lds[at[q] + rr * C::CW + c] = v[q][k][cc];
             }
+        }
+}
+
+// The slab of one (atlas, dz): MRI plane p at z = zdz-1+p (scaled), CT plane j
+// at z = zdz+j.  The first slab of an atlas is copied whole (`whole`, slots
+// reset by the caller); a slab after it takes over the planes of the one before
+// and copies the last MRI and the last CT plane (slots advanced by the caller).
+// Copying every slab whole took 12-40 % of an item's time, more the smaller the
+// window (BZ = 2: 88 plane rows' loads an atlas at NH 11, 38 now).
+template <class C, int NW>
+__device__ __forceinline__ void stage_slab(float* __restrict__ lds, const SlabSlots<C>& slots,
+                                           bool whole, const float* __restrict__ A,
+                                           const float* __restrict__ L, float scale, int zdz,
+                                           int xs, int ys, int nx, int ny, int nz,
+                                           long long plane, int wv, int lane) {
+    if (whole) {
+        static_assert(C::APLANES % 2 == 0 && C::LPLANES % 2 == 0, "planes are copied in pairs");
+#pragma unroll 1
+        for (int p = 0; p < C::APLANES; p += 2)
+            stage_two<C, NW>(lds, {A, A}, {scale, scale}, {zdz - 1 + p, zdz + p},
+                             {p * C::PS, (p + 1) * C::PS}, xs, ys, nx, ny, nz, plane, wv, lane);
+#pragma unroll 1
+        for (int p = 0; p < C::LPLANES; p += 2)
+            stage_two<C, NW>(lds, {L, L}, {1.f, 1.f}, {zdz + p, zdz + p + 1},
+                             {C::LOFF + p * C::PS, C::LOFF + (p + 1) * C::PS}, xs, ys, nx, ny, nz,
+                             plane, wv, lane);
+    } else {
+        stage_two<C, NW>(lds, {A, L}, {scale, 1.f},
+                         {zdz - 2 + C::APLANES, zdz - 1 + C::LPLANES},
+                         {slots.mri[C::APLANES - 1], slots.ct[C::LPLANES - 1]}, xs, ys, nx, ny, nz,
+                         plane, wv, lane);
     }
 }
 
@@ -426,8 +503,9 @@ template <int W, int BX, int BZ, int NW, int HW>
 __device__ __forceinline__ void tiled_item(const TiledArgs& args, int item,
                                            float* __restrict__ lds) {
     using C = TiledCfg<W, BX, BZ, NW, HW>;
-    const int g = item / args.n_tiles;
-    int t = item - g * args.n_tiles;
+    const int part = item / args.n_tiles;   // (atlas group, part of the window)
+    const int g = part / args.n_split, sp = part - g * args.n_split;
+    int t = item - part * args.n_tiles;
     const int ty = t % args.tiles_y;
     t /= args.tiles_y;
     const int tx = t % args.tiles_x;
@@ -465,26 +543,32 @@ __device__ __forceinline__ void tiled_item(const TiledArgs& args, int item,
     const int ys = y0 - 1 - HW;   // volume y of LDS column 0
     const int a_begin = g * args.group;
     const int a_end = min(args.n_atlas, a_begin + args.group);
+    const int dz_begin = sp * (2 * HW + 1) / args.n_split - HW;
+    const int dz_end = (sp + 1) * (2 * HW + 1) / args.n_split - HW;
     const bool live = wave_has_rows<C, BX>(x0, nx - r, wv);
 
     for (int a = a_begin; a < a_end; ++a) {
         const float* __restrict__ A = args.atlas + (long long)a * args.N;
         const float* __restrict__ L = args.label + (long long)a * args.N;
-        for (int dz = -HW; dz <= HW; ++dz) {
+        SlabSlots<C> slots;
+        slots.reset();
+        for (int dz = dz_begin; dz < dz_end; ++dz) {
+            if (dz > dz_begin) slots.advance();
             __syncthreads();
-            stage_slab<C, NW>(lds, A, L, args.scale, z0 + dz, xs, ys, nx, ny, nz, plane, wv, lane);
+            stage_slab<C, NW>(lds, slots, dz == dz_begin, A, L, args.scale, z0 + dz, xs, ys, nx,
+                              ny, nz, plane, wv, lane);
             __syncthreads();
             if (!live) continue;
             // dy rolled, dx unrolled: consecutive dx share MRI and CT rows
 #pragma unroll 1
             for (int dy = 0; dy <= 2 * HW; ++dy)
-                tiled_dx_sweep<C, BX, BZ, HW>(lds, lane_base + dy, tv, P, S);
+                tiled_dx_sweep<C, BX, BZ, HW>(lds, lane_base + dy, slots, tv, P, S);
         }
     }
 
     // Store the group's partial sums for the lane's valid outputs.
     if (ly >= 1 && ly <= W - 2 && y < ny - r) {
-        float* __restrict__ wsP = args.ws + (long long)(2 * g) * args.N;
+        float* __restrict__ wsP = args.ws + (long long)(2 * part) * args.N;
         float* __restrict__ wsS = wsP + args.N;
 #pragma unroll
         for (int j = 0; j < BZ; ++j)
@@ -644,7 +728,12 @@ __device__ __forceinline__ void load_mri_xt(const unsigned (&b)[XtCfg<C>::NB],
 // dy's bases.  Per candidate the lane forms C with separable sums (x sums as
 // FMA chains of products, then z pairwise, then y across lanes), then
 // w~ = 2^C, P += w~ L~, S += w~ E; t2 holds 2 T'.
-template <class C, int BX, int BZ, int HW>
+//
+// ROT is how many slabs the planes have moved on since the whole slab was copied
+// (modulo APLANES; see stage_next_xt): MRI plane pz sits in slot (pz + ROT) mod
+// APLANES, CT plane j in slot (j + ROT) mod LPLANES.  The slots of a pair come
+// in one read, so the rotation only names registers, at compile time.
+template <class C, int BX, int BZ, int HW, int ROT>
 __device__ __forceinline__ void xterm_dx_sweep(const unsigned (&b)[XtCfg<C>::NBS],
                                                const float (&t2)[BZ + 2][BX + 2],
                                                float (&P)[BZ][BX], float (&S)[BZ][BX]) {
@@ -655,14 +744,15 @@ __device__ __forceinline__ void xterm_dx_sweep(const unsigned (&b)[XtCfg<C>::NBS
 #pragma unroll
         for (int k = 0; k < X::MPAIRS; ++k) {
             const f32x2 v = pair_at_sweep<C>(b, k, r * C::CW);
-            rows[r][2 * k] = v.x;
-            rows[r][2 * k + 1] = v.y;
+            rows[r][(2 * k + C::APLANES - ROT) % C::APLANES] = v.x;
+            rows[r][(2 * k + 1 + C::APLANES - ROT) % C::APLANES] = v.y;
         }
     };
     f32x2 le[2 * HW + BX][BZ];   // (L~, E) of candidate dx, output i: row dx + i
     auto load_le = [&](int r) {
 #pragma unroll
-        for (int j = 0; j < BZ; ++j) le[r][j] = pair_at_sweep<C>(b, X::MPAIRS + j, (r + 1) * C::CW);
+        for (int j = 0; j < BZ; ++j)
+            le[r][j] = pair_at_sweep<C>(b, X::MPAIRS + (j + ROT) % BZ, (r + 1) * C::CW);
     };
     float w[BZ][BX];
     auto accumulate = [&](int dx) {
@@ -682,29 +772,35 @@ __device__ __forceinline__ void xterm_dx_sweep(const unsigned (&b)[XtCfg<C>::NBS
     for (int dx = 0; dx <= 2 * HW; ++dx) {
         // paired part: sums over x and z, and the sums of the candidate before
         if (dx < 2 * HW) load_row(dx + BX + 2);
-        float c[BZ][BX], ex[BZ + 2][BX];
+        float c[BZ][BX];
+        if constexpr (BX == 2 && BZ == 2) {
+            window_sums_2x2([&](int pz, int i) { return t2[pz][i]; },
+                            [&](int pz, int i) { return rows[dx + i][pz]; }, c);
+        } else {
+            float ex[BZ + 2][BX];
 #pragma unroll
-        for (int pz = 0; pz < BZ + 2; ++pz) {
+            for (int pz = 0; pz < BZ + 2; ++pz) {
 #pragma unroll
-            for (int i = 0; i < BX; i += 2) {
-                float q = t2[pz][i + 1] * rows[dx + i + 1][pz];
-                q = fmaf(t2[pz][i + 2], rows[dx + i + 2][pz], q);
-                ex[pz][i] = fmaf(t2[pz][i], rows[dx + i][pz], q);
-                ex[pz][i + 1] = fmaf(t2[pz][i + 3], rows[dx + i + 3][pz], q);
+                for (int i = 0; i < BX; i += 2) {
+                    float q = t2[pz][i + 1] * rows[dx + i + 1][pz];
+                    q = fmaf(t2[pz][i + 2], rows[dx + i + 2][pz], q);
+                    ex[pz][i] = fmaf(t2[pz][i], rows[dx + i][pz], q);
+                    ex[pz][i + 1] = fmaf(t2[pz][i + 3], rows[dx + i + 3][pz], q);
+                }
             }
+#pragma unroll
+            for (int j = 0; j < BZ; j += 2)
+#pragma unroll
+                for (int i = 0; i < BX; ++i) {
+                    const float q = ex[j + 1][i] + ex[j + 2][i];
+                    c[j][i] = ex[j][i] + q;
+                    c[j + 1][i] = q + ex[j + 3][i];
+                }
         }
         if (dx > 0) {
             accumulate(dx - 1);
             load_le(dx + BX - 1);
         }
-#pragma unroll
-        for (int j = 0; j < BZ; j += 2)
-#pragma unroll
-            for (int i = 0; i < BX; ++i) {
-                const float q = ex[j + 1][i] + ex[j + 2][i];
-                c[j][i] = ex[j][i] + q;
-                c[j + 1][i] = q + ex[j + 3][i];
-            }
         // exclusive part: sums over y and the weights
         issue_first();
 #pragma unroll
@@ -786,6 +882,8 @@ __device__ __forceinline__ int stage_slab_xt(float* __restrict__ lds, const floa
                                              long long plane, int wv, int lane) {
     using X = XtCfg<C>;
     constexpr int RPW = (C::RX + NW - 1) / NW;   // rows per wave and plane
+    wv = opaque(wv);   // see stage_two
+    lane = opaque(lane);
     unsigned long long bad = 0;
     f32x2* __restrict__ lp = reinterpret_cast<f32x2*>(lds);
     int ycl[C::COLCHUNKS];
@@ -869,6 +967,67 @@ __device__ __forceinline__ int stage_slab_xt(float* __restrict__ lds, const floa
     return bad != 0;
 }
 
+// Moves the cross-term slab on by one dz: the last MRI plane (z = zdz + BZ) and
+// the last CT plane's pairs (z = zdz + BZ - 1) into the slots of the planes that
+// leave, MRI slot `mslot` (half of a pair plane) and CT slot `cslot`.  Returns the
+// range flag of stage_slab_xt for the new planes; the caller goes on only from
+// slabs without one, so the planes kept are in range.
+template <class C, int NW>
+__device__ __forceinline__ int stage_next_xt(float* __restrict__ lds, int mslot, int cslot,
+                                             const float* __restrict__ A,
+                                             const f32x2* __restrict__ LE, float scale, int zdz,
+                                             int xs, int ys, int nx, int ny, int nz,
+                                             long long plane, int wv, int lane) {
+    using X = XtCfg<C>;
+    constexpr int RPW = (C::RX + NW - 1) / NW;
+    wv = opaque(wv);   // see stage_two
+    lane = opaque(lane);
+    unsigned long long bad = 0;
+    int ycl[C::COLCHUNKS];
+    bool yin[C::COLCHUNKS];
+    lane_columns<C>(ys, ny, lane, ycl, yin);
+    const int zm = zdz + C::LPLANES, zl = zm - 1;
+    const bool mok = zm >= 0 && zm < nz, lok = zl >= 0 && zl < nz;
+    const long long mo = (long long)clampi(zm, nz) * plane, lo = (long long)clampi(zl, nz) * plane;
+    float v[RPW][C::COLCHUNKS];
+    f32x2 g[RPW][C::COLCHUNKS];
+#pragma unroll
+    for (int r = 0; r < RPW; ++r) {
+        const long long ro = (long long)clampi(xs + wv + r * NW, nx) * ny;
+#pragma unroll
+        for (int cc = 0; cc < C::COLCHUNKS; ++cc) {
+            v[r][cc] = A[mo + ro + ycl[cc]];
+            g[r][cc] = LE[lo + ro + ycl[cc]];
+        }
+    }
+    // every load is issued before the first select (see stage_slab_xt)
+#pragma unroll
+    for (int r = 0; r < RPW; ++r)
+#pragma unroll
+        for (int cc = 0; cc < C::COLCHUNKS; ++cc)
+            asm volatile("" : "+v"(v[r][cc]), "+v"(g[r][cc]));
+    float* __restrict__ mp = lds + 2 * ((mslot >> 1) * C::PS) + (mslot & 1);
+    f32x2* __restrict__ lp = reinterpret_cast<f32x2*>(lds) + (X::MPAIRS + cslot) * C::PS;
+#pragma unroll
+    for (int r = 0; r < RPW; ++r) {
+        const int rr = wv + r * NW;
+        const int xx = xs + rr;
+        const bool xok = rr < C::RX && xx >= 0 && xx < nx;
+#pragma unroll
+        for (int cc = 0; cc < C::COLCHUNKS; ++cc) {
+            const int c = lane + cc * 64;
+            const float t = (xok && mok && yin[cc]) ? v[r][cc] * scale : 0.f;
+            const f32x2 p = (xok && lok && yin[cc]) ? g[r][cc] : f32x2{0.f, 0.f};
+            bad |= __ballot(!(fabsf(t) <= kXtBound)) | __ballot(fabsf(p.x) > kXtLabelBound);
+            if (rr < C::RX && c < C::CW) {
+                mp[2 * (rr * C::CW + c)] = t;
+                lp[rr * C::CW + c] = p;
+            }
+        }
+    }
+    return bad != 0;
+}
+
 // Rewrites the first float of every (L~, E) pair of the slab with the raw CT
 // (zero outside the volume), for the squared-difference weighing of a slab
 // out of the cross-term range.
@@ -919,8 +1078,9 @@ __device__ __forceinline__ void tiled_item_xt(const TiledArgs& args, int item,
                                               float* __restrict__ lds) {
     using C = TiledCfg<W, BX, BZ, NW, HW>;
     using X = XtCfg<C>;
-    const int g = item / args.n_tiles;
-    int t = item - g * args.n_tiles;
+    const int part = item / args.n_tiles;   // (atlas group, part of the window)
+    const int g = part / args.n_split, sp = part - g * args.n_split;
+    int t = item - part * args.n_tiles;
     const int ty = t % args.tiles_y;
     t /= args.tiles_y;
     const int tx = t % args.tiles_x;
@@ -961,6 +1121,8 @@ __device__ __forceinline__ void tiled_item_xt(const TiledArgs& args, int item,
     const int ys = y0 - 1 - HW;
     const int a_begin = g * args.group;
     const int a_end = min(args.n_atlas, a_begin + args.group);
+    const int dz_begin = sp * (2 * HW + 1) / args.n_split - HW;
+    const int dz_end = (sp + 1) * (2 * HW + 1) / args.n_split - HW;
     // 2^-TT per output (1 where the item keeps the squared differences)
     float f[BZ][BX];
 
@@ -970,15 +1132,18 @@ __device__ __forceinline__ void tiled_item_xt(const TiledArgs& args, int item,
         for (int a = a_begin; a < a_end; ++a) {
             const float* __restrict__ A = args.atlas + (long long)a * args.N;
             const float* __restrict__ L = args.label + (long long)a * args.N;
-            for (int dz = -HW; dz <= HW; ++dz) {
+            SlabSlots<C> slots;
+            slots.reset();
+            for (int dz = dz_begin; dz < dz_end; ++dz) {
+                if (dz > dz_begin) slots.advance();
                 __syncthreads();
-                stage_slab<C, NW>(lds, A, L, args.scale, z0 + dz, xs, ys, nx, ny, nz, plane, wv,
-                                  lane);
+                stage_slab<C, NW>(lds, slots, dz == dz_begin, A, L, args.scale, z0 + dz, xs, ys,
+                                  nx, ny, nz, plane, wv, lane);
                 __syncthreads();
                 if (!live) continue;
 #pragma unroll 1
                 for (int dy = 0; dy <= 2 * HW; ++dy)
-                    tiled_dx_sweep<C, BX, BZ, HW>(lds, lane_base + dy, tv, P, S);
+                    tiled_dx_sweep<C, BX, BZ, HW>(lds, lane_base + dy, slots, tv, P, S);
             }
         }
 #pragma unroll
@@ -1004,23 +1169,55 @@ __device__ __forceinline__ void tiled_item_xt(const TiledArgs& args, int item,
 #pragma unroll
             for (int i = 0; i < BX + 2; ++i) tv[pz][i] *= 2.f;
         const unsigned lds0 = lds_byte_address(lds);
+        // one sweep is compiled per rotation of the planes: four for BZ = 2
+        constexpr bool kMoves = BZ == 2;
         for (int a = a_begin; a < a_end; ++a) {
             const float* __restrict__ A = args.atlas + (long long)a * args.N;
             const float* __restrict__ L = args.label + (long long)a * args.N;
             const f32x2* __restrict__ LE = args.le + (long long)a * args.N;
-            for (int dz = -HW; dz <= HW; ++dz) {
-                __syncthreads();
-                const int flag = stage_slab_xt<C, NW>(lds, A, LE, args.scale, z0 + dz, xs, ys, nx,
-                                                      ny, nz, plane, wv, lane);
-                if (__syncthreads_or(flag) == 0) {
+            // Slabs that follow one in range (moved >= 0: by how many dz the
+            // planes have moved on) copy two planes; the others are copied whole.
+            int moved = -1;
+            for (int dz = dz_begin; dz < dz_end; ++dz) {
+                bool ok = false;
+                if (kMoves && moved >= 0) {
+                    ++moved;
+                    __syncthreads();
+                    const int flag = stage_next_xt<C, NW>(
+                        lds, (moved + C::APLANES - 1) % C::APLANES,
+                        (moved + C::LPLANES - 1) % C::LPLANES, A, LE, args.scale, z0 + dz, xs, ys,
+                        nx, ny, nz, plane, wv, lane);
+                    ok = __syncthreads_or(flag) == 0;
+                }
+                if (!ok) {
+                    moved = 0;
+                    __syncthreads();
+                    const int flag = stage_slab_xt<C, NW>(lds, A, LE, args.scale, z0 + dz, xs, ys,
+                                                          nx, ny, nz, plane, wv, lane);
+                    ok = __syncthreads_or(flag) == 0;
+                }
+                if (ok) {
                     if (!live) continue;
+                    auto sweep = [&](auto rot) {
 #pragma unroll 1
-                    for (int dy = 0; dy <= 2 * HW; ++dy) {
-                        unsigned b[X::NBS];
-                        make_bases_sweep<C>(lds0, lane_base + dy, b);
-                        xterm_dx_sweep<C, BX, BZ, HW>(b, tv, P, S);
+                        for (int dy = 0; dy <= 2 * HW; ++dy) {
+                            unsigned b[X::NBS];
+                            make_bases_sweep<C>(lds0, lane_base + dy, b);
+                            xterm_dx_sweep<C, BX, BZ, HW, decltype(rot)::value>(b, tv, P, S);
+                        }
+                    };
+                    if constexpr (!kMoves) {
+                        sweep(std::integral_constant<int, 0>{});
+                    } else {
+                        switch (moved & 3) {   // uniform
+                            case 0: sweep(std::integral_constant<int, 0>{}); break;
+                            case 1: sweep(std::integral_constant<int, 1>{}); break;
+                            case 2: sweep(std::integral_constant<int, 2>{}); break;
+                            default: sweep(std::integral_constant<int, 3>{}); break;
+                        }
                     }
                 } else {
+                    moved = -1;   // the raw CT replaces the pairs
                     restage_ct_raw<C, NW>(lds, L, z0 + dz, xs, ys, nx, ny, nz, plane, wv, lane);
                     __syncthreads();
                     if (!live) continue;
@@ -1043,7 +1240,7 @@ __device__ __forceinline__ void tiled_item_xt(const TiledArgs& args, int item,
     }
 
     if (ly >= 1 && ly <= W - 2 && y < ny - r) {
-        float* __restrict__ wsP = args.ws + (long long)(2 * g) * args.N;
+        float* __restrict__ wsP = args.ws + (long long)(2 * part) * args.N;
         float* __restrict__ wsS = wsP + args.N;
 #pragma unroll
         for (int j = 0; j < BZ; ++j)
@@ -1059,15 +1256,19 @@ __device__ __forceinline__ void tiled_item_xt(const TiledArgs& args, int item,
     }
 }
 
-// Waves per SIMD the registers are kept for.  The 2 x 2 blocks' sweep needs 137
-// registers with the next row's loads in flight; held to 128, four waves stay
-// resident (the spills lie outside the sweep): 15.4 ms against 15.9 with three
-// waves at 222x222x112, n=10, NH=11.  LDS holds the larger blocks to two.
-constexpr int xt_min_waves(int bx, int bz) { return bx * bz <= 4 ? 4 : 2; }
+// Waves per SIMD the registers are kept for: as many as LDS holds, up to five (96
+// registers), for the 2 x 2 blocks, whose sweep takes 106-110 registers left to
+// itself (NH 7 at 160x160x96, n=4: 1.03 ms with five waves, 1.05 with four; NH 5
+// 0.45 and 0.47).  LDS holds the larger blocks to two.
+template <class C>
+constexpr int xt_min_waves() {
+    const int by_lds = kLdsPerCu / XtCfg<C>::LDS_BYTES * C::NWv / 4;
+    return C::BXv * C::BZv > 4 ? 2 : by_lds < 1 ? 1 : by_lds > 5 ? 5 : by_lds;
+}
 
 template <int W, int BX, int BZ, int NW, int HW>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(
-    xt_min_waves(BX, BZ)))) void fuse_tiled_xt(TiledArgs args) {
+    xt_min_waves<TiledCfg<W, BX, BZ, NW, HW>>()))) void fuse_tiled_xt(TiledArgs args) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int item = xcd_contiguous(blockIdx.x, args.n_items);
     if (args.only && !args.only[item]) return;   // uniform over the workgroup
@@ -1078,14 +1279,12 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(
 // host helpers shared by pct_fuse.hip and pct_batch.hip (defined in pct_fuse.hip)
 // ---------------------------------------------------------------------------
 
-constexpr int kLdsPerCu = 160 * 1024;
-
 // The tiled shapes compiled into the library; index = pct_tile_config.id.
 const std::vector<TileShape>& shapes();
 
 // Geometry of `shape_id` for a problem (false if the shape/window has no
 // kernel or does not fit the LDS).
-bool make_geometry(const pct_problem* pb, int shape_id, int group, TileGeometry* g);
+bool make_geometry(const pct_problem* pb, int shape_id, int group, TileGeometry* g, int split = 1);
 
 // Cost model: time of one work item of `shape_id` (relative units, the same
 // for every shape), or -1 where the shape has no geometry for the problem.
@@ -1102,11 +1301,11 @@ int check_device(int* dev_out);
 // The library's per-device workspace, grown to at least `bytes`.
 int ensure_workspace(int dev, size_t bytes, void** ptr);
 
-// Bytes of workspace a tiled run of `shape_id` with `n_groups` atlas groups
-// needs: the partial sums, then for a cross-term shape the (L * 2^-AA, 2^-AA)
+// Bytes of workspace a tiled run of `shape_id` with `n_parts` partial sums per
+// voxel needs: the partial sums, then for a cross-term shape the (L * 2^-AA, 2^-AA)
 // pair of every atlas voxel (at tiled_le_offset).
-size_t tiled_ws_bytes(const pct_problem* pb, int n_groups, int shape_id);
-size_t tiled_le_offset(const pct_problem* pb, int n_groups);
+size_t tiled_ws_bytes(const pct_problem* pb, int n_parts, int shape_id);
+size_t tiled_le_offset(const pct_problem* pb, int n_parts);
 
 // Bytes of workspace the device post chain needs for a volume, and the chain
 // itself on a caller's workspace of at least that size (pct_post.hip).
