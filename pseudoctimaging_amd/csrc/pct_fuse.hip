@@ -394,85 +394,126 @@ bool make_geometry(const pct_problem* pb, int shape_id, int group, TileGeometry*
     return g->n_items < INT_MAX;
 }
 
-// Cost model: issue slots per output-candidate for one lane, including the
-// halo lanes and halo rows, times the number of rounds the grid needs.
-// Relative VALU issue rate a SIMD sustains on this kernel with w resident
-// waves.  Fitted to the tiled kernels measured on MI355X at 222x222x112
-// (n=10, NH=11; n=5, NH=9): one wave per SIMD issues far below the VALU
-// rate, throughput grows with occupancy and saturates around five waves.
-static double simd_efficiency(double w) {
-    if (w <= 1.0) return 0.25 * w;
-    if (w <= 2.0) return 0.25 + 0.30 * (w - 1.0);
-    if (w <= 3.0) return 0.55 + 0.13 * (w - 2.0);
-    if (w <= 4.0) return 0.68 + 0.04 * (w - 3.0);
-    return std::min(0.78, 0.72 + 0.06 * (w - 4.0));
-}
+// ---- cost model -------------------------------------------------------------
+//
+// Time of one fusion call with a tile shape, atlas group and split of the
+// window's dz, in microseconds.  The form is the kernel's: per candidate a wave
+// issues `plain` FP32 instructions, which pair between waves, 2 BZ BX DPP adds
+// and BZ BX exps; per slab it copies rows; an item runs its candidates at the
+// rate one wave alone reaches (latency) or at the SIMD's, whichever is slower for
+// the waves resident; a grid runs floor(items / slots) rounds and a tail.  The
+// coefficients are a least-squares fit on MI355X to 5492 timed (problem, shape,
+// group, split) points of 66 problems: random sizes from 24 to 256 voxels, 1 to
+// 10 atlases, NH 3 to 15, times from 9 us to 15 ms, squared-difference shapes
+// also on data out of the cross-term range.  RMS error 7 %; the configuration
+// the model picks is within 3.3 % of the fastest one timed on average (worst
+// 20 %, at 15 us), where a fixed shape per window and one part were 1.0 to 3.9
+// times slower, the more the smaller the problem.
+namespace model {
+constexpr double kPlain = 5.389, kExp = 2.013;        // cycles, SIMD saturated
+constexpr double kAlone = 5.902, kAlone0 = 42.3;      // cycles per instruction and candidate, one wave
+constexpr double kRow = 53.1, kSlab = 596.0;          // cycles per copied plane row, per slab
+constexpr double kRound = 1003.0;                     // latency of one batch of copies
+constexpr double kWaves = 0.698;                      // exponent of the resident waves
+constexpr double kTail = 0.229;                       // part of a round the last items add
+constexpr double kMhz = 2350.0;
+constexpr double kLaunch = 6.5 + 4.3;                 // kernel and finalize launches
+constexpr double kFinalize = 1.264 * 4 / 4e6;         // per float read or written
+constexpr double kPairs0 = 7.3, kPairs = 1.532 * 16 / 4e6;   // pair pre-pass
+// measured over modelled, by shape
+constexpr double kShape[] = {1.12, 1.12, 1.02, 1.05, 0.96, 0.96, 0.99, 0.96, 0.88, 0.95,
+                             1.00, 0.97, 0.96, 0.99, 0.88, 1.04, 1.07, 1.11, 1.01, 1.06};
+}   // namespace model
 
-// Cost model: VALU issue slots of one item per wave, times the rounds of
-// items the grid needs, divided by the efficiency the occupancy allows.
-// Per (dx, dy) step the instruction count is the fit
-//   1.7 (BZ+2)(BX+2) + 1.5 (BZ+2) BX + 6.5 BZ BX
-// (squared differences, x sums, then z sums, DPP y sums, exp, accumulation
-// per output), within 5% of the compiled kernels; exp issues as four slots.
-double model_item_time(const pct_problem* pb, int shape_id, int group, TileGeometry* geo) {
-    TileGeometry g;
-    if (!make_geometry(pb, shape_id, group, &g)) return -1;
+// Microseconds one item takes with `wgs` workgroups resident per CU.
+static double item_time(int shape_id, const TileGeometry& g, double wgs) {
+    using namespace model;
     const TileShape& s = shapes()[shape_id];
-    const double bx = s.bx, bz = s.bz;
-    const double nh = 2 * g.hw + 1;
-    // cross-term shapes: per step 2 (BZ+2) BX FMA-chain instructions for the
-    // x sums, 1.5 BZ BX for z, 2 BZ BX DPP adds for y, 2 BZ BX FMAs for P and
-    // S, BZ BX exp and one address add; scaled like the fit below (measured:
-    // {32, 2, 2, 4} at 222x222x112, n=10, NH=11 runs at 85 % of its VALU
-    // issue rate, its squared-difference twin at 100 %)
-    const double step = s.form == 1
-                            ? 1.28 / 0.85 * (2.0 * (bz + 2) * bx + 6.5 * bz * bx + 1.0)
-                            : 1.7 * (bz + 2) * (bx + 2) + 1.5 * (bz + 2) * bx + 6.5 * bz * bx +
-                                  3.0 * bz * bx;
-    // staging per dz step: address, load, scale, LDS store per element (the
-    // cross-term slab also loads AA and forms (L~, E) for its CT planes)
-    const int S = 64 / s.seg_width;
-    const double rows = (s.form == 1 ? 3 * bz + 2 : 2 * bz + 2) *
-                        (s.waves * S * s.bx + 2 + 2 * g.hw);
-    const double stage = rows / s.waves * 8.0 * ((s.seg_width + 2 * g.hw + 63) / 64);
-    // one-segment (64-lane) shapes measured about 1.5x slower than their
-    // instruction counts predict
-    const double width_penalty = s.seg_width == 64 ? 1.5 : 1.0;
-    const double wave_time = width_penalty * g.group * nh * (nh * nh * step + stage);
-    const double w = (double)g.wg_per_cu * s.waves / 4.0;  // waves per SIMD
-    if (geo) *geo = g;
-    return wave_time * std::max(1.0, w) / simd_efficiency(w);
+    const double bx = s.bx, bz = s.bz, nh = 2 * g.hw + 1;
+    const bool xt = s.form == 1, moves = !xt || s.bz == 2;   // slabs keep shared planes
+    const double sums = s.bx == 2 && s.bz == 2 ? 20 : 2 * (bz + 2) * bx + 1.5 * bz * bx;
+    const double plain = (xt ? 0 : (bz + 2) * (bx + 2)) + sums + 2 * bz * bx;
+    const double busy = kPlain * plain + kExp * bz * bx;
+    const double alone = kAlone * (plain + 2 * bz * bx) + kExp * bz * bx + kAlone0;
+    const int segs = 64 / s.seg_width;
+    const double rows = (double)(s.waves * segs * s.bx + 2 + 2 * g.hw) / s.waves *
+                        ((s.seg_width + 2 * g.hw + 63) / 64);
+    const double whole = rows * (xt ? 3 * bz + 2 : 2 * bz + 2);
+    const double next = moves ? rows * (xt ? 3 : 2) : whole;
+    const double batches = xt ? 1.5 * bz + 1 : bz + 1;
+    const double slabs = std::ceil(nh / g.n_split);
+    const double copies = kRow * (whole + (slabs - 1) * next) + kSlab * slabs;
+    const double latency = kRound * (batches + (slabs - 1) * (moves ? 1 : batches));
+    const double waves = std::max(wgs * s.waves / 4.0, 0.25);   // resident per SIMD
+    const double cycles =
+        g.group * std::max(slabs * nh * nh * alone + copies + latency,
+                           std::pow(waves, kWaves) * (slabs * nh * nh * busy + copies));
+    return cycles / kMhz * kShape[shape_id];
 }
 
-static double model_cost(const pct_problem* pb, int shape_id, int group, TileGeometry* geo) {
+static double model_cost(const pct_problem* pb, int shape_id, int group, TileGeometry* geo,
+                         int split = 1) {
+    using namespace model;
     TileGeometry g;
-    const double item_time = model_item_time(pb, shape_id, group, &g);
-    if (item_time < 0) return -1;
-    const double rounds = std::ceil((double)g.n_items / ((double)kNumCu * g.wg_per_cu));
+    if (!make_geometry(pb, shape_id, group, &g, split)) return -1;
+    static_assert(sizeof(kShape) / sizeof(kShape[0]) == 20, "one factor per shape");
     if (geo) *geo = g;
-    return rounds * item_time;
+    const double N = (double)pb->nx * pb->ny * pb->nz;
+    const double per_cu = (double)g.n_items / kNumCu, slots = g.wg_per_cu;
+    const double kernel =
+        per_cu <= slots ? item_time(shape_id, g, std::max(1.0, std::ceil(per_cu)))
+                        : (per_cu / slots + kTail) * item_time(shape_id, g, slots);
+    double us = kernel + kLaunch + kFinalize * N * (1 + 2 * g.n_parts());
+    if (shapes()[shape_id].form == 1) us += kPairs0 + kPairs * N * pb->n_atlas;
+    return us;
 }
 
-// Tile shape that measured fastest on MI355X for a half window, or -1 where
-// the cost model decides.  Autotuning at 222x222x112 (n=10, NH=11; n=5 and
-// 7, NH=11), 192x192x96 and 256x256x128 (NH=9), 160x160x96 and 128x128x64
-// (NH=7): the analytic model is within about 15 % of the measured times,
-// while the best shapes of a window lie within 5 % of each other.
-int preferred_shape(int hw) {
-    switch (hw) {
-        // every shape timed at group 1 and 2 on one box (ms): NH 7: the
-        // cross-term {32, 2, 2, 4} (16) 0.318 against 0.312 for {64, 2, 2, 4}
-        // (19) at 160x160x96, n=1, and 0.928 against 0.946 at 128x128x64,
-        // n=10; NH 9: 19 2.124 against 2.366 for 16 at 192x192x96, n=3, and
-        // 16.65 against 17.03 at 256x256x128, n=10; NH 11: 16 8.93 and
-        // 17.13 at 222x222x112, n=5 and 10, against 9.03 and 17.79 for
-        // {32, 2, 2, 8} (17) and 9.85 and 19.62 for the best
-        // squared-difference shape
-        case 3: return 16;
-        case 4: return 19;
-        case 5: return 16;
-        default: return -1;
+double model_class_cost(const std::vector<const pct_problem*>& pbs, int shape_id, int group) {
+    using namespace model;
+    std::vector<TileGeometry> geo(pbs.size());
+    double items = 0, us = 0, slots = 1;
+    for (size_t i = 0; i < pbs.size(); ++i) {
+        if (!make_geometry(pbs[i], shape_id, std::min(group, pbs[i]->n_atlas), &geo[i])) return -1;
+        items += (double)geo[i].n_items;
+        slots = geo[i].wg_per_cu;
     }
+    const double wgs = std::min(slots, std::max(1.0, std::ceil(items / kNumCu)));
+    double rounds = 0, longest = 0;
+    for (size_t i = 0; i < pbs.size(); ++i) {
+        const double t = item_time(shape_id, geo[i], wgs);
+        rounds += (double)geo[i].n_items / (kNumCu * wgs) * t;
+        longest = std::max(longest, t);
+        const double N = (double)pbs[i]->nx * pbs[i]->ny * pbs[i]->nz;
+        us += kFinalize * N * (1 + 2 * geo[i].n_parts());
+        if (shapes()[shape_id].form == 1) us += kPairs0 + kPairs * N * pbs[i]->n_atlas;
+    }
+    return us + std::max(longest, rounds + kTail * longest);
+}
+
+// Whether MRI values of about unit range lie in the cross-term range.  The
+// library cannot know the values when it picks a shape; outside the range the
+// cross-term shapes fall back to squared differences item by item, slower than
+// the squared-difference shapes made for them (128x128x64, n=4, NH 5, sigma 0.25:
+// 241 us against 169).
+static bool unit_range_in_bound(const pct_problem* pb) {
+    return std::sqrt(1.4426950408889634 / problem_divisor(pb)) <= (double)kXtBound;
+}
+
+// Candidate splits of the window: whole, halves, thirds, pairs of dz and single
+// ones.  The partial sums of a split may not need more memory than 256 MiB (or
+// than the groups alone).  Groups are of one atlas: several to an item save up to
+// 2 % from NH 7 on and 9 % at NH 3 (fewer partial sums), but one sum over ten
+// atlases rounds five times as far off, and a host-buffer call copies the next
+// group while one runs.
+static std::vector<int> candidate_splits(const pct_problem* pb, int group) {
+    const int nh = 2 * ((pb->nh - 1) / 2) + 1;
+    const double per_part = 8.0 * pb->nx * pb->ny * pb->nz *
+                            ((pb->n_atlas + group - 1) / group);
+    std::vector<int> out;
+    for (int s : {1, 2, 3, (nh + 1) / 2, nh})
+        if (s <= nh && (out.empty() || s > out.back()) && (s == 1 || s * per_part <= 268435456.0))
+            out.push_back(s);
+    return out;
 }
 
 struct ShapeKey {
@@ -482,52 +523,69 @@ struct ShapeKey {
     }
 };
 
+struct Config {
+    int shape_id = -1, group = 1, split = 1;
+};
+
 static std::mutex g_cfg_mutex;
-static std::map<ShapeKey, std::pair<int, int>> g_tuned;   // shape -> (shape_id, group)
+static std::map<ShapeKey, Config> g_tuned;
+// the model's choices, so that a call costs a lookup and not 100 evaluations
+// (about 10 us); cleared when it holds kPlanned of them
+static std::map<std::pair<ShapeKey, bool>, Config> g_planned;
+constexpr size_t kPlanned = 256;
 static int g_forced_id = -1, g_forced_group = 0;
 
-static bool choose(const pct_problem* pb, int* shape_id, int* group, double* cost,
-                   TileGeometry* geo) {
-    {
-        std::lock_guard<std::mutex> lk(g_cfg_mutex);
-        if (g_forced_id >= 0) {
-            *shape_id = g_forced_id;
-            *group = g_forced_group > 0 ? g_forced_group : 1;
-            double c = model_cost(pb, *shape_id, *group, geo);
-            if (cost) *cost = c;
-            return c >= 0;
-        }
-        auto it = g_tuned.find(ShapeKey{pb->nx, pb->ny, pb->nz, pb->n_atlas, pb->nh});
-        if (it != g_tuned.end()) {
-            *shape_id = it->second.first;
-            *group = it->second.second;
-            double c = model_cost(pb, *shape_id, *group, geo);
-            if (cost) *cost = c;
-            return c >= 0;
-        }
-    }
-    // a measured preference for the window fixes the shape and the model
-    // picks the atlas group; without one (or where it does not fit) the model
-    // picks both
-    const int pref = preferred_shape((pb->nh - 1) / 2);
-    double best = -1;
-    for (int pass = pref >= 0 ? 0 : 1; pass < 2 && best < 0; ++pass)
+static Config model_choice(const pct_problem* pb, bool xt, bool* known) {
+    Config best;
+    double best_us = -1;
+    *known = true;
+    for (int pass = 0; pass < 2 && best_us < 0; ++pass)   // any shape where none fits
         for (int sid = 0; sid < (int)shapes().size(); ++sid) {
-            if (pass == 0 && sid != pref) continue;
-            for (int grp = 1; grp <= pb->n_atlas; ++grp) {
-                TileGeometry g;
-                const double c = model_cost(pb, sid, grp, &g);
-                if (c < 0) continue;
-                if (best < 0 || c < best * 0.999) {
-                    best = c;
-                    *shape_id = sid;
-                    *group = grp;
-                    if (geo) *geo = g;
+            if (pass == 0 && !xt && shapes()[sid].form == 1) continue;
+            for (int sp : candidate_splits(pb, 1)) {
+                const double us = model_cost(pb, sid, 1, nullptr, sp);
+                if (us < 0) continue;
+                if (best_us < 0 || us < best_us * 0.999) {
+                    best_us = us;
+                    best = Config{sid, 1, sp};
                 }
             }
         }
-    if (cost) *cost = best;
-    return best >= 0;
+    if (best.shape_id >= 0) *known = find_entry(best.shape_id, (pb->nh - 1) / 2)->occupancy > 0;
+    return best;
+}
+
+// The configuration of a problem: forced, tuned, or the model's.
+static bool choose(const pct_problem* pb, int* shape_id, double* cost, TileGeometry* geo) {
+    Config c;
+    const ShapeKey key{pb->nx, pb->ny, pb->nz, pb->n_atlas, pb->nh};
+    {
+        std::lock_guard<std::mutex> lk(g_cfg_mutex);
+        if (g_forced_id >= 0) {
+            c = Config{g_forced_id, g_forced_group > 0 ? g_forced_group : 1, 1};
+        } else if (auto it = g_tuned.find(key); it != g_tuned.end()) {
+            c = it->second;
+        } else {
+            const bool xt = unit_range_in_bound(pb);
+            const auto pk = std::make_pair(key, xt);
+            const auto pl = g_planned.find(pk);
+            if (pl != g_planned.end()) {
+                c = pl->second;
+            } else {
+                bool known = false;   // whether a device's occupancy went into it
+                c = model_choice(pb, xt, &known);
+                if (known) {
+                    if (g_planned.size() >= kPlanned) g_planned.clear();
+                    g_planned.emplace(pk, c);
+                }
+            }
+        }
+    }
+    if (c.shape_id < 0) return false;
+    *shape_id = c.shape_id;
+    if (!cost) return make_geometry(pb, c.shape_id, c.group, geo, c.split);
+    *cost = model_cost(pb, c.shape_id, c.group, geo, c.split);
+    return *cost >= 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -831,9 +889,9 @@ extern "C" int pct_normalize_labels_dev(float* d_label, size_t n, pct_stream_t s
 extern "C" size_t pct_fuse_workspace_size(const pct_problem* pb, int choice) {
     if (validate_problem(pb) != PCT_OK) return 0;
     if (!is_tiled_choice(pb, choice)) return 0;
-    int sid = 0, grp = 1;
+    int sid = 0;
     TileGeometry g;
-    if (!choose(pb, &sid, &grp, nullptr, &g)) return 0;
+    if (!choose(pb, &sid, nullptr, &g)) return 0;
     return tiled_ws_bytes(pb, g.n_parts(), sid);
 }
 
@@ -848,9 +906,9 @@ static int fuse_dev_impl(const pct_problem* pb, const float* img, const float* a
     rc = check_device(&dev);
     if (rc) return rc;
     if (!is_tiled_choice(pb, choice)) return launch_direct(pb, img, atlas, label, out, stream);
-    int sid = 0, grp = 1;
+    int sid = 0;
     TileGeometry g;
-    if (!choose(pb, &sid, &grp, nullptr, &g)) return PCT_ERR_UNSUPPORTED;
+    if (!choose(pb, &sid, nullptr, &g)) return PCT_ERR_UNSUPPORTED;
     const size_t need = tiled_ws_bytes(pb, g.n_parts(), sid);
     if (own_ws) {
         rc = ensure_workspace(dev, need, &ws);
@@ -908,17 +966,8 @@ static int scratch_address(int dev, void** ptr) {
     return PCT_OK;
 }
 
-// The squared-difference shape with one atlas group: the window's measured
-// squared-difference preference where it fits, else the cost model's choice
-// among squared-difference shapes.
+// The squared-difference shape the model picks for one atlas group.
 static bool choose_noalloc(const pct_problem* pb, int* shape_id, TileGeometry* geo) {
-    static const int kSquaredPref[kMaxTiledHalfWindow + 1] = {-1, -1, -1, 11, 9, 7, -1, -1};
-    const int hw = (pb->nh - 1) / 2;
-    const int pref = hw >= 1 && hw <= kMaxTiledHalfWindow ? kSquaredPref[hw] : -1;
-    if (pref >= 0 && make_geometry(pb, pref, pb->n_atlas, geo)) {
-        *shape_id = pref;
-        return true;
-    }
     double best = -1;
     for (int sid = 0; sid < (int)shapes().size(); ++sid) {
         if (is_xterm_shape(sid)) continue;
@@ -1161,9 +1210,9 @@ static int fuse_host_impl(const pct_problem* pb, const float* img, const float* 
     rc = prepare_host_state(st, N, NA);
     if (rc) return rc;
     hipStream_t s = st.compute, cs = st.copy;
-    int sid = 0, grp = 1;
+    int sid = 0;
     TileGeometry g;
-    const bool tiled = is_tiled_choice(pb, choice) && choose(pb, &sid, &grp, nullptr, &g);
+    const bool tiled = is_tiled_choice(pb, choice) && choose(pb, &sid, nullptr, &g);
     void* ws = nullptr;
     {
         size_t need = post ? postprocess_ws_bytes(pb->nh, pb->nx, pb->ny, pb->nz) : 0;
@@ -1272,8 +1321,7 @@ extern "C" int pct_pseudo_ct_host(const pct_problem* pb, const float* img, const
 
 extern "C" int pct_tile_config_count(void) { return (int)shapes().size(); }
 
-static void fill_config(const pct_problem* pb, int sid, int grp, double cost,
-                        const TileGeometry& g, pct_tile_config* out) {
+static void fill_config(int sid, double cost, const TileGeometry& g, pct_tile_config* out) {
     const TileShape& s = shapes()[sid];
     out->id = sid;
     out->seg_width = s.seg_width;
@@ -1286,19 +1334,17 @@ static void fill_config(const pct_problem* pb, int sid, int grp, double cost,
     out->est_cost = cost;
     out->measured_ms = -1;
     out->form = s.form;
-    (void)pb;
-    (void)grp;
 }
 
 extern "C" int pct_tile_config_choose(const pct_problem* pb, pct_tile_config* out) {
     int rc = validate_problem(pb);
     if (rc) return rc;
     if (!out) return PCT_ERR_INVALID;
-    int sid = 0, grp = 1;
+    int sid = 0;
     double cost = 0;
     TileGeometry g;
-    if (!choose(pb, &sid, &grp, &cost, &g)) return PCT_ERR_UNSUPPORTED;
-    fill_config(pb, sid, grp, cost, g, out);
+    if (!choose(pb, &sid, &cost, &g)) return PCT_ERR_UNSUPPORTED;
+    fill_config(sid, cost, g, out);
     return PCT_OK;
 }
 
@@ -1325,27 +1371,26 @@ extern "C" int pct_autotune(const pct_problem* pb, const float* d_img, const flo
     hipEvent_t e0, e1;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) return PCT_ERR_HIP;
     double best_ms = -1;
-    int best_sid = -1, best_grp = 1;
+    Config best_c;
     TileGeometry best_g;
-    // candidate groups: 1, the model's choice per shape, and n
+    // per shape: groups of one atlas and of all, and the model's split
     for (int sid = 0; sid < (int)shapes().size(); ++sid) {
-        std::vector<int> groups = {1, pb->n_atlas};
+        std::vector<Config> tries = {{sid, 1, 1}};
+        if (pb->n_atlas > 1) tries.push_back({sid, pb->n_atlas, 1});
         double bc = -1;
-        int bg = 1;
-        for (int grp = 1; grp <= pb->n_atlas; ++grp) {
-            double c = model_cost(pb, sid, grp, nullptr);
+        Config m;
+        for (int sp : candidate_splits(pb, 1)) {
+            const double c = model_cost(pb, sid, 1, nullptr, sp);
             if (c >= 0 && (bc < 0 || c < bc * 0.999)) {
                 bc = c;
-                bg = grp;
+                m = Config{sid, 1, sp};
             }
         }
         if (bc < 0) continue;
-        groups.push_back(bg);
-        std::sort(groups.begin(), groups.end());
-        groups.erase(std::unique(groups.begin(), groups.end()), groups.end());
-        for (int grp : groups) {
+        if (m.split != 1) tries.push_back(m);
+        for (const Config& t : tries) {
             TileGeometry g;
-            if (!make_geometry(pb, sid, grp, &g)) continue;
+            if (!make_geometry(pb, t.shape_id, t.group, &g, t.split)) continue;
             void* ws = nullptr;
             const size_t need = tiled_ws_bytes(pb, g.n_parts(), sid);
             rc = ensure_workspace(dev, need, &ws);
@@ -1364,8 +1409,7 @@ extern "C" int pct_autotune(const pct_problem* pb, const float* d_img, const flo
             ms /= reps;
             if (best_ms < 0 || ms < best_ms) {
                 best_ms = ms;
-                best_sid = sid;
-                best_grp = grp;
+                best_c = t;
                 best_g = g;
             }
         }
@@ -1374,13 +1418,14 @@ extern "C" int pct_autotune(const pct_problem* pb, const float* d_img, const flo
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc) return rc;
-    if (best_sid < 0) return PCT_ERR_UNSUPPORTED;
+    if (best_c.shape_id < 0) return PCT_ERR_UNSUPPORTED;
     {
         std::lock_guard<std::mutex> lk(g_cfg_mutex);
-        g_tuned[ShapeKey{pb->nx, pb->ny, pb->nz, pb->n_atlas, pb->nh}] = {best_sid, best_grp};
+        g_tuned[ShapeKey{pb->nx, pb->ny, pb->nz, pb->n_atlas, pb->nh}] = best_c;
     }
     if (best) {
-        fill_config(pb, best_sid, best_grp, model_cost(pb, best_sid, best_grp, nullptr), best_g,
+        fill_config(best_c.shape_id,
+                    model_cost(pb, best_c.shape_id, best_c.group, nullptr, best_c.split), best_g,
                     best);
         best->measured_ms = best_ms;
     }

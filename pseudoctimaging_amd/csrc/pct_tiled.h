@@ -327,32 +327,39 @@ __device__ __forceinline__ void stage_two(float* __restrict__ lds, const float* 
     float v[2][RPW][C::COLCHUNKS];
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
-        const bool zok = z[q] >= 0 && z[q] < nz;
         const float* __restrict__ sz = src[q] + (long long)clampi(z[q], nz) * plane;
 #pragma unroll
         for (int k = 0; k < RPW; ++k) {
-            const int rr = wv + k * NW;
-            const int xx = xs + rr;
-            const bool xok = zok && rr < C::RX && xx >= 0 && xx < nx;
-            const float* __restrict__ sr = sz + (long long)clampi(xx, nx) * ny;
+            const float* __restrict__ sr = sz + (long long)clampi(xs + wv + k * NW, nx) * ny;
 #pragma unroll
-            for (int cc = 0; cc < C::COLCHUNKS; ++cc) {
-                const float raw = sr[ycl[cc]];
-                v[q][k][cc] = (xok && yin[cc]) ? raw * mul[q] : 0.f;
-            }
+            for (int cc = 0; cc < C::COLCHUNKS; ++cc) v[q][k][cc] = sr[ycl[cc]];
         }
     }
+    // every load is issued before the first select: without the barrier the
+    // compiler moves each load under its own branch and waits for it there
 #pragma unroll
     for (int q = 0; q < 2; ++q)
 #pragma unroll
+        for (int k = 0; k < RPW; ++k)
+#pragma unroll
+            for (int cc = 0; cc < C::COLCHUNKS; ++cc) asm volatile("" : "+v"(v[q][k][cc]));
+    const int to = wv * C::CW + lane;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const bool zok = z[q] >= 0 && z[q] < nz;
+#pragma unroll
         for (int k = 0; k < RPW; ++k) {
-            const int rr = wv + k * NW;
+            const int xx = xs + wv + k * NW;
+            const bool xok = zok && xx >= 0 && xx < nx;
+            const bool in_slab = (k + 1) * NW <= C::RX || wv + k * NW < C::RX;
 #pragma unroll
             for (int cc = 0; cc < C::COLCHUNKS; ++cc) {
-                const int c = lane + cc * 64;
-                if (rr < C::RX && c < C::CW) lds[at[q] + rr * C::CW + c] = v[q][k][cc];
+                const float t = (xok && yin[cc]) ? v[q][k][cc] * mul[q] : 0.f;
+                if (in_slab && ((cc + 1) * 64 <= C::CW || lane + cc * 64 < C::CW))
+                    lds[at[q] + to + k * NW * C::CW + cc * 64] = t;
             }
         }
+    }
 }
 
 // The slab of one (atlas, dz): MRI plane p at z = zdz-1+p (scaled), CT plane j
@@ -896,18 +903,32 @@ __device__ __forceinline__ int stage_slab_xt(float* __restrict__ lds, const floa
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int zz = zdz - 1 + 2 * k + h;
-            const bool zok = zz >= 0 && zz < nz;
             const float* __restrict__ Az = A + (long long)clampi(zz, nz) * plane;
+#pragma unroll
+            for (int r = 0; r < RPW; ++r) {
+                const float* __restrict__ Ar =
+                    Az + (long long)clampi(xs + wv + r * NW, nx) * ny;
+#pragma unroll
+                for (int cc = 0; cc < C::COLCHUNKS; ++cc) v[r][cc][h] = Ar[ycl[cc]];
+            }
+        }
+        // every load is issued before the first select (see stage_two)
+#pragma unroll
+        for (int r = 0; r < RPW; ++r)
+#pragma unroll
+            for (int cc = 0; cc < C::COLCHUNKS; ++cc) asm volatile("" : "+v"(v[r][cc]));
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int zz = zdz - 1 + 2 * k + h;
+            const bool zok = zz >= 0 && zz < nz;
 #pragma unroll
             for (int r = 0; r < RPW; ++r) {
                 const int rr = wv + r * NW;
                 const int xx = xs + rr;
                 const bool xok = zok && rr < C::RX && xx >= 0 && xx < nx;
-                const float* __restrict__ Ar = Az + (long long)clampi(xx, nx) * ny;
 #pragma unroll
                 for (int cc = 0; cc < C::COLCHUNKS; ++cc) {
-                    const float raw = Ar[ycl[cc]];
-                    const float t = (xok && yin[cc]) ? raw * scale : 0.f;
+                    const float t = (xok && yin[cc]) ? v[r][cc][h] * scale : 0.f;
                     bad |= __ballot(!(fabsf(t) <= kXtBound));
                     v[r][cc][h] = t;
                 }
@@ -1006,22 +1027,22 @@ __device__ __forceinline__ int stage_next_xt(float* __restrict__ lds, int mslot,
 #pragma unroll
         for (int cc = 0; cc < C::COLCHUNKS; ++cc)
             asm volatile("" : "+v"(v[r][cc]), "+v"(g[r][cc]));
-    float* __restrict__ mp = lds + 2 * ((mslot >> 1) * C::PS) + (mslot & 1);
-    f32x2* __restrict__ lp = reinterpret_cast<f32x2*>(lds) + (X::MPAIRS + cslot) * C::PS;
+    const int to = wv * C::CW + lane;
+    float* __restrict__ mp = lds + 2 * ((mslot >> 1) * C::PS + to) + (mslot & 1);
+    f32x2* __restrict__ lp = reinterpret_cast<f32x2*>(lds) + (X::MPAIRS + cslot) * C::PS + to;
 #pragma unroll
     for (int r = 0; r < RPW; ++r) {
-        const int rr = wv + r * NW;
-        const int xx = xs + rr;
-        const bool xok = rr < C::RX && xx >= 0 && xx < nx;
+        const int xx = xs + wv + r * NW;
+        const bool in_slab = (r + 1) * NW <= C::RX || wv + r * NW < C::RX;
+        const bool xok = in_slab && xx >= 0 && xx < nx;
 #pragma unroll
         for (int cc = 0; cc < C::COLCHUNKS; ++cc) {
-            const int c = lane + cc * 64;
             const float t = (xok && mok && yin[cc]) ? v[r][cc] * scale : 0.f;
             const f32x2 p = (xok && lok && yin[cc]) ? g[r][cc] : f32x2{0.f, 0.f};
             bad |= __ballot(!(fabsf(t) <= kXtBound)) | __ballot(fabsf(p.x) > kXtLabelBound);
-            if (rr < C::RX && c < C::CW) {
-                mp[2 * (rr * C::CW + c)] = t;
-                lp[rr * C::CW + c] = p;
+            if (in_slab && ((cc + 1) * 64 <= C::CW || lane + cc * 64 < C::CW)) {
+                mp[2 * (r * NW * C::CW + cc * 64)] = t;
+                lp[r * NW * C::CW + cc * 64] = p;
             }
         }
     }
@@ -1049,15 +1070,22 @@ __device__ __forceinline__ void restage_ct_raw(float* __restrict__ lds,
         float lv[RPW][C::COLCHUNKS];
 #pragma unroll
         for (int r = 0; r < RPW; ++r) {
+            const float* __restrict__ Lr = Lz + (long long)clampi(xs + wv + r * NW, nx) * ny;
+#pragma unroll
+            for (int cc = 0; cc < C::COLCHUNKS; ++cc) lv[r][cc] = Lr[ycl[cc]];
+        }
+#pragma unroll
+        for (int r = 0; r < RPW; ++r)
+#pragma unroll
+            for (int cc = 0; cc < C::COLCHUNKS; ++cc) asm volatile("" : "+v"(lv[r][cc]));
+#pragma unroll
+        for (int r = 0; r < RPW; ++r) {
             const int rr = wv + r * NW;
             const int xx = xs + rr;
             const bool xok = zok && rr < C::RX && xx >= 0 && xx < nx;
-            const float* __restrict__ Lr = Lz + (long long)clampi(xx, nx) * ny;
 #pragma unroll
-            for (int cc = 0; cc < C::COLCHUNKS; ++cc) {
-                const float raw = Lr[ycl[cc]];
-                lv[r][cc] = (xok && yin[cc]) ? raw : 0.f;
-            }
+            for (int cc = 0; cc < C::COLCHUNKS; ++cc)
+                lv[r][cc] = (xok && yin[cc]) ? lv[r][cc] : 0.f;
         }
 #pragma unroll
         for (int r = 0; r < RPW; ++r) {
@@ -1286,12 +1314,10 @@ const std::vector<TileShape>& shapes();
 // kernel or does not fit the LDS).
 bool make_geometry(const pct_problem* pb, int shape_id, int group, TileGeometry* g, int split = 1);
 
-// Cost model: time of one work item of `shape_id` (relative units, the same
-// for every shape), or -1 where the shape has no geometry for the problem.
-double model_item_time(const pct_problem* pb, int shape_id, int group, TileGeometry* geo);
-
-// Tile shape that measured fastest for a half window, or -1.
-int preferred_shape(int hw);
+// Cost model: microseconds of a batch's window class, its subjects' items pooled
+// on a persistent grid, with this tile shape and atlas group; -1 where the shape
+// has no geometry for one of them.
+double model_class_cost(const std::vector<const pct_problem*>& pbs, int shape_id, int group);
 
 constexpr int kNumCu = 256;
 
