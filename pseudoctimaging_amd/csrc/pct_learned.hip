@@ -1370,33 +1370,33 @@ struct SampleMoments {
 
 // As tiled_step, also summing the CT of the evaluated candidates (Le) and
 // the weights of the lattice samples (Ws); with ERR also the moments of the
-// samples.
+// samples.  The window is read as plane pairs: 16 LDS reads for BX = 2 and BZ =
+// 4, where the planes one by one took 32.
 template <class C, int BX, int BZ, bool SAMPLE, bool ERR>
-__device__ __forceinline__ void pruned_step(const float* __restrict__ lds, int base,
-                                            const float (&tv)[BZ + 2][BX + 2],
+__device__ __forceinline__ void pruned_step(unsigned at, const float (&tv)[BZ + 2][BX + 2],
                                             float (&P)[BZ][BX], float (&S)[BZ][BX],
                                             float (&Le)[BZ][BX], float (&Ws)[BZ][BX],
                                             SampleMoments& m) {
-    constexpr int NBA = (BZ + 2 + C::PPB - 1) / C::PPB;
-    constexpr int NBL = (BZ + C::PPB - 1) / C::PPB;
-    int ba[NBA];
-    int bl[NBL];
+    using X = PairSlab<C>;
+    unsigned b[X::NB];   // LDS byte address of the window's first position
 #pragma unroll
-    for (int b = 0; b < NBA; ++b) ba[b] = b ? opaque(base + b * C::PPB * C::PS) : base;
+    for (int k = 0; k < X::NB; ++k)
+        b[k] = k ? opaque_u(at + 8u * (unsigned)(k * X::PPB * C::PS)) : at;
+    auto pair = [&](int pl, int row) {
+        const lds_pair_t* q = (const lds_pair_t*)(size_t)b[pl / X::PPB];
+        return q[(pl % X::PPB) * C::PS + row * C::CW];
+    };
+    f32x2 a[X::MPAIRS][BX + 2], l2[X::LPAIRS][BX];
 #pragma unroll
-    for (int b = 0; b < NBL; ++b) bl[b] = opaque(base + C::LOFF + b * C::PPB * C::PS);
-    float c[BZ][BX], ct[BZ][BX];
-    squared_sums_xz<BX, BZ>(
-        tv,
-        [&](int pz, int i) {
-            return lds[ba[pz / C::PPB] + (pz % C::PPB) * C::PS + i * C::CW];
-        },
-        c);
+    for (int k = 0; k < X::MPAIRS; ++k)
 #pragma unroll
-    for (int j = 0; j < BZ; ++j)
+        for (int i = 0; i < BX + 2; ++i) a[k][i] = pair(k, i);
 #pragma unroll
-        for (int i = 0; i < BX; ++i)
-            ct[j][i] = lds[bl[j / C::PPB] + (j % C::PPB) * C::PS + (i + 1) * C::CW];
+    for (int k = 0; k < X::LPAIRS; ++k)
+#pragma unroll
+        for (int i = 0; i < BX; ++i) l2[k][i] = pair(X::MPAIRS + k, i + 1);
+    float c[BZ][BX];
+    squared_sums_xz<BX, BZ>(tv, [&](int pz, int i) { return a[pz >> 1][i][pz & 1]; }, c);
     issue_first();
 #pragma unroll
     for (int j = 0; j < BZ; ++j)
@@ -1412,7 +1412,7 @@ __device__ __forceinline__ void pruned_step(const float* __restrict__ lds, int b
     for (int j = 0; j < BZ; ++j)
 #pragma unroll
         for (int i = 0; i < BX; ++i) {
-            const float w = c[j][i], l = ct[j][i];
+            const float w = c[j][i], l = l2[j >> 1][i][j & 1];
             P[j][i] = fmaf(w, l, P[j][i]);
             S[j][i] += w;
             Le[j][i] += l;
@@ -1424,15 +1424,19 @@ __device__ __forceinline__ void pruned_step(const float* __restrict__ lds, int b
         }
 }
 
+// Bound by latency more than by issue: the offsets of a tile lie anywhere in the
+// window, so no sums are shared between them and every plane is staged for a
+// handful of offsets.  What it holds is therefore 4 waves per SIMD (two workgroups
+// per CU hide each other's staging), pair reads, an offset list in registers and a
+// staging that waits once per plane pair.  222x222x112, n = 10, NH = 11, top-32,
+// whole pipeline: 2250 us with 32-bit reads and the list in LDS, 2222 with pairs
+// and the list in memory, 2105 with the list in registers, 2051 with the scale
+// pass batched.
 template <int W, int BX, int BZ, int NW, int HW>
-__global__ __launch_bounds__(NW * 64) void pruned_kernel(PrunedArgs pa) {
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) void pruned_kernel(
+    PrunedArgs pa) {
     using C = TiledCfg<W, BX, BZ, NW, HW>;
-    extern __shared__ float lds[];
-    // the offset list: per dz plane (ascending), the kept offsets, then the
-    // lattice samples that are not kept; each entry's dz and LDS delta
-    __shared__ int odz[kMaxOffsets];
-    __shared__ int odel[kMaxOffsets];
-    __shared__ int is_sample[kMaxOffsets];
+    extern __shared__ __attribute__((aligned(16))) float lds[];
     const TiledArgs& args = pa.t;
     const int item = xcd_contiguous(blockIdx.x, args.n_items);
     if (pa.flag[item]) return;            // full search handles it (uniform)
@@ -1443,16 +1447,19 @@ __global__ __launch_bounds__(NW * 64) void pruned_kernel(PrunedArgs pa) {
     const int tx = t % args.tiles_x;
     const int tz = t / args.tiles_x;
 
+    // the offset list (merge_offsets_kernel): per dz plane (ascending), the kept
+    // offsets, then the lattice samples that are not kept.  Entry k sits in lane
+    // k & 63 of one of two registers and comes out by a lane read: read through
+    // LDS, or from memory, the fields of an entry cost as much latency as its
+    // whole arithmetic.
     const int* __restrict__ mo = pa.merged + (long long)item * kMergedStride;
-    const int hdr = mo[0];
+    const int hdr = __builtin_amdgcn_readfirstlane(mo[0]);
     const int n_offs = hdr & 0xffff, n_samp_eff = hdr >> 16;
-    if ((int)threadIdx.x < n_offs) {   // n_offs <= kMaxOffsets < NW * 64
-        const unsigned e = (unsigned)mo[1 + threadIdx.x];
-        odz[threadIdx.x] = (int)((e >> 16) & 15u) - 8;
-        odel[threadIdx.x] = (int)(e & 0xffffu);
-        is_sample[threadIdx.x] = (int)(e >> 31);
-    }
-    __syncthreads();
+    const int list0 = mo[1 + (threadIdx.x & 63)];
+    const int list1 = mo[min(65 + (int)(threadIdx.x & 63), kMergedStride - 1)];
+    static_assert(kMaxOffsets <= 64 + kMergedStride - 65, "the list fits two registers");
+    auto entry_dz = [](int e) { return ((e >> 16) & 15) - 8; };
+    auto entry_at = [](int e) { return 8u * (unsigned)(e & 0xffff); };   // bytes
 
     const int tid = threadIdx.x;
     const int wv = tid >> 6;
@@ -1478,7 +1485,8 @@ __global__ __launch_bounds__(NW * 64) void pruned_kernel(PrunedArgs pa) {
         for (int i = 0; i < BX; ++i) P[j][i] = S[j][i] = Le[j][i] = Ws[j][i] = 0.f;
     const bool err = pa.max_err > 0.f;   // uniform over the grid
 
-    const int lane_base = sg * BX * C::CW + ly;
+    // LDS byte address of the lane's window at offset (0, 0)
+    const unsigned lane_at = lds_byte_address(lds) + 8u * (unsigned)(sg * BX * C::CW + ly);
     const int xs = x0 - 1 - HW;
     const int ys = y0 - 1 - HW;
     DirectPlan<C, NW> dp;
@@ -1486,21 +1494,27 @@ __global__ __launch_bounds__(NW * 64) void pruned_kernel(PrunedArgs pa) {
     const float* __restrict__ A = args.atlas + (long long)at * args.N;
     const float* __restrict__ L = args.label + (long long)at * args.N;
     const int m = n_offs;
-    int k = 0;
+    auto entry = [&](int i) {
+        return __builtin_amdgcn_readlane(i < 64 ? list0 : list1, i & 63);
+    };
+    int k = 0, e = entry(0);
+    auto advance = [&]() { e = entry(++k); };   // not used where k = m
     while (k < m) {
-        const int dz = odz[k];
+        const int dz = entry_dz(e);
         __syncthreads();
         stage_slab_direct<C, NW>(lds, A, L, args.scale, z0 + dz, nz, plane, wv, dp);
-        for (; k < m && odz[k] == dz && !is_sample[k]; ++k)
-            pruned_step<C, BX, BZ, false, false>(lds, lane_base + odel[k], tv, P, S, Le, Ws, mom);
-        if (err) {
-            for (; k < m && odz[k] == dz; ++k)
-                pruned_step<C, BX, BZ, true, true>(lds, lane_base + odel[k], tv, P, S, Le, Ws,
-                                                   mom);
-        } else {
-            for (; k < m && odz[k] == dz; ++k)
-                pruned_step<C, BX, BZ, true, false>(lds, lane_base + odel[k], tv, P, S, Le, Ws,
-                                                    mom);
+        while (k < m && entry_dz(e) == dz && e >= 0) {
+            const unsigned at = lane_at + entry_at(e);
+            advance();
+            pruned_step<C, BX, BZ, false, false>(at, tv, P, S, Le, Ws, mom);
+        }
+        while (k < m && entry_dz(e) == dz) {
+            const unsigned at = lane_at + entry_at(e);
+            advance();
+            if (err)
+                pruned_step<C, BX, BZ, true, true>(at, tv, P, S, Le, Ws, mom);
+            else
+                pruned_step<C, BX, BZ, true, false>(at, tv, P, S, Le, Ws, mom);
         }
     }
 

@@ -108,13 +108,6 @@ struct TiledCfg {
     static constexpr int LDS_FLOATS = (APLANES + LPLANES) * PS;
     static constexpr int LDS_BYTES = LDS_FLOATS * 4;
     static constexpr int COLCHUNKS = (CW + 63) / 64;
-    // ds_read_b32 takes a 16-bit byte offset: planes are addressed from
-    // several base registers, PPB planes (plus row offsets) per base.
-    // The immediate also carries the candidate's dy (up to 2 HW).
-    static constexpr int PPB = (16383 - (BX + 1) * CW - 2 * HW) / PS + 1;
-    static_assert(PPB >= 1, "one plane must fit an LDS immediate window");
-    static constexpr int NBA = (APLANES + PPB - 1) / PPB;   // base registers, MRI planes
-    static constexpr int NBL = (LPLANES + PPB - 1) / PPB;   // base registers, CT planes
     // the dx sweep's immediates carry the row (up to 2 HW + BX + 1) alone
     static_assert((2 * HW + BX + 1) * CW <= 16383, "rows must fit an LDS immediate");
     static_assert(64 % W == 0, "segment width must divide the wavefront");
@@ -396,17 +389,35 @@ __device__ __forceinline__ void stage_slab(float* __restrict__ lds, const SlabSl
 // Zeros read by lanes whose slab position lies outside the volume.
 __device__ const float kZeros[64] = {};
 
-// The slab of stage_slab, copied with direct global-to-LDS loads
-// (global_load_lds_dword): every lane of a wave instruction fills one of 64
-// consecutive LDS floats of a plane, so a plane is PS/64 instructions, all of
+// The slab of one (atlas, dz) with its planes interleaved in pairs: pair plane k
+// < MPAIRS holds MRI planes 2 k and 2 k + 1, pair plane MPAIRS + k CT planes 2 k
+// and 2 k + 1, so that one 64-bit LDS read returns two planes at a position (a
+// 32-bit read costs as much and returns one).
+template <class C>
+struct PairSlab {
+    static constexpr int MPAIRS = C::APLANES / 2, LPAIRS = C::LPLANES / 2;
+    static_assert(C::APLANES % 2 == 0 && C::LPLANES % 2 == 0, "planes pair up");
+    static constexpr int FLOATS = 2 * C::PS;            // of a pair plane
+    // pair planes per base register: a 64-bit read's 16-bit byte immediate also
+    // carries the row (up to BX + 1)
+    static constexpr int PPB = (8191 - (C::BXv + 1) * C::CW) / C::PS + 1;
+    static_assert(PPB >= 1, "one pair plane must fit an LDS immediate window");
+    static constexpr int NB = (MPAIRS + LPAIRS + PPB - 1) / PPB;
+};
+
+// Copies a pair slab with direct global-to-LDS loads (global_load_lds_dword):
+// every lane of a wave instruction fills one of 64 consecutive LDS floats, even
+// lanes from the first and odd lanes from the second plane of the pair; all of
 // the slab's loads are in flight at once, and no VGPR holds the data.  Wave w
-// copies chunks j = w, w + NW, ... of every plane, so a lane's in-plane
+// copies chunks j = w, w + NW, ... of every pair plane, so a lane's in-plane
 // source offsets depend only on the tile: DirectPlan computes them once per
 // item, and a copy costs one address add per instruction.
 template <class C, int NW>
 struct DirectPlan {
-    static constexpr int CH = (C::PS + 63) / 64;      // 64-float chunks per plane
-    static constexpr int JN = (CH + NW - 1) / NW;     // chunks per wave and plane
+    static constexpr int CH = (2 * C::PS + 63) / 64;  // 64-float chunks per pair plane
+    static constexpr int JN = (CH + NW - 1) / NW;     // chunks per wave and pair plane
+    // whether every lane of every wave has an element in its k-th chunk
+    static constexpr bool all(int k) { return (k + 1) * NW * 64 <= 2 * C::PS; }
     // x * ny + y of the lane's source voxel within a plane, -1 outside the
     // volume (reads zeros), -2 past the end of the plane (no copy)
     int off[JN];
@@ -415,7 +426,7 @@ struct DirectPlan {
 #pragma unroll
         for (int k = 0; k < JN; ++k) {
             const int j = wv + k * NW;
-            const int p = j * 64 + lane;
+            const int p = j * 32 + (lane >> 1);
             const int row = p / C::CW, col = p - (p / C::CW) * C::CW;
             const int xx = xs + row, yy = ys + col;
             int o = -2;
@@ -426,11 +437,11 @@ struct DirectPlan {
     }
 };
 
-// Copies the slab of stage_slab from the unscaled atlas MRI; positions
-// outside the volume read zeros.  Once its own loads have landed, each lane
-// multiplies the MRI positions they wrote by `scale`: the product stage_slab
-// forms before its LDS store (zeros stay zero), so both stagings hold the same
-// bits.  Ends with a workgroup barrier.
+// Copies the pair slab from the unscaled atlas MRI; positions outside the volume
+// read zeros.  Once its own loads have landed, each lane multiplies the MRI
+// positions they wrote by `scale`: the product stage_slab forms before its LDS
+// store (zeros stay zero), so both hold the same values.  Ends with a workgroup
+// barrier.
 template <class C, int NW>
 __device__ __forceinline__ void stage_slab_direct(float* __restrict__ lds,
                                                   const float* __restrict__ A,
@@ -438,37 +449,41 @@ __device__ __forceinline__ void stage_slab_direct(float* __restrict__ lds,
                                                   int zdz, int nz, long long plane, int wv,
                                                   const DirectPlan<C, NW>& dp) {
     typedef __attribute__((address_space(3))) void* lds_ptr;
-    constexpr int NP = C::APLANES + C::LPLANES;
+    using X = PairSlab<C>;
     using P = DirectPlan<C, NW>;
-#pragma unroll 2
-    for (int pl = 0; pl < NP; ++pl) {
-        const bool is_mri = pl < C::APLANES;
-        const int zz = is_mri ? zdz - 1 + pl : zdz + (pl - C::APLANES);
+    const int lane = (int)(threadIdx.x & 63u), half = lane & 1;
+#pragma unroll 1
+    for (int pl = 0; pl < X::MPAIRS + X::LPAIRS; ++pl) {
+        const bool is_mri = pl < X::MPAIRS;
+        const int zz = (is_mri ? zdz - 1 + 2 * pl : zdz + 2 * (pl - X::MPAIRS)) + half;
         const bool zok = zz >= 0 && zz < nz;
         const float* base = (is_mri ? A : L) + (zok ? zz : 0) * plane;
 #pragma unroll
         for (int k = 0; k < P::JN; ++k) {
             const int j = wv + k * NW;
             const int o = dp.off[k];
-            if (o >= -1) {
+            if (P::all(k) || o >= -1) {
                 const float* src = (zok && o >= 0) ? base + o : kZeros;
-                __builtin_amdgcn_global_load_lds(src, (lds_ptr)(lds + pl * C::PS + j * 64), 4,
+                __builtin_amdgcn_global_load_lds(src, (lds_ptr)(lds + pl * X::FLOATS + j * 64), 4,
                                                  0, 0);
             }
         }
     }
     __builtin_amdgcn_s_waitcnt(0);
     __asm__ volatile("" ::: "memory");
-    // lane l of load (plane pl, chunk j) wrote LDS element pl * PS + j * 64 + l
-    const int lane = (int)(threadIdx.x & 63u);
+    // lane l of load (pair plane pl, chunk j) wrote LDS element pl * FLOATS + j *
+    // 64 + l; a pair plane's elements are read together, one latency for all
 #pragma unroll
-    for (int pl = 0; pl < C::APLANES; ++pl)
+    for (int pl = 0; pl < X::MPAIRS; ++pl) {
+        float* q = lds + pl * X::FLOATS + wv * 64 + lane;
+        float v[P::JN];
 #pragma unroll
         for (int k = 0; k < P::JN; ++k)
-            if (dp.off[k] >= -1) {
-                float* q = lds + pl * C::PS + (wv + k * NW) * 64 + lane;
-                *q = *q * scale;
-            }
+            v[k] = P::all(k) || dp.off[k] >= -1 ? q[k * NW * 64] : 0.f;
+#pragma unroll
+        for (int k = 0; k < P::JN; ++k)
+            if (P::all(k) || dp.off[k] >= -1) q[k * NW * 64] = v[k] * scale;
+    }
     __syncthreads();
 }
 
