@@ -164,7 +164,7 @@ __device__ __forceinline__ float neighbourhood_median(const float* arr, int id, 
 // an LDS copy that starts before the wait with what no tile before it changes.
 // A level takes about 810 cycles, the copy after the wait 1900, the release
 // 1700.  222x222x112 with 4.2e6 NaN voxels: 48.2 ms for the one-workgroup sweep
-// (46 us a level), 1.63 ms here, 1.52 of it in fill_tiles_kernel.  Tiles of
+// (46 us a level), 1.56 ms here, 1.52 of it in fill_tiles_kernel.  Tiles of
 // {4, 8, 32} took 2.7 ms (before the early copy), {4, 8, 8} 2.04, {8, 8, 8}
 // 2.22, {4, 16, 8} 2.56; 512 workgroups 1.70.  Polling with acquire loads,
 // which invalidate the caches each time, took 4.6-6.2 ms.
@@ -222,21 +222,10 @@ struct FillState {
     int* diag;        // [n_diag + 1] tiles per diagonal, then their places
 };
 
-__global__ void fill_clear_kernel(FillState st, int n_diag) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t <= n_diag) st.diag[t] = 0;
-    if (t == 0) *st.next = *st.n_busy = *st.left = 0;
-}
-
-// One wave per tile: whether it holds an interior NaN voxel.
-constexpr int kScanWaves = 4;
-__global__ __launch_bounds__(kScanWaves * 64) void fill_scan_kernel(
-    const float* __restrict__ arr, FillTiles f, FillState st) {
+// Whether tile (i, j, k) holds an interior NaN voxel; one wave per tile.
+__device__ __forceinline__ bool tile_has_nan(const float* __restrict__ arr, const FillTiles& f,
+                                             int i, int j, int k) {
     const int lane = threadIdx.x & 63;
-    const int tile = blockIdx.x * kScanWaves + (threadIdx.x >> 6);
-    if (tile >= f.n_tiles) return;   // per wave; no barrier below
-    int i, j, k;
-    tile_coords(f, tile, &i, &j, &k);
     constexpr int kLoads = kTZ * kTX * kTY / 64;
     bool nan = false;
 #pragma unroll 8
@@ -251,20 +240,49 @@ __global__ __launch_bounds__(kScanWaves * 64) void fill_scan_kernel(
         const float v = arr[in ? id : 0];
         nan |= in && isnan(v);
     }
-    const bool busy = __ballot(nan) != 0;
-    if (lane == 0) {
+    return __ballot(nan) != 0;
+}
+
+// The tiles with work, listed by diagonal.  Up to kPlanDiags diagonals and
+// kPlanTiles tiles one workgroup does it with the histogram in LDS, after a scan
+// kernel or, for up to kPlanScan tiles, with the scan as well: the chain then
+// takes 4 launches on the smallest volumes and 5 on others, where clearing,
+// counting, placing and listing as kernels of their own make it 7 (28x26x24, 0.2 %
+// NaN: 28.0 -> 21.2 us; 222x222x112, 4.2e6 NaN: 1.62 -> 1.56 ms).  Past that one
+// workgroup would be the slower one (or its LDS too small) and those kernels run.
+constexpr int kPlanDiags = 4096, kPlanTiles = 1 << 16, kPlanScan = 256, kPlanThreads = 1024;
+
+// The general path: the counters, the scan with its histogram, the places of the
+// diagonals and the list.
+__global__ void fill_clear_kernel(FillState st, int n_diag) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t <= n_diag) st.diag[t] = 0;
+    if (t == 0) *st.next = *st.n_busy = *st.left = 0;
+}
+
+constexpr int kScanWaves = 4;
+template <bool COUNT>   // COUNT: into the histogram too
+__global__ __launch_bounds__(kScanWaves * 64) void fill_scan_kernel(
+    const float* __restrict__ arr, FillTiles f, FillState st) {
+    const int tile = blockIdx.x * kScanWaves + (threadIdx.x >> 6);
+    if (tile >= f.n_tiles) return;   // per wave; no barrier below
+    int i, j, k;
+    tile_coords(f, tile, &i, &j, &k);
+    const bool busy = tile_has_nan(arr, f, i, j, k);
+    if ((threadIdx.x & 63) == 0) {
         st.done[tile] = busy ? 0 : 1;
-        if (busy) atomicAdd(st.diag + (i + j + k), 1);
+        if (COUNT && busy) atomicAdd(st.diag + (i + j + k), 1);
     }
 }
 
-// Places of the diagonals in the order list (exclusive prefix of the counts).
-__global__ __launch_bounds__(1024) void fill_places_kernel(FillState st, int n_diag) {
-    __shared__ int wtot[16];
-    const int seg = (n_diag + 1023) / 1024;
-    const int b0 = min(n_diag, (int)threadIdx.x * seg), b1 = min(n_diag, b0 + seg);
+// Exclusive prefix of the n counts at `diag` by a workgroup of kPlanThreads, in
+// place; returns the total.
+__device__ __forceinline__ int diagonal_places(int* diag, int n) {
+    __shared__ int wtot[kPlanThreads / 64];
+    const int seg = (n + kPlanThreads - 1) / kPlanThreads;
+    const int b0 = min(n, (int)threadIdx.x * seg), b1 = min(n, b0 + seg);
     int own = 0;
-    for (int b = b0; b < b1; ++b) own += st.diag[b];
+    for (int b = b0; b < b1; ++b) own += diag[b];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     int incl = own;
 #pragma unroll
@@ -274,15 +292,23 @@ __global__ __launch_bounds__(1024) void fill_places_kernel(FillState st, int n_d
     }
     if (lane == 63) wtot[w] = incl;
     __syncthreads();
-    int before = 0;
-    for (int j = 0; j < w; ++j) before += wtot[j];
+    int before = 0, total = 0;
+    for (int j = 0; j < kPlanThreads / 64; ++j) {
+        before += j < w ? wtot[j] : 0;
+        total += wtot[j];
+    }
     int run = before + incl - own;
     for (int b = b0; b < b1; ++b) {
-        const int c = st.diag[b];
-        st.diag[b] = run;
+        const int c = diag[b];
+        diag[b] = run;
         run += c;
     }
-    if (threadIdx.x == 1023) *st.n_busy = before + incl;
+    return total;
+}
+
+__global__ __launch_bounds__(kPlanThreads) void fill_places_kernel(FillState st, int n_diag) {
+    const int total = diagonal_places(st.diag, n_diag);
+    if (threadIdx.x == 0) *st.n_busy = total;
 }
 
 // Busy tiles into the list by diagonal (any order within one).
@@ -292,6 +318,44 @@ __global__ void fill_order_kernel(FillTiles f, FillState st) {
     int i, j, k;
     tile_coords(f, tile, &i, &j, &k);
     st.order[atomicAdd(st.diag + (i + j + k), 1)] = tile;
+}
+
+// The whole plan in one workgroup (n_diag <= kPlanDiags).  SCAN: f.n_tiles <=
+// kPlanScan tiles are scanned here; otherwise fill_scan_kernel left the flags.
+template <bool SCAN>
+__global__ __launch_bounds__(kPlanThreads) void fill_plan_kernel(const float* __restrict__ arr,
+                                                                 FillTiles f, FillState st) {
+    __shared__ int diag[kPlanDiags];
+    __shared__ int busy[SCAN ? kPlanScan : 1];
+    for (int d = threadIdx.x; d < f.n_diag; d += kPlanThreads) diag[d] = 0;
+    if (SCAN)
+        for (int t = threadIdx.x >> 6; t < f.n_tiles; t += kPlanThreads / 64) {
+            int i, j, k;
+            tile_coords(f, t, &i, &j, &k);
+            const bool nan = tile_has_nan(arr, f, i, j, k);
+            if ((threadIdx.x & 63) == 0) {
+                busy[t] = nan ? 1 : 0;
+                st.done[t] = nan ? 0 : 1;
+            }
+        }
+    __syncthreads();
+    auto each = [&](auto use) {   // the busy tiles' (tile, diagonal)
+        for (int t = threadIdx.x; t < f.n_tiles; t += kPlanThreads) {
+            if (SCAN ? !busy[t] : st.done[t] != 0) continue;
+            int i, j, k;
+            tile_coords(f, t, &i, &j, &k);
+            use(t, i + j + k);
+        }
+    };
+    each([&](int, int d) { atomicAdd(&diag[d], 1); });
+    __syncthreads();
+    const int total = diagonal_places(diag, f.n_diag);
+    __syncthreads();
+    each([&](int t, int d) { st.order[atomicAdd(&diag[d], 1)] = t; });
+    if (threadIdx.x == 0) {
+        *st.next = *st.left = 0;
+        *st.n_busy = total;
+    }
 }
 
 // Lane exchanges within the eight lanes of a voxel.
@@ -746,13 +810,24 @@ static int enqueue_fill(int nh, int nx, int ny, int nz, float* d_arr, void* ws, 
     st.done = reinterpret_cast<int*>(w + lay.done);
     st.order = reinterpret_cast<int*>(w + lay.order);
     st.diag = reinterpret_cast<int*>(w + lay.diag);
-    hipLaunchKernelGGL(fill_clear_kernel, dim3((unsigned)(f.n_diag / 256 + 1)), dim3(256), 0, s,
-                       st, f.n_diag);
-    hipLaunchKernelGGL(fill_scan_kernel, dim3((unsigned)((f.n_tiles + kScanWaves - 1) / kScanWaves)),
-                       dim3(kScanWaves * 64), 0, s, d_arr, f, st);
-    hipLaunchKernelGGL(fill_places_kernel, dim3(1), dim3(1024), 0, s, st, f.n_diag);
-    hipLaunchKernelGGL(fill_order_kernel, dim3((unsigned)((f.n_tiles + 255) / 256)), dim3(256), 0,
-                       s, f, st);
+    const dim3 scan_grid((unsigned)((f.n_tiles + kScanWaves - 1) / kScanWaves));
+    if (f.n_diag > kPlanDiags || f.n_tiles > kPlanTiles) {
+        hipLaunchKernelGGL(fill_clear_kernel, dim3((unsigned)(f.n_diag / 256 + 1)), dim3(256), 0,
+                           s, st, f.n_diag);
+        hipLaunchKernelGGL(fill_scan_kernel<true>, scan_grid, dim3(kScanWaves * 64), 0, s, d_arr,
+                           f, st);
+        hipLaunchKernelGGL(fill_places_kernel, dim3(1), dim3(kPlanThreads), 0, s, st, f.n_diag);
+        hipLaunchKernelGGL(fill_order_kernel, dim3((unsigned)((f.n_tiles + 255) / 256)),
+                           dim3(256), 0, s, f, st);
+    } else if (f.n_tiles > kPlanScan) {
+        hipLaunchKernelGGL(fill_scan_kernel<false>, scan_grid, dim3(kScanWaves * 64), 0, s, d_arr,
+                           f, st);
+        hipLaunchKernelGGL(fill_plan_kernel<false>, dim3(1), dim3(kPlanThreads), 0, s, d_arr, f,
+                           st);
+    } else {
+        hipLaunchKernelGGL(fill_plan_kernel<true>, dim3(1), dim3(kPlanThreads), 0, s, d_arr, f,
+                           st);
+    }
     hipLaunchKernelGGL(fill_tiles_kernel, dim3((unsigned)std::min(f.n_tiles, kTileWgs)),
                        dim3(kTileThreads), 0, s, d_arr, f, st, la);
     hipLaunchKernelGGL(nan_fill_levels_kernel, dim3(1), dim3(kFillThreads), 0, s, d_arr, la, lb,

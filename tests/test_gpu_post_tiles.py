@@ -43,3 +43,21 @@ def test_tiled_fill_matches_host(gpu, interior, kind, nh):
         nan = np.isnan(v)
         assert np.array_equal(np.isnan(got), nan)
         assert np.array_equal(got.view(np.uint32)[~nan], v.view(np.uint32)[~nan])
+
+
+# fewer than 256 tiles (one kernel scans and lists them), more (a scan kernel
+# first), and more than 4096 diagonals (clear, scan, places and list as kernels)
+@pytest.mark.parametrize("interior", [(9, 40, 150), (12, 40, 150), (2, 3, 70000)])
+def test_tile_list_paths(gpu, interior):
+    import torch
+    nh, lo = 3, 2
+    shape = tuple(n + 2 * lo for n in interior)
+    rng = np.random.default_rng(interior[0])
+    for density in (0.001, 0.5):
+        v = rng.normal(size=shape).astype(np.float32)
+        v[rng.random(shape) < density] = np.nan
+        dev = torch.from_numpy(v.copy()).cuda()
+        pct.regularization_step_device(dev, nh)
+        got = dev.cpu().numpy()
+        pct.regularization_step(v, nh)
+        assert np.array_equal(got.view(np.uint32), v.view(np.uint32))
