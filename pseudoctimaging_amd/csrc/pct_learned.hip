@@ -662,17 +662,46 @@ static int launch_embed_windows(const float* params, const void* d_model, const 
 // window box sums of the atlas CT
 // ---------------------------------------------------------------------------
 
+// out[m] = w[m] + ... + w[m + K - 1] for m < M: sums of 2, 4 and 8 consecutive
+// values, shared by the windows, then the terms of K in binary.  3 to 5 adds per
+// window of 7 to 15 in place of 6 to 14.
+template <int K, int M>
+__device__ __forceinline__ void window_sums(const float (&w)[M + K - 1], float (&out)[M]) {
+    constexpr int W = M + K - 1;
+    float s[W];
+    int at = 0;   // of the next term, a constant once unrolled
+#pragma unroll
+    for (int i = 0; i < W; ++i) s[i] = w[i];
+#pragma unroll
+    for (int len = 1; len <= K; len *= 2) {
+        if (K & len) {
+#pragma unroll
+            for (int m = 0; m < M; ++m) out[m] = at ? out[m] + s[m + at] : s[m];
+            at += len;
+        }
+#pragma unroll
+        for (int i = 0; i + len < W; ++i) s[i] += s[i + len];
+    }
+}
+
 // The NH^3 window sums in one pass.  A block owns a kBoxTX x kBoxTY column
 // tile of one volume over a run of kBoxRun output planes and sweeps the
 // planes that feed it.  Each plane's tile, with a halo of HW (zeros outside
-// the volume), goes through LDS and is summed over y (4 outputs per task,
+// the volume), goes through LDS and is summed over y (8 outputs per task,
 // from 128-bit LDS reads), then over x.  The plane sums enter a running sum
 // over z in double, and the last 2 HW + 2 of them stay in registers for the
 // subtraction; the double sum of float plane sums is exact in practice, so
-// the result does not depend on where a run starts.  Every thread owns 2
+// the result does not depend on where a run starts.  Every thread owns 4
 // consecutive x of one y of the tile, and the loads of the next two planes
 // are in flight during a plane's sums (two register buffers).
-constexpr int kBoxTX = 16, kBoxTY = 64, kBoxRun = 32, kBoxThreads = 512;
+//
+// What bounds it is the wait for a plane's loads, next to LDS traffic: hence
+// loads and stores that the compiler can count (below), 125 registers at HW = 5
+// (4 waves per SIMD; 194 with the addresses of plain loads and stores), and 8
+// outputs to a y task.  222x222x112, n = 10, NH = 11: 265 -> 202 us alone (the bytes
+// it must move take 95), beside the embeddings 714 -> 260, the pruned fusion 2019 ->
+// 1933.  Row pitches without bank conflicts gained nothing.
+constexpr int kBoxTX = 16, kBoxTY = 64, kBoxRun = 32, kBoxThreads = 256;
 
 template <int HW>
 __global__ __launch_bounds__(kBoxThreads) void box_xyz(const float* __restrict__ in,
@@ -681,17 +710,16 @@ __global__ __launch_bounds__(kBoxThreads) void box_xyz(const float* __restrict__
     constexpr int K = 2 * HW + 1;
     constexpr int KR = K + 1;                    // ring length, even
     constexpr int R = kBoxTX + 2 * HW, C = kBoxTY + 2 * HW;
-    constexpr int NQ = (4 + 2 * HW + 3) / 4;     // float4 reads per y-sum task
-    constexpr int CP = kBoxTY - 4 + 4 * NQ;      // LDS row pitch (>= C, multiple of 4)
+    constexpr int MY = 8;                        // outputs of a y-sum task
+    constexpr int NQ = (MY + 2 * HW + 3) / 4;    // float4 reads per y-sum task
+    constexpr int CP = kBoxTY - MY + 4 * NQ;     // LDS row pitch (>= C, multiple of 4)
     constexpr int NLD = (R * C + kBoxThreads - 1) / kBoxThreads;   // tile loads per thread
-    constexpr int NYT = R * (kBoxTY / 4);        // y-sum tasks
+    constexpr int NYT = R * (kBoxTY / MY);       // y-sum tasks
     constexpr int OX = kBoxTX / (kBoxThreads / 64);   // x outputs per thread
-    // row pitch of the y sums: a multiple of 4 for the 128-bit stores, and
-    // not of 64, so the column reads of the x sums (two rows per
-    // instruction) hit different banks
+    // row pitch of the y sums: a multiple of 4 for the 128-bit stores
     constexpr int YP = kBoxTY + 4;
     static_assert(CP >= C && CP % 4 == 0, "row pitch");
-    static_assert(NYT <= kBoxThreads && OX == 2, "one y-sum task and 2 outputs per thread");
+    static_assert(NYT <= kBoxThreads, "one y-sum task");
     __shared__ __align__(16) float T[R * CP];
     __shared__ __align__(16) float Y[R * YP];
 
@@ -711,34 +739,41 @@ __global__ __launch_bounds__(kBoxThreads) void box_xyz(const float* __restrict__
     const float* __restrict__ src = in + vi * plane * nz;
     float* __restrict__ dst = out + vi * plane * nz;
 
-    // load slots: in-plane offset of the tile element (0 where it lies
-    // outside the volume or past the tile, so that every load is
-    // unconditional and the loads of two planes stay in flight: a load under
-    // a branch makes the compiler wait for every earlier load), whether it
-    // lies in the volume (else a zero is stored), and whether it lies in the
-    // tile (else nothing is stored)
-    int lofs[NLD];
-    bool lin[NLD], lst[NLD];
+    // Loads and stores go through buffer descriptors that start at the tile's
+    // corner of a plane: an offset past the descriptor's range reads zero and
+    // stores nothing, so every plane issues the same loads and stores on every
+    // path and the compiler can count those in flight: it waits for the older of
+    // the two planes, where a branch around any of them made it wait for nearly
+    // all (vmcnt counts stores too).  A tile's offsets stay below 30 rows of
+    // 65535.
+    constexpr unsigned kOut = 0xfffffff0u;   // past the range
+    auto tile_rsrc = [&](const float* p) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, 0x7fffffff, 0x00020000);
+    };
+    unsigned lofs[NLD];   // of the tile element
+    bool lst[NLD];        // whether the element lies in the tile (else not stored to LDS)
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
         const int e = (int)threadIdx.x + i * kBoxThreads;
         const int rr = e / C, cc = e - (e / C) * C;
         const int x = x0 - HW + rr, y = y0 - HW + cc;
         lst[i] = e < R * C;
-        lin[i] = lst[i] && x >= 0 && x < nx && y >= 0 && y < ny;
-        lofs[i] = lin[i] ? x * ny + y : 0;
+        const bool in = lst[i] && x >= 0 && x < nx && y >= 0 && y < ny;
+        lofs[i] = in ? 4u * (unsigned)(rr * ny + cc) : kOut;
     }
+    const long long corner = (long long)(x0 - HW) * ny + (y0 - HW);
     float va[NLD], vb[NLD];
     auto load = [&](int p, float (&v)[NLD]) {
-        const float* __restrict__ sp = src + p * plane;
+        const auto rs = tile_rsrc(src + p * plane + corner);
 #pragma unroll
-        for (int i = 0; i < NLD; ++i) v[i] = sp[lofs[i]];
+        for (int i = 0; i < NLD; ++i)
+            v[i] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, (int)lofs[i], 0, 0));
     };
 
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int ox = OX * wv, oy = lane;   // outputs (x0 + ox + m, y0 + oy), m < OX
     float ring[KR][OX];
-    double acc[OX] = {0.0, 0.0};
+    double acc[OX] = {};
     const int pa = max(0, z0 - HW), pe = z1 - 1 + HW;   // planes >= nz are zero
     load(pa, va);
     load(min(pa + 1, nz - 1), vb);
@@ -748,15 +783,14 @@ __global__ __launch_bounds__(kBoxThreads) void box_xyz(const float* __restrict__
             const int p = pb + j;
             if (p > pe) break;   // uniform
             float(&cur)[NLD] = (j & 1) ? vb : va;   // holds plane p
-            float bs[OX] = {0.f, 0.f};
-            if (p < nz) {        // uniform
-                __syncthreads();   // the previous plane's y sums are done with T
+            float bs[OX] = {};
+            if (p < nz) {        // uniform; the last barrier ended the reads of T
 #pragma unroll
                 for (int i = 0; i < NLD; ++i) asm volatile("" : "+v"(cur[i]));
 #pragma unroll
                 for (int i = 0; i < NLD; ++i) {
                     const int e = (int)threadIdx.x + i * kBoxThreads;
-                    if (lst[i]) T[(e / C) * CP + e - (e / C) * C] = lin[i] ? cur[i] : 0.f;
+                    if (lst[i]) T[(e / C) * CP + e - (e / C) * C] = cur[i];
                 }
             }
             // plane p + 2, in flight for two planes; loaded on every path (a
@@ -766,55 +800,49 @@ __global__ __launch_bounds__(kBoxThreads) void box_xyz(const float* __restrict__
             if (p < nz) {        // uniform
                 __syncthreads();
                 if ((int)threadIdx.x < NYT) {
-                    const int rr = threadIdx.x >> 4, c0 = 4 * (threadIdx.x & 15);
-                    float w4[4 * NQ];
+                    constexpr int TY = kBoxTY / MY;   // tasks of a row
+                    const int rr = threadIdx.x / TY, c0 = MY * (threadIdx.x % TY);
+                    float w[MY + 2 * HW], o[MY];
 #pragma unroll
                     for (int q = 0; q < NQ; ++q) {
                         const float4 f = *reinterpret_cast<const float4*>(&T[rr * CP + c0 + 4 * q]);
-                        w4[4 * q] = f.x;
-                        w4[4 * q + 1] = f.y;
-                        w4[4 * q + 2] = f.z;
-                        w4[4 * q + 3] = f.w;
-                    }
-                    float4 o;
-                    float* op = reinterpret_cast<float*>(&o);
+                        const float e[4] = {f.x, f.y, f.z, f.w};
 #pragma unroll
-                    for (int m = 0; m < 4; ++m) {
-                        float sacc = 0.f;
-#pragma unroll
-                        for (int k = 0; k < K; ++k) sacc += w4[m + k];
-                        op[m] = sacc;
+                        for (int i = 0; i < 4; ++i)
+                            if (4 * q + i < MY + 2 * HW) w[4 * q + i] = e[i];
                     }
-                    *reinterpret_cast<float4*>(&Y[rr * YP + c0]) = o;
+                    window_sums<K, MY>(w, o);
+#pragma unroll
+                    for (int m = 0; m < MY; m += 4)
+                        *reinterpret_cast<float4*>(&Y[rr * YP + c0 + m]) =
+                            make_float4(o[m], o[m + 1], o[m + 2], o[m + 3]);
                 }
                 __syncthreads();
                 float col[OX + 2 * HW];
 #pragma unroll
                 for (int k = 0; k < OX + 2 * HW; ++k) col[k] = Y[(ox + k) * YP + oy];
-#pragma unroll
-                for (int m = 0; m < OX; ++m) {
-                    float sacc = 0.f;
-#pragma unroll
-                    for (int k = 0; k < K; ++k) sacc += col[m + k];
-                    bs[m] = sacc;
-                }
+                window_sums<K, OX>(col, bs);
             }
 #pragma unroll
             for (int m = 0; m < OX; ++m) {
                 acc[m] += (double)bs[m];
+                // kept as a float: as the double added above, which the compiler
+                // would reuse for the subtraction, the ring is twice the registers
+                asm volatile("" : "+v"(bs[m]));
                 ring[j][m] = bs[m];
             }
-            const int z = p - HW;   // the output whose window ends at p
-            if (z >= z0) {
-                const int y = y0 + oy;
+            // the output whose window ends at p, from z0 on
+            const int z = p - HW;
+            const auto rs = tile_rsrc(dst + max(z, 0) * plane + (long long)x0 * ny + y0);
 #pragma unroll
-                for (int m = 0; m < OX; ++m) {
-                    const int x = x0 + ox + m;
-                    if (x < nx && y < ny) dst[z * plane + (long long)x * ny + y] = (float)acc[m];
-                    // plane z - HW = p - 2 HW leaves the window; it sits in
-                    // ring slot (j - 2 HW) mod KR = (j + 2) mod KR
-                    if (z - HW >= pa) acc[m] -= (double)ring[(j + 2) % KR][m];
-                }
+            for (int m = 0; m < OX; ++m) {
+                const bool in = z >= z0 && x0 + ox + m < nx && y0 + oy < ny;
+                __builtin_amdgcn_raw_buffer_store_b32(
+                    __float_as_int((float)acc[m]), rs,
+                    in ? (int)(4u * (unsigned)((ox + m) * ny + oy)) : (int)kOut, 0, 0);
+                // plane z - HW = p - 2 HW leaves the window; it sits in
+                // ring slot (j - 2 HW) mod KR = (j + 2) mod KR
+                if (z >= z0 && z - HW >= pa) acc[m] -= (double)ring[(j + 2) % KR][m];
             }
         }
     }
