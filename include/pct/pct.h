@@ -335,7 +335,8 @@ typedef struct pct_train_opts {
 
 /* Loss and gradient (host, PCT_MLP_NPARAMS floats; 0 for mu, inv_sd and the
  * unused W1 rows) for the given anchors (host, [n_anchors][4] = z, x, y,
- * atlas).  Deterministic.  Synchronises. */
+ * atlas).  Deterministic.  Synchronises.  Exchanges its inputs and results
+ * through 1 MiB of pinned host memory per device (freed by pct_release). */
 int pct_mlp_loss_grad_dev(const pct_problem* pb, const float* params, const int* anchors,
                           int n_anchors, float tau, float teacher_t, const float* d_img,
                           const float* d_atlas, double* loss, float* grad, pct_stream_t stream);

@@ -1394,6 +1394,9 @@ void release_batch_graphs();
 // Frees the per-device copies of the embedding network (pct_learned.hip).
 void release_learned_models();
 
+// Frees the gradient calls' pinned buffers (pct_train.hip).
+void release_train_buffers();
+
 // Frees the device buffers, streams and events of the host-buffer entry
 // points (pct_fuse.hip).
 void release_host_buffers();
