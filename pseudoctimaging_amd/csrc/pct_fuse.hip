@@ -418,7 +418,10 @@ bool make_geometry(const pct_problem* pb, int shape_id, int group, TileGeometry*
     g->n_tiles = (long long)g->tiles_y * g->tiles_x * g->tiles_z;
     g->group = std::max(1, std::min(group, pb->n_atlas));
     g->n_groups = (pb->n_atlas + g->group - 1) / g->group;
-    g->n_split = std::max(1, std::min(split, 2 * hw + 1));
+    // more parts than dz: a multiple of them, with squared differences only
+    const int nw = 2 * hw + 1;
+    if (s.form == 1) split = std::min(split, nw);
+    g->n_split = split <= nw ? std::max(1, split) : nw * std::min(split / nw, nw);
     g->n_items = g->n_tiles * g->n_parts();
     g->lds_bytes = e->lds_bytes;
     const int by_lds = kLdsPerCu / e->lds_bytes;
@@ -430,7 +433,7 @@ bool make_geometry(const pct_problem* pb, int shape_id, int group, TileGeometry*
 // ---- cost model -------------------------------------------------------------
 //
 // Time of one fusion call with a tile shape, atlas group and split of the
-// window's dz, in microseconds.  The form is the kernel's: per candidate a wave
+// window, in microseconds.  The form is the kernel's: per candidate a wave
 // issues `plain` FP32 instructions, which pair between waves, 2 BZ BX DPP adds
 // and BZ BX exps; per slab it copies rows; an item runs its candidates at the
 // rate one wave alone reaches (latency) or at the SIMD's, whichever is slower for
@@ -452,6 +455,7 @@ constexpr double kTail = 0.229;                       // part of a round the las
 constexpr double kMhz = 2350.0;
 constexpr double kLaunch = 6.5 + 4.3;                 // kernel and finalize launches
 constexpr double kFinalize = 1.264 * 4 / 4e6;         // per float read or written
+constexpr double kFinalRound = 0.6;                   // latency of eight partials
 constexpr double kPairs0 = 7.3, kPairs = 1.532 * 16 / 4e6;   // pair pre-pass
 // measured over modelled, by shape
 constexpr double kShape[] = {1.12, 1.12, 1.02, 1.05, 0.96, 0.96, 0.99, 0.96, 0.88, 0.95,
@@ -475,12 +479,13 @@ static double item_time(int shape_id, const TileGeometry& g, double wgs) {
     const double next = moves ? rows * (xt ? 3 : 2) : whole;
     const double batches = xt ? 1.5 * bz + 1 : bz + 1;
     const double slabs = std::ceil(nh / g.n_split);
+    const double lines = g.n_split > nh ? std::ceil(nh * nh / g.n_split) : nh;   // dy
     const double copies = kRow * (whole + (slabs - 1) * next) + kSlab * slabs;
     const double latency = kRound * (batches + (slabs - 1) * (moves ? 1 : batches));
     const double waves = std::max(wgs * s.waves / 4.0, 0.25);   // resident per SIMD
     const double cycles =
-        g.group * std::max(slabs * nh * nh * alone + copies + latency,
-                           std::pow(waves, kWaves) * (slabs * nh * nh * busy + copies));
+        g.group * std::max(slabs * lines * nh * alone + copies + latency,
+                           std::pow(waves, kWaves) * (slabs * lines * nh * busy + copies));
     return cycles / kMhz * kShape[shape_id];
 }
 
@@ -496,7 +501,8 @@ static double model_cost(const pct_problem* pb, int shape_id, int group, TileGeo
     const double kernel =
         per_cu <= slots ? item_time(shape_id, g, std::max(1.0, std::ceil(per_cu)))
                         : (per_cu / slots + kTail) * item_time(shape_id, g, slots);
-    double us = kernel + kLaunch + kFinalize * N * (1 + 2 * g.n_parts());
+    double us = kernel + kLaunch + kFinalize * N * (1 + 2 * g.n_parts()) +
+                kFinalRound * (g.n_parts() / 8);
     if (shapes()[shape_id].form == 1) us += kPairs0 + kPairs * N * pb->n_atlas;
     return us;
 }
@@ -532,8 +538,8 @@ static bool unit_range_in_bound(const pct_problem* pb) {
     return std::sqrt(1.4426950408889634 / problem_divisor(pb)) <= (double)kXtBound;
 }
 
-// Candidate splits of the window: whole, halves, thirds, pairs of dz and single
-// ones.  The partial sums of a split may not need more memory than 256 MiB (or
+// Candidate splits of the window: whole, halves, thirds, pairs of dz, single ones,
+// and halves, thirds, fifths and single dy of each.  The partial sums of a split may not need more memory than 256 MiB (or
 // than the groups alone).  Groups are of one atlas: several to an item save up to
 // 2 % from NH 7 on and 9 % at NH 3 (fewer partial sums), but one sum over ten
 // atlases rounds five times as far off, and a host-buffer call copies the next
@@ -543,8 +549,8 @@ static std::vector<int> candidate_splits(const pct_problem* pb, int group) {
     const double per_part = 8.0 * pb->nx * pb->ny * pb->nz *
                             ((pb->n_atlas + group - 1) / group);
     std::vector<int> out;
-    for (int s : {1, 2, 3, (nh + 1) / 2, nh})
-        if (s <= nh && (out.empty() || s > out.back()) && (s == 1 || s * per_part <= 268435456.0))
+    for (int s : {1, 2, 3, (nh + 1) / 2, nh, 2 * nh, 3 * nh, 5 * nh, nh * nh})
+        if (s <= nh * nh && (s > 3 || s <= nh) && (out.empty() || s > out.back()) && (s == 1 || s * per_part <= 268435456.0))
             out.push_back(s);
     return out;
 }

@@ -82,7 +82,7 @@ struct TiledArgs {
     int n_tiles;
     int n_items;
     int n_atlas, group;
-    int n_split;      // parts of the window's dz, each an item of its own
+    int n_split;      // parts of the window (see WindowPart), each an item of its own
     float scale;      // sqrt(log2(e)/div)
     // optional item filter: when set, items whose byte is 0 are skipped
     const unsigned char* only;
@@ -518,6 +518,22 @@ __device__ __forceinline__ bool wave_has_rows(int x0, int x_end, int wv) {
     return x0 + __builtin_amdgcn_readfirstlane(wv) * C::S * BX < x_end;
 }
 
+// The candidates of part sp of n_split: up to NH parts a range of dz, more (a
+// multiple of NH) one dz and a range of dy.  A volume of a few tiles leaves most
+// of the chip idle even with an item per dz (24x25x23, n = 1, NH = 15: 37.8 -> 19.2
+// us; 48x40x30, NH = 9: 21.4 -> 18.0).
+struct WindowPart {
+    int dz_begin, dz_end;   // -HW .. HW + 1
+    int dy_first, dy_count;
+};
+template <int HW>
+__device__ __forceinline__ WindowPart window_part(int sp, int n_split) {
+    constexpr int K = 2 * HW + 1;
+    if (n_split <= K) return {sp * K / n_split - HW, (sp + 1) * K / n_split - HW, 0, K};
+    const int q = n_split / K, dz = sp / q, j = sp - dz * q;
+    return {dz - HW, dz - HW + 1, j * K / q, (j + 1) * K / q - j * K / q};
+}
+
 // One work item (tile, atlas group) of one problem: the whole workgroup runs
 // it.  Shared by the single-problem kernel and the persistent batched kernel,
 // so a problem gives bit-identical results through either.
@@ -565,8 +581,8 @@ __device__ __forceinline__ void tiled_item(const TiledArgs& args, int item,
     const int ys = y0 - 1 - HW;   // volume y of LDS column 0
     const int a_begin = g * args.group;
     const int a_end = min(args.n_atlas, a_begin + args.group);
-    const int dz_begin = sp * (2 * HW + 1) / args.n_split - HW;
-    const int dz_end = (sp + 1) * (2 * HW + 1) / args.n_split - HW;
+    const WindowPart wp = window_part<HW>(sp, args.n_split);
+    const int first = lane_base + wp.dy_first;   // the lane's LDS position at (0, dy_first)
     const bool live = wave_has_rows<C, BX>(x0, nx - r, wv);
 
     for (int a = a_begin; a < a_end; ++a) {
@@ -574,17 +590,17 @@ __device__ __forceinline__ void tiled_item(const TiledArgs& args, int item,
         const float* __restrict__ L = args.label + (long long)a * args.N;
         SlabSlots<C> slots;
         slots.reset();
-        for (int dz = dz_begin; dz < dz_end; ++dz) {
-            if (dz > dz_begin) slots.advance();
+        for (int dz = wp.dz_begin; dz < wp.dz_end; ++dz) {
+            if (dz > wp.dz_begin) slots.advance();
             __syncthreads();
-            stage_slab<C, NW>(lds, slots, dz == dz_begin, A, L, args.scale, z0 + dz, xs, ys, nx,
+            stage_slab<C, NW>(lds, slots, dz == wp.dz_begin, A, L, args.scale, z0 + dz, xs, ys, nx,
                               ny, nz, plane, wv, lane);
             __syncthreads();
             if (!live) continue;
             // dy rolled, dx unrolled: consecutive dx share MRI and CT rows
 #pragma unroll 1
-            for (int dy = 0; dy <= 2 * HW; ++dy)
-                tiled_dx_sweep<C, BX, BZ, HW>(lds, lane_base + dy, slots, tv, P, S);
+            for (int dy = 0; dy < wp.dy_count; ++dy)
+                tiled_dx_sweep<C, BX, BZ, HW>(lds, first + dy, slots, tv, P, S);
         }
     }
 
@@ -1164,6 +1180,8 @@ __device__ __forceinline__ void tiled_item_xt(const TiledArgs& args, int item,
     const int ys = y0 - 1 - HW;
     const int a_begin = g * args.group;
     const int a_end = min(args.n_atlas, a_begin + args.group);
+    // whole dz only: a dy loop of variable length costs this kernel 1 % (160^2x96, n =
+    // 1, NH = 7: 261 against 258 us), and it is not the one for volumes that small
     const int dz_begin = sp * (2 * HW + 1) / args.n_split - HW;
     const int dz_end = (sp + 1) * (2 * HW + 1) / args.n_split - HW;
     // 2^-TT per output (1 where the item keeps the squared differences)

@@ -1,4 +1,4 @@
-"""Small problems split the window's dz over work items.  The default
+"""Small problems split the window over work items, by dz and then by dy.  The default
 configuration against the FP64 oracle and against one forced configuration
 without a split, for every window at sizes below a tile, one tile and just past
 it; host and device calls bit for bit.
