@@ -20,8 +20,7 @@
 //                 plane at a time), the topk offsets kept (radix select; a
 //                 bitonic sort where a positive margin needs the order
 //                 statistics), a low score gap flags the item for the full
-//                 search.
-//  merge_offsets_kernel  per item, the offsets to evaluate in the pruned
+//                 search; then the offsets to evaluate in the pruned
 //                 kernel's order (kept, then samples, per dz plane).
 //  pruned_kernel  per (tile, atlas): the kept offsets and a 3x3x3 lattice of
 //                 sample offsets, weighted exactly with the same LDS slabs and
@@ -265,8 +264,17 @@ struct EmbedWinArgs {
 // column reaches.  One wave per (volume, tile column, z): it stages the 3 x
 // (window rows + 2) neighbour rows in LDS and runs the MFMA chain of
 // embed_kernel on 16 voxels at a time, with the same feature arithmetic, so
-// the values equal embed_kernel's bit for bit.
-__global__ __launch_bounds__(kEmbWaves * 64) void embed_windows_kernel(EmbedWinArgs a) {
+// the values equal embed_kernel's bit for bit.  One launch embeds the atlases
+// (the first blocks0 workgroups) and the target (34x40x30, n = 3, NH = 7: with the
+// merge in the selection the pruned fusion takes 88 us, 100 with launches of their
+// own).
+__global__ __launch_bounds__(kEmbWaves * 64) void embed_windows_kernel(EmbedWinArgs a0,
+                                                                      int blocks0,
+                                                                      EmbedWinArgs a1) {
+    const bool first = (int)blockIdx.x < blocks0;
+    const EmbedWinArgs a = first ? a0 : a1;
+    const int block = first ? blockIdx.x : blockIdx.x - blocks0;
+    const int blocks = first ? blocks0 : gridDim.x - blocks0;
     __shared__ float rows[kEmbWaves][3 * 18 * kWinRow];
     __shared__ __align__(16) float sbias[144];   // b1[64], b2[64], b3[16]
     __shared__ v4s sw2[16][64];                  // layer-2 weight fragments (t, s) by lane
@@ -290,7 +298,7 @@ __global__ __launch_bounds__(kEmbWaves * 64) void embed_windows_kernel(EmbedWinA
 
     float* __restrict__ R = rows[wv];
     const long long vsize = (long long)a.nx * a.ny * a.nz;
-    for (int base = blockIdx.x * kEmbWaves; base < a.jobs; base += gridDim.x * kEmbWaves) {
+    for (int base = block * kEmbWaves; base < a.jobs; base += blocks * kEmbWaves) {
         const int job = base + wv;
         const bool active = job < a.jobs;
         int z = 0, tx = 0, ty = 0, vi = 0;
@@ -615,14 +623,15 @@ static int launch_embed(const float* params, const void* d_model, const float* v
     return hipGetLastError() == hipSuccess ? PCT_OK : PCT_ERR_HIP;
 }
 
-// Embeddings inside the selection's probe windows (see embed_windows_kernel):
-// `nvol` volumes, window half-width `whw` around each probe cluster (the
-// search half window for the atlases, 0 for the target, whose probe
-// clusters alone are read); tile geometry as in pct_fuse_pruned_dev.
-static int launch_embed_windows(const float* params, const void* d_model, const float* vol,
-                                int nvol, int whw, const pct_problem* pb, const TileGeometry& g,
-                                int oy, int wx, int bz, unsigned short* emb, hipStream_t stream,
-                                const int* d_zlist = nullptr, int nzl = 0) {
+// Arguments and workgroups for the embeddings inside the selection's probe
+// windows (see embed_windows_kernel; a problem with tiles): `nvol` volumes, window
+// half-width `whw` around each probe cluster (the search half window for the
+// atlases, 0 for the target, whose probe clusters alone are read); tile geometry
+// as in pct_fuse_pruned_dev.
+static int embed_windows_args(const float* params, const void* d_model, const float* vol,
+                              int nvol, int whw, const pct_problem* pb, const TileGeometry& g,
+                              int oy, int wx, int bz, unsigned short* emb, const int* d_zlist,
+                              int nzl, EmbedWinArgs* out, int* blocks) {
     EmbedWinArgs a;
     a.vol = vol;
     a.emb = emb;
@@ -638,7 +647,6 @@ static int launch_embed_windows(const float* params, const void* d_model, const 
     a.tiles_y = g.tiles_y;
     a.oy = oy;
     a.wx = wx;
-    if (g.n_tiles == 0) return PCT_OK;
     const int z_first = probe_origin(0, bz, g.r, pb->nz, 2);
     const int z_last = probe_origin(g.tiles_z - 1, bz, g.r, pb->nz, 2);
     a.zlo = std::max(z_first - whw, 0);
@@ -651,11 +659,9 @@ static int launch_embed_windows(const float* params, const void* d_model, const 
     a.jobs = (int)jobs;
     a.mu = params[kOffMu];
     a.inv_sd = params[kOffSd];
-    const long long blocks = std::min<long long>((jobs + kEmbWaves - 1) / kEmbWaves, 256LL * 16);
-    if (blocks > 0)
-        hipLaunchKernelGGL(embed_windows_kernel, dim3((unsigned)blocks), dim3(kEmbWaves * 64), 0,
-                           stream, a);
-    return hipGetLastError() == hipSuccess ? PCT_OK : PCT_ERR_HIP;
+    *out = a;
+    *blocks = (int)std::min<long long>((jobs + kEmbWaves - 1) / kEmbWaves, 256LL * 16);
+    return PCT_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -860,7 +866,7 @@ static const BoxFn kBoxXyz[kMaxTiledHalfWindow] = {&box_xyz<1>, &box_xyz<2>, &bo
 struct SelectArgs {
     const unsigned short* embT;   // [N][16]
     const unsigned short* embA;   // [n][N][16]
-    int* sel;                     // [items][topk] kept offset indices, ascending, kNoOffset after
+    int* merged;                  // [items][kMergedStride] offsets to evaluate (merge_offsets)
     unsigned char* flag;          // [items] 1 = full search
     long long N;
     int nx, ny, nz, hw, r;
@@ -874,6 +880,9 @@ struct SelectArgs {
     unsigned score_bits;          // dz indices (dz + hw) whose offsets are scored
     unsigned fixed_allowed;       // the allowed dz indices when they do not depend on the
                                   // scores, else 0
+    int cw;                       // row length of the pruned kernel's slab
+    int n_samples;
+    int samples[kSamples];        // lattice offset indices, ascending
 };
 
 constexpr int kSelThreads = 256;
@@ -881,6 +890,66 @@ constexpr int kSelPerThread = 16;   // 4096 offsets (NH = 15: 3375)
 static_assert(kSelThreads >= 16 * 15, "16 threads per dz slab in the slab minima");
 static_assert(kSelThreads >= 15 * 15, "one thread per (dx, dy) in the gathers");
 constexpr int kNoOffset = 1 << 30;
+
+// The offsets the pruned kernel evaluates for an item, in its
+// order: per dz plane (ascending), the kept offsets, then the lattice samples
+// that are not kept (a sample that is also kept counts once, as kept).  One
+// wave, every entry placed by counting: a kept offset goes after the
+// kept offsets before it and the samples of the earlier planes; a sample goes
+// after the kept offsets of its plane and the planes before, and after the
+// samples before it.  Entry 0 holds the count and the number of samples;
+// entry 1 + k holds offset k as (sample << 31) | ((dz + 8) << 16) | LDS delta
+// (dy + dx rows of the slab, row length cw).  `kept`: the kept offset indices,
+// ascending, kNoOffset after.  As a kernel of its own it took 29 us
+// after a selection of 228 at 222x222x112, n = 10, NH = 11, and 10 after 14 at
+// 34x40x30, n = 3, NH = 7; at the end of the selection, by scalar reads of the
+// lanes, the two take 245 and 19.
+constexpr int kMergedStride = 96;   // >= 1 + kMaxOffsets
+static_assert(kMergedStride >= 1 + kMaxOffsets, "merged list stride");
+static_assert(kMaxTopk <= 64 && kSamples <= 64, "one lane per kept offset and per sample");
+
+__device__ __forceinline__ void merge_offsets(const SelectArgs& a, int item, const int* kept) {
+    const int lane = threadIdx.x & 63;
+    const int nw1 = 2 * a.hw + 1, nw2 = nw1 * nw1;
+    const int kv = lane < a.topk ? kept[lane] : kNoOffset;
+    int sv = kNoOffset;   // the lane's sample (uniform indices into the arguments)
+    for (int j = 0; j < kSamples; ++j)
+        if (j == lane && j < a.n_samples) sv = a.samples[j];
+    const bool has_k = kv < kNoOffset, has_s = sv < kNoOffset;
+    // the kept offsets of a dz plane in (dy, dx) order, the order in which
+    // the plain kernel sweeps a slab's candidates (dy outer, dx inner), so
+    // that evaluating every candidate sums in the plain kernel's order: the
+    // rank among the kept offsets by the key (dz, dy, dx)
+    const int key = has_k ? (kv / nw2) * nw2 + (kv % nw1) * nw1 + (kv / nw1) % nw1 : INT_MAX;
+    const int klo = has_k ? (kv / nw2) * nw2 : 0;          // first offset of the kept plane
+    const int shi = has_s ? (sv / nw2 + 1) * nw2 : 0;      // end of the sample's plane
+    bool dup = false;
+    int before_s = 0, rank = 0;
+    for (int q = 0; q < a.topk; ++q) {   // uniform
+        const int v = __builtin_amdgcn_readlane(kv, q);
+        dup |= v == sv;
+        before_s += v < shi;
+        rank += __builtin_amdgcn_readlane(key, q) < key;
+    }
+    const unsigned long long smask = __ballot(has_s && !dup);   // samples evaluated
+    const unsigned long long kmask = __ballot(has_k);
+    int before_k = 0;
+    for (int j = 0; j < a.n_samples; ++j)
+        before_k += (int)((smask >> j) & 1ull) & (a.samples[j] < klo);
+    auto pack = [&](int o, unsigned smpl) {
+        const int dz = o / nw2 - a.hw;
+        const int del = ((o / nw1) % nw1) * a.cw + o % nw1;
+        return (int)((smpl << 31) | ((unsigned)(dz + 8) << 16) | (unsigned)del);
+    };
+    int* out = a.merged + (long long)item * kMergedStride;
+    if (has_k) out[1 + rank + before_k] = pack(kv, 0u);
+    if (has_s && !dup)
+        out[1 + before_s + __popcll(smask & ((1ull << lane) - 1ull))] = pack(sv, 1u);
+    if (lane == 0) {
+        const int ns = __popcll(smask);
+        out[0] = (__popcll(kmask) + ns) | (ns << 16);
+    }
+}
 
 // One workgroup per item = (atlas, tile), item = atlas * n_tiles + tile.
 // Order-preserving integer image of a float score (-0 is taken as +0, as the
@@ -891,7 +960,7 @@ __device__ __forceinline__ unsigned order_key(float f) {
 }
 
 // The topk smallest (score, offset index) pairs among the m candidates of the
-// allowed slabs, written in ascending offset order, and the item's flag for a
+// allowed slabs, into `kept` in ascending offset order, and the item's flag for a
 // margin <= 0 (set for a negative margin).  Thread t holds the scores of
 // offsets t + q kSelThreads.  A four-pass radix select over the order keys
 // finds T, the key of the k-th smallest; keys below T are kept, and of the
@@ -901,7 +970,7 @@ __device__ __forceinline__ unsigned order_key(float f) {
 __device__ __forceinline__ void select_topk_radix(
     const SelectArgs& a, int item, int ncand, int nw2, const float (&sc)[kSelPerThread],
     const float* key, unsigned allowed_bits, int m, unsigned* hist, unsigned& sh_T,
-    int& sh_need, int& sh_cnt, int* tie, int* wcnt) {
+    int& sh_need, int& sh_cnt, int* tie, int* wcnt, int* kept) {
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int k = min(a.topk, m);
     bool al[kSelPerThread];
@@ -991,7 +1060,6 @@ __device__ __forceinline__ void select_topk_radix(
         }
         keep[q] = kp;
     }
-    int* out = a.sel + (long long)item * a.topk;
     int base = 0;
 #pragma unroll
     for (int q = 0; q < kSelPerThread; ++q) {
@@ -1012,11 +1080,11 @@ __device__ __forceinline__ void select_topk_radix(
             tot += wcnt[w];
         }
         if (keep[q])
-            out[off + __popcll(bal & ((1ull << lane) - 1ull))] = threadIdx.x + q * kSelThreads;
+            kept[off + __popcll(bal & ((1ull << lane) - 1ull))] = threadIdx.x + q * kSelThreads;
         __syncthreads();   // wcnt is rewritten for the next q
         base += tot;
     }
-    for (int i = k + threadIdx.x; i < a.topk; i += kSelThreads) out[i] = kNoOffset;
+    for (int i = k + threadIdx.x; i < a.topk; i += kSelThreads) kept[i] = kNoOffset;
     if (threadIdx.x == 0) a.flag[item] = (unsigned char)(a.margin < 0.f ? 1 : 0);
 }
 
@@ -1031,6 +1099,7 @@ __global__ __launch_bounds__(kSelThreads) void select_kernel(SelectArgs a) {
     __shared__ int rs_need, rs_cnt;
     __shared__ int rs_tie[kMaxTopk];
     __shared__ int rs_wcnt[kSelThreads / 64];
+    __shared__ int kept[kMaxTopk];         // kept offset indices, ascending, kNoOffset after
     const int item = blockIdx.x;
     const int at = item / a.n_tiles;
     int t = item - at * a.n_tiles;
@@ -1242,7 +1311,9 @@ __global__ __launch_bounds__(kSelThreads) void select_kernel(SelectArgs a) {
         // set - the topk smallest (score, offset index) pairs of the allowed
         // slabs - comes from a radix select, without a sort.
         select_topk_radix(a, item, ncand, nw2, sc, key, allowed_bits, n_allowed * nw2, rs_hist,
-                          rs_T, rs_need, rs_cnt, rs_tie, rs_wcnt);
+                          rs_T, rs_need, rs_cnt, rs_tie, rs_wcnt, kept);
+        __syncthreads();
+        if (wv == 0) merge_offsets(a, item, kept);
         return;
     }
     // candidates of the allowed slabs, then bitonic sort ascending by
@@ -1295,17 +1366,18 @@ __global__ __launch_bounds__(kSelThreads) void select_kernel(SelectArgs a) {
         a.flag[item] = (unsigned char)f;
     }
     // kept offsets in ascending index order (dz-major), by rank counting
-    int* out = a.sel + (long long)item * a.topk;
     for (int i = threadIdx.x; i < a.topk; i += kSelThreads) {
         if (i < k) {
             const int v = val2[i];
             int rank = 0;
             for (int j = 0; j < k; ++j) rank += val2[j] < v;
-            out[rank] = v;
+            kept[rank] = v;
         } else {
-            out[i] = kNoOffset;
+            kept[i] = kNoOffset;
         }
     }
+    __syncthreads();
+    if (wv == 0) merge_offsets(a, item, kept);
 }
 
 // ---------------------------------------------------------------------------
@@ -1314,79 +1386,12 @@ __global__ __launch_bounds__(kSelThreads) void select_kernel(SelectArgs a) {
 
 struct PrunedArgs {
     TiledArgs t;                    // problem, tiles (group = 1), workspace partials
-    const int* sel;                 // [items][topk]
     unsigned char* flag;            // [items]: 1 flagged by the selection, 2 by the error check
     const float* boxL;              // [n][N] window sums of the CT
-    const int* merged;              // [items][kMergedStride] offset lists (merge_offsets_kernel)
+    const int* merged;              // [items][kMergedStride] offset lists (merge_offsets)
     int ncand;                      // NH^3
     float max_err;                  // > 0: error bound (label units) above which an item is flagged
 };
-
-// Per (tile, atlas) item, the offsets the pruned kernel evaluates, in its
-// order: per dz plane (ascending), the kept offsets, then the lattice samples
-// that are not kept (a sample that is also kept counts once, as kept).  One
-// wave per item, every entry placed by counting: a kept offset goes after the
-// kept offsets before it and the samples of the earlier planes; a sample goes
-// after the kept offsets of its plane and the planes before, and after the
-// samples before it.  Entry 0 holds the count and the number of samples;
-// entry 1 + k holds offset k as (sample << 31) | ((dz + 8) << 16) | LDS delta
-// (dy + dx rows of the slab, row length cw).
-constexpr int kMergeWaves = 4;
-constexpr int kMergedStride = 96;   // >= 1 + kMaxOffsets
-static_assert(kMergedStride >= 1 + kMaxOffsets, "merged list stride");
-static_assert(kMaxTopk <= 64 && kSamples <= 64, "one lane per kept offset and per sample");
-
-struct MergeArgs {
-    const int* sel;                 // [items][topk] kept offsets, ascending, kNoOffset after
-    int* merged;                    // [items][kMergedStride]
-    long long items;
-    int topk, hw, cw;
-    int n_samples;
-    int samples[kSamples];          // lattice offset indices, ascending
-};
-
-__global__ __launch_bounds__(kMergeWaves * 64) void merge_offsets_kernel(MergeArgs a) {
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const long long item = (long long)blockIdx.x * kMergeWaves + wv;
-    if (item >= a.items) return;   // per wave; no workgroup barrier below
-    const int nw1 = 2 * a.hw + 1, nw2 = nw1 * nw1;
-    const int kv = lane < a.topk ? a.sel[item * a.topk + lane] : kNoOffset;
-    int sv = kNoOffset;   // the lane's sample (uniform indices into the arguments)
-    for (int j = 0; j < kSamples; ++j)
-        if (j == lane && j < a.n_samples) sv = a.samples[j];
-    const bool has_k = kv < kNoOffset, has_s = sv < kNoOffset;
-    bool dup = false;
-    for (int q = 0; q < a.topk; ++q) dup |= __shfl(kv, q) == sv;
-    const unsigned long long smask = __ballot(has_s && !dup);   // samples evaluated
-    const unsigned long long kmask = __ballot(has_k);
-    const int klo = has_k ? (kv / nw2) * nw2 : 0;          // first offset of the kept plane
-    const int shi = has_s ? (sv / nw2 + 1) * nw2 : 0;      // end of the sample's plane
-    int before_k = 0, before_s = 0;
-    for (int j = 0; j < a.n_samples; ++j)
-        before_k += (int)((smask >> j) & 1ull) & (__shfl(sv, j) < klo);
-    for (int q = 0; q < a.topk; ++q) before_s += __shfl(kv, q) < shi;
-    auto pack = [&](int o, unsigned smpl) {
-        const int dz = o / nw2 - a.hw;
-        const int del = ((o / nw1) % nw1) * a.cw + o % nw1;
-        return (int)((smpl << 31) | ((unsigned)(dz + 8) << 16) | (unsigned)del);
-    };
-    // the kept offsets of a dz plane in (dy, dx) order, the order in which
-    // the plain kernel sweeps a slab's candidates (dy outer, dx inner), so
-    // that evaluating every candidate sums in the plain kernel's order: the
-    // rank among the kept offsets by the key (dz, dy, dx), made once per lane
-    // (every lane runs the shuffles; only lanes with a kept offset use the rank)
-    const int key = has_k ? (kv / nw2) * nw2 + (kv % nw1) * nw1 + (kv / nw1) % nw1 : INT_MAX;
-    int rank = 0;
-    for (int q = 0; q < a.topk; ++q) rank += __shfl(key, q) < key;
-    int* out = a.merged + item * kMergedStride;
-    if (has_k) out[1 + rank + before_k] = pack(kv, 0u);
-    if (has_s && !dup)
-        out[1 + before_s + __popcll(smask & ((1ull << lane) - 1ull))] = pack(sv, 1u);
-    if (lane == 0) {
-        const int ns = __popcll(smask);
-        out[0] = (__popcll(kmask) + ns) | (ns << 16);
-    }
-}
 
 // Sums over the lattice samples of the lane's first output (z0, x = xb),
 // for the error estimate of the tail term: w L and L (the sum of w is Ws).
@@ -1475,7 +1480,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) vo
     const int tx = t % args.tiles_x;
     const int tz = t / args.tiles_x;
 
-    // the offset list (merge_offsets_kernel): per dz plane (ascending), the kept
+    // the offset list (merge_offsets): per dz plane (ascending), the kept
     // offsets, then the lattice samples that are not kept.  Entry k sits in lane
     // k & 63 of one of two registers and comes out by a lane read: read through
     // LDS, or from memory, the fields of an entry cost as much latency as its
@@ -1688,7 +1693,6 @@ extern "C" int pct_fuse_pruned_dev(const pct_problem* pb, const float* params,
     const size_t o_embT = off; off = align(off + 32 * (size_t)N);
     const size_t o_embA = off; off = align(off + 32 * (size_t)N * n);
     const size_t o_boxL = off; off = align(off + sizeof(float) * (size_t)N * n);
-    const size_t o_sel = off; off = align(off + sizeof(int) * (size_t)items * topk);
     const size_t o_flag = off; off = align(off + (size_t)items);
     const size_t o_merged = off; off = align(off + sizeof(int) * (size_t)items * kMergedStride);
     void* ws = nullptr;
@@ -1789,12 +1793,22 @@ extern "C" int pct_fuse_pruned_dev(const pct_problem* pb, const float* params,
         rc = launch_embed(params, model, d_img, pb->nx, pb->ny, pb->nz, 1, embT, s);
         if (!rc) rc = launch_embed(params, model, d_atlas, pb->nx, pb->ny, pb->nz, n, embA, s);
     } else {
-        rc = launch_embed_windows(params, model, d_img, 1, 0, pb, g, t_oy, t_wx, sh.bz, embT, s);
         const int* d_zlist = nullptr;
-        if (!rc && !zlist.empty()) rc = device_zlist(dev, zlist, s, &d_zlist);
-        if (!rc)
-            rc = launch_embed_windows(params, model, d_atlas, n, hw, pb, g, t_oy, t_wx, sh.bz,
-                                      embA, s, d_zlist, (int)zlist.size());
+        if (!zlist.empty()) rc = device_zlist(dev, zlist, s, &d_zlist);
+        if (!rc && g.n_tiles > 0) {
+            EmbedWinArgs ea, et;
+            int na = 0, nt = 0;
+            rc = embed_windows_args(params, model, d_atlas, n, hw, pb, g, t_oy, t_wx, sh.bz, embA,
+                                    d_zlist, (int)zlist.size(), &ea, &na);
+            if (!rc)
+                rc = embed_windows_args(params, model, d_img, 1, 0, pb, g, t_oy, t_wx, sh.bz,
+                                        embT, nullptr, 0, &et, &nt);
+            if (!rc) {
+                hipLaunchKernelGGL(embed_windows_kernel, dim3((unsigned)(na + nt)),
+                                   dim3(kEmbWaves * 64), 0, s, ea, na, et);
+                if (hipGetLastError() != hipSuccess) rc = PCT_ERR_HIP;
+            }
+        }
     }
     if (rc) return rc;
 
@@ -1802,7 +1816,10 @@ extern "C" int pct_fuse_pruned_dev(const pct_problem* pb, const float* params,
     SelectArgs sa;
     sa.embT = embT;
     sa.embA = embA;
-    sa.sel = reinterpret_cast<int*>(w + o_sel);
+    sa.merged = reinterpret_cast<int*>(w + o_merged);
+    sa.cw = sh.seg_width + 2 * hw;   // LDS row length of the tiled slab (TiledCfg::CW)
+    sa.n_samples = n_samples;
+    std::memcpy(sa.samples, samples, sizeof(samples));
     sa.flag = reinterpret_cast<unsigned char*>(w + o_flag);
     sa.N = N;
     sa.nx = pb->nx;
@@ -1858,30 +1875,11 @@ extern "C" int pct_fuse_pruned_dev(const pct_problem* pb, const float* params,
     // after the second stream's work
     if (hipStreamWaitEvent(s, g_side.join[dev], 0) != hipSuccess) return PCT_ERR_HIP;
     side_lk.unlock();
-    pa.sel = sa.sel;
     pa.flag = sa.flag;
     pa.boxL = boxL;
     pa.ncand = ncand;
     pa.max_err = opts->max_err > 0.f ? opts->max_err : 0.f;
-    // the evaluated offsets of every item, merged once (one wave per item)
-    {
-        MergeArgs ma;
-        ma.sel = sa.sel;
-        ma.merged = reinterpret_cast<int*>(w + o_merged);
-        ma.items = items;
-        ma.topk = topk;
-        ma.hw = hw;
-        ma.cw = sh.seg_width + 2 * hw;   // LDS row length of the tiled slab (TiledCfg::CW)
-        ma.n_samples = n_samples;
-        std::memcpy(ma.samples, samples, sizeof(samples));
-        if (items > 0) {
-            hipLaunchKernelGGL(merge_offsets_kernel,
-                               dim3((unsigned)((items + kMergeWaves - 1) / kMergeWaves)),
-                               dim3(kMergeWaves * 64), 0, s, ma);
-            if (hipGetLastError() != hipSuccess) return PCT_ERR_HIP;
-        }
-        pa.merged = ma.merged;
-    }
+    pa.merged = sa.merged;
     PrunedFn fn = pe->fn[hw - 1];
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
                               hipFuncAttributeMaxDynamicSharedMemorySize, g.lds_bytes);
