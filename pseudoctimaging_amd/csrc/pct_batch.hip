@@ -537,6 +537,7 @@ using namespace pct;
 
 extern "C" size_t pct_fuse_batch_workspace_size(const pct_subject* subjects, int n_subjects) {
     if (validate_batch(subjects, n_subjects)) return 0;
+    (void)check_device(nullptr);   // so that the call that follows chooses the same
     BatchPlan p;
     if (!plan_batch(subjects, n_subjects, choose_batch(subjects, n_subjects), &p)) return 0;
     return p.ws_bytes;

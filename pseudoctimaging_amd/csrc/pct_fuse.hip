@@ -929,6 +929,9 @@ extern "C" int pct_normalize_labels_dev(float* d_label, size_t n, pct_stream_t s
 extern "C" size_t pct_fuse_workspace_size(const pct_problem* pb, int choice) {
     if (validate_problem(pb) != PCT_OK) return 0;
     if (!is_tiled_choice(pb, choice)) return 0;
+    // the choice depends on the kernels' occupancy: known from here on, so that the
+    // call that follows chooses the same
+    (void)check_device(nullptr);
     int sid = 0;
     TileGeometry g;
     if (!choose(pb, &sid, nullptr, &g)) return 0;
@@ -949,9 +952,13 @@ static int fuse_dev_impl(const pct_problem* pb, const float* img, const float* a
     int sid = 0;
     TileGeometry g;
     if (!choose(pb, &sid, nullptr, &g)) return PCT_ERR_UNSUPPORTED;
-    const size_t need = tiled_ws_bytes(pb, g.n_parts(), sid);
+    size_t need = tiled_ws_bytes(pb, g.n_parts(), sid);
     if (own_ws) {
         rc = ensure_workspace(dev, need, &ws);
+        if (rc == PCT_ERR_NO_MEMORY && g.n_split > 1 && make_geometry(pb, sid, g.group, &g, 1)) {
+            need = tiled_ws_bytes(pb, g.n_parts(), sid);   // the partial sums of a whole window
+            rc = ensure_workspace(dev, need, &ws);
+        }
         if (rc) return rc;
         ws_bytes = need;
     } else if (!ws || ws_bytes < need || (reinterpret_cast<uintptr_t>(ws) & 255)) {
@@ -1255,10 +1262,15 @@ static int fuse_host_impl(const pct_problem* pb, const float* img, const float* 
     const bool tiled = is_tiled_choice(pb, choice) && choose(pb, &sid, nullptr, &g);
     void* ws = nullptr;
     {
-        size_t need = post ? postprocess_ws_bytes(pb->nh, pb->nx, pb->ny, pb->nz) : 0;
-        if (tiled) need = std::max(need, tiled_ws_bytes(pb, g.n_parts(), sid));
-        if (!need) need = 256;
-        rc = host_workspace(st, need, &ws);
+        const size_t post_need =
+            std::max<size_t>(post ? postprocess_ws_bytes(pb->nh, pb->nx, pb->ny, pb->nz) : 0, 256);
+        auto need = [&]() {
+            return tiled ? std::max(post_need, tiled_ws_bytes(pb, g.n_parts(), sid)) : post_need;
+        };
+        rc = host_workspace(st, need(), &ws);
+        if (rc == PCT_ERR_NO_MEMORY && tiled && g.n_split > 1 &&
+            make_geometry(pb, sid, g.group, &g, 1))
+            rc = host_workspace(st, need(), &ws);   // the partial sums of a whole window
     }
     f32x2* le = tiled && is_xterm_shape(sid)
                     ? reinterpret_cast<f32x2*>(static_cast<char*>(ws) +

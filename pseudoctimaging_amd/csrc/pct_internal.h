@@ -26,7 +26,7 @@ struct TileGeometry {
     int hw = 0, r = 0;
     int tiles_y = 0, tiles_x = 0, tiles_z = 0;
     int group = 1, n_groups = 1;   // atlases per group, groups
-    int n_split = 1;               // parts the window's dz are split into
+    int n_split = 1;               // parts the window is split into
     long long n_tiles = 0, n_items = 0;
     int lds_bytes = 0;
     int wg_per_cu = 0;
