@@ -14,7 +14,8 @@ Extra fields:
                 profiles/, used only when the profile's source stamp matches
                 the kernel sources built here) / kernel time; frac =
                 achieved / peak; issue_frac = VALU instructions issued /
-                the non-packed issue ceiling.  effective_tflops counts the
+                one per 4 cycles and SIMD (plain instructions of two waves
+                pair, so it can pass 1).  effective_tflops counts the
                 reference's direct formulation instead (86 FLOP per
                 candidate-voxel pair: 27 sub + 27 FMA + scale + exp + 3 for
                 the accumulation), which the kernel's box-sum reuse beats.
@@ -55,7 +56,7 @@ METRIC = ("pseudo-CT voxels/s @222\u00d7222\u00d7112 n=10 NH=11: plain vs learne
 KERNEL_SOURCES = ("pseudoctimaging_amd/csrc/pct_tiled.h", "pseudoctimaging_amd/csrc/pct_fuse.hip",
                   "pseudoctimaging_amd/csrc/pct_learned.hip", "pseudoctimaging_amd/csrc/Makefile")
 PROFILE = os.path.join("profiles", "fuse_tiled_222x222x112_n10_nh11_traffic.json")
-VALU_ISSUE_PER_S = 1024 * 2.4e9 / 4   # wave64 FP32 instructions, non-packed
+VALU_ISSUE_PER_S = 1024 * 2.4e9 / 4   # wave64 FP32 instructions of one wave per SIMD
 
 
 def kernel_source_stamp() -> str:
