@@ -172,9 +172,10 @@ __device__ __forceinline__ v4f relu(v4f v) {
 
 // Bound by the matrix pipe: 112 products of 32 cycles for 16 slots, 31 us at
 // 3.4e5 slots (60 us measured, with the fragments' loads; 181 us with one thread
-// per slot and the hidden activations written out).  Each wave keeps the 112 weight fragments in registers and takes
-// a run of consecutive tiles; the next tile's patch loads are in flight during
-// the products.
+// per slot and the hidden activations written out).  Each wave keeps the 112
+// weight fragments in registers and takes a run of consecutive tiles; the next
+// tile's patch loads are in flight during the products.  Fetching the parameters
+// through LDS changes nothing.
 constexpr int kFwdWaves = 4;
 constexpr int kWaves = 2048;   // waves that share the tiles (two per SIMD)
 __global__ __launch_bounds__(kFwdWaves * 64, 2) void train_forward(TrainArgs a, long long tiles,
