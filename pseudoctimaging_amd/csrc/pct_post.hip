@@ -248,8 +248,10 @@ __device__ __forceinline__ bool tile_has_nan(const float* __restrict__ arr, cons
 // kernel or, for up to kPlanScan tiles, with the scan as well: the chain then
 // takes 4 launches on the smallest volumes and 5 on others, where clearing,
 // counting, placing and listing as kernels of their own make it 7 (28x26x24, 0.2 %
-// NaN: 28.0 -> 21.2 us; 222x222x112, 4.2e6 NaN: 1.62 -> 1.56 ms).  Past that one
-// workgroup would be the slower one (or its LDS too small) and those kernels run.
+// NaN: 28.0 -> 21.2 us; 222x222x112, 4.2e6 NaN: 1.62 -> 1.56 ms, with 0.2 % NaN 112.5
+// -> 113.6 us; 128x128x64, 0.2 %: 54.5 -> 52.6).  Past that one workgroup would be
+// the slower one (330x320x200, 45000 tiles, 0.2 %: 350 against 357 us) or its LDS too
+// small, and those kernels run.
 constexpr int kPlanDiags = 4096, kPlanTiles = 1 << 16, kPlanScan = 256, kPlanThreads = 1024;
 
 // The general path: the counters, the scan with its histogram, the places of the
@@ -339,9 +341,31 @@ __global__ __launch_bounds__(kPlanThreads) void fill_plan_kernel(const float* __
             }
         }
     __syncthreads();
+    // the thread's busy tiles: bit 8 i + k is tile 8192 i + 8 threadIdx.x + k (SCAN:
+    // bit 0, tile threadIdx.x)
+    constexpr int kRound = 8 * kPlanThreads;
+    static_assert(kPlanTiles <= 8 * kRound, "one bit per tile");
+    unsigned long long mine = 0;
+    if (SCAN) {
+        mine = (int)threadIdx.x < f.n_tiles && busy[threadIdx.x] ? 1 : 0;
+    } else {
+        for (int i = 0; i * kRound < f.n_tiles; ++i) {
+            const int t0 = i * kRound + 8 * threadIdx.x;
+            if (t0 >= f.n_tiles) break;
+            // up to 7 flags past the last tile's are read: the array is a multiple
+            // of 64 long
+            const int4* p = reinterpret_cast<const int4*>(st.done + t0);
+            const int4 lo = p[0], hi = p[1];
+            const int v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (t0 + k < f.n_tiles && v[k] == 0) mine |= 1ull << (8 * i + k);
+        }
+    }
     auto each = [&](auto use) {   // the busy tiles' (tile, diagonal)
-        for (int t = threadIdx.x; t < f.n_tiles; t += kPlanThreads) {
-            if (SCAN ? !busy[t] : st.done[t] != 0) continue;
+        for (unsigned long long m = mine; m; m &= m - 1) {
+            const int bit = __ffsll((long long)m) - 1;
+            const int t = SCAN ? threadIdx.x : (bit >> 3) * kRound + 8 * threadIdx.x + (bit & 7);
             int i, j, k;
             tile_coords(f, t, &i, &j, &k);
             use(t, i + j + k);
