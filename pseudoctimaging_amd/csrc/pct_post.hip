@@ -180,6 +180,7 @@ constexpr int kAfter = (kSZ - 1) * (kSX - 2) * (kSY - 4), kBefore = kStage - kAf
 constexpr int kAfterLoads = (kAfter + kTileThreads - 1) / kTileThreads;
 constexpr int kBeforeLoads = (kBefore + kTileThreads - 1) / kTileThreads;
 constexpr int kTileWgs = 256;                              // workgroups that take tiles
+constexpr int kWaitStores = 0x0f70;                        // s_waitcnt vmcnt(0), no other counter
 static_assert(kTileLevels <= 32, "one mask bit per level");
 static_assert(kTX % 4 == 0 && kTY >= 4 && kTX >= 2 && kTZ >= 1, "neighbours lie in adjacent tiles");
 
@@ -635,7 +636,13 @@ __global__ __launch_bounds__(kTileThreads) void fill_tiles_kernel(float* arr, Fi
             }
             __syncthreads();
         }
-        __syncthreads();   // every wave's values come before the release
+        // The release below waits for the stores of its own wave alone (and a
+        // workgroup barrier for none in memory), so each wave waits here for the
+        // values it stored: they are in the L2 before the barrier, and the release
+        // writes that back before the flag.
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(kWaitStores);
+        __syncthreads();
         if (tid == 0)
             __hip_atomic_store(st.done + tile, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
     }
