@@ -125,11 +125,20 @@ int pct_fuse_dev(const pct_problem* pb, const float* d_img, const float* d_atlas
                  const float* d_atlas_label_norm, float* d_out, int choice,
                  pct_stream_t stream);
 
-/* Bytes of device workspace pct_fuse_dev_ws needs for this problem/choice. */
+/* Bytes of device workspace pct_fuse_dev_ws needs for this problem/choice:
+ * 8 * nx*ny*nz * n_atlas for the partial sums, and as much again where a
+ * cross-term configuration may be chosen (NH 7 to 15, MRI of unit range within
+ * its bound at this sigma and beta; a forced or tuned configuration's own size
+ * where there is one).  It grows with every extent and with n_atlas, so that
+ * a workspace for the largest subject serves the others.  No GPU work. */
 size_t pct_fuse_workspace_size(const pct_problem* pb, int choice);
 
 /* Same as pct_fuse_dev with a caller-provided workspace of at least
- * pct_fuse_workspace_size() bytes (256-byte aligned). */
+ * pct_fuse_workspace_size() bytes (256-byte aligned), and the same output bits
+ * whatever its size.  Small volumes split the window into parts with a partial
+ * sum each: a workspace that holds fewer of these sums runs the parts in
+ * rounds.  256 MiB above the size hold them all for every problem
+ * (30x34x22, n = 2, NH = 7: 15 us, in the least workspace 95). */
 int pct_fuse_dev_ws(const pct_problem* pb, const float* d_img, const float* d_atlas,
                     const float* d_atlas_label_norm, float* d_out, int choice,
                     void* d_workspace, size_t workspace_bytes, pct_stream_t stream);
@@ -160,7 +169,7 @@ typedef struct pct_tile_config {
     int atlas_group;   /* atlases per work item */
     int lds_bytes;     /* dynamic LDS per workgroup */
     long long items;   /* work items (workgroups) launched */
-    double est_cost;   /* cost-model estimate (arbitrary units) */
+    double est_cost;   /* cost-model estimate (microseconds) */
     double measured_ms;/* <0 if not measured */
     int form;          /* 0: squared differences per candidate; 1: cross terms
                           (2 T'A' products, per-voxel 2^-AA folded into the

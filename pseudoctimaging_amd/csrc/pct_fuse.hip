@@ -97,6 +97,17 @@ __global__ __launch_bounds__(64 * kFinRows) void fuse_finalize(const float* __re
     out[idx] = v;
 }
 
+// Adds the n partial sums after the first to it, in order, as the finalize pass
+// would (see launch_rounds).
+__global__ __launch_bounds__(256) void fold_partials(float* __restrict__ ws, int n,
+                                                     long long floats) {
+    const long long i = blockIdx.x * 256LL + threadIdx.x;
+    if (i >= floats) return;
+    float v = ws[i];
+    for (int j = 1; j <= n; ++j) v += ws[j * floats + i];
+    ws[i] = v;
+}
+
 // ---------------------------------------------------------------------------
 // direct kernel (GM / GM2 surface)
 // ---------------------------------------------------------------------------
@@ -422,6 +433,7 @@ bool make_geometry(const pct_problem* pb, int shape_id, int group, TileGeometry*
     const int nw = 2 * hw + 1;
     if (s.form == 1) split = std::min(split, nw);
     g->n_split = split <= nw ? std::max(1, split) : nw * std::min(split / nw, nw);
+    g->slots = 0;
     g->n_items = g->n_tiles * g->n_parts();
     g->lds_bytes = e->lds_bytes;
     const int by_lds = kLdsPerCu / e->lds_bytes;
@@ -538,6 +550,13 @@ static bool unit_range_in_bound(const pct_problem* pb) {
     return std::sqrt(1.4426950408889634 / problem_divisor(pb)) <= (double)kXtBound;
 }
 
+// Whether the model may pick a cross-term shape.  Below NH 7 it never does: the
+// candidates are too few to pay for the pair pre-pass.  Written down because the
+// size of a caller's workspace depends on it.
+static bool may_take_xterm(const pct_problem* pb) {
+    return (pb->nh - 1) / 2 >= 3 && unit_range_in_bound(pb);
+}
+
 // Candidate splits of the window: whole, halves, thirds, pairs of dz, single ones,
 // and halves, thirds, fifths and single dy of each.  The partial sums of a split may not need more memory than 256 MiB (or
 // than the groups alone).  Groups are of one atlas: several to an item save up to
@@ -578,45 +597,51 @@ static Config model_choice(const pct_problem* pb, bool xt, bool* known) {
     Config best;
     double best_us = -1;
     *known = true;
-    for (int pass = 0; pass < 2 && best_us < 0; ++pass)   // any shape where none fits
-        for (int sid = 0; sid < (int)shapes().size(); ++sid) {
-            if (pass == 0 && !xt && shapes()[sid].form == 1) continue;
-            for (int sp : candidate_splits(pb, 1)) {
-                const double us = model_cost(pb, sid, 1, nullptr, sp);
-                if (us < 0) continue;
-                if (best_us < 0 || us < best_us * 0.999) {
-                    best_us = us;
-                    best = Config{sid, 1, sp};
-                }
+    for (int sid = 0; sid < (int)shapes().size(); ++sid) {
+        if (!xt && shapes()[sid].form == 1) continue;
+        for (int sp : candidate_splits(pb, 1)) {
+            const double us = model_cost(pb, sid, 1, nullptr, sp);
+            if (us < 0) continue;
+            if (best_us < 0 || us < best_us * 0.999) {
+                best_us = us;
+                best = Config{sid, 1, sp};
             }
         }
+    }
     if (best.shape_id >= 0) *known = find_entry(best.shape_id, (pb->nh - 1) / 2)->occupancy > 0;
     return best;
+}
+
+// The forced or tuned configuration of a problem, if there is one.
+static bool fixed_config(const pct_problem* pb, Config* c) {
+    std::lock_guard<std::mutex> lk(g_cfg_mutex);
+    if (g_forced_id >= 0) {
+        *c = Config{g_forced_id, g_forced_group > 0 ? g_forced_group : 1, 1};
+        return true;
+    }
+    const auto it = g_tuned.find(ShapeKey{pb->nx, pb->ny, pb->nz, pb->n_atlas, pb->nh});
+    if (it == g_tuned.end()) return false;
+    *c = it->second;
+    return true;
 }
 
 // The configuration of a problem: forced, tuned, or the model's.
 static bool choose(const pct_problem* pb, int* shape_id, double* cost, TileGeometry* geo) {
     Config c;
-    const ShapeKey key{pb->nx, pb->ny, pb->nz, pb->n_atlas, pb->nh};
-    {
+    if (!fixed_config(pb, &c)) {
+        const bool xt = may_take_xterm(pb);
+        const auto key =
+            std::make_pair(ShapeKey{pb->nx, pb->ny, pb->nz, pb->n_atlas, pb->nh}, xt);
         std::lock_guard<std::mutex> lk(g_cfg_mutex);
-        if (g_forced_id >= 0) {
-            c = Config{g_forced_id, g_forced_group > 0 ? g_forced_group : 1, 1};
-        } else if (auto it = g_tuned.find(key); it != g_tuned.end()) {
-            c = it->second;
+        const auto pl = g_planned.find(key);
+        if (pl != g_planned.end()) {
+            c = pl->second;
         } else {
-            const bool xt = unit_range_in_bound(pb);
-            const auto pk = std::make_pair(key, xt);
-            const auto pl = g_planned.find(pk);
-            if (pl != g_planned.end()) {
-                c = pl->second;
-            } else {
-                bool known = false;   // whether a device's occupancy went into it
-                c = model_choice(pb, xt, &known);
-                if (known) {
-                    if (g_planned.size() >= kPlanned) g_planned.clear();
-                    g_planned.emplace(pk, c);
-                }
+            bool known = false;   // whether a device's occupancy went into it
+            c = model_choice(pb, xt, &known);
+            if (known) {
+                if (g_planned.size() >= kPlanned) g_planned.clear();
+                g_planned.emplace(key, c);
             }
         }
     }
@@ -695,17 +720,44 @@ bool is_xterm_shape(int shape_id) {
     return shape_id >= 0 && shape_id < (int)shapes().size() && shapes()[shape_id].form == 1;
 }
 
-size_t tiled_le_offset(const pct_problem* pb, int n_parts) {
+size_t tiled_le_offset(const pct_problem* pb, int n_slots) {
     const size_t N = (size_t)pb->nx * pb->ny * pb->nz;
-    return ((2 * (size_t)n_parts * N * sizeof(float)) + 255) & ~(size_t)255;
+    return ((2 * (size_t)n_slots * N * sizeof(float)) + 255) & ~(size_t)255;
 }
 
-size_t tiled_ws_bytes(const pct_problem* pb, int n_parts, int shape_id) {
+static size_t pairs_bytes(const pct_problem* pb) {
     const size_t N = (size_t)pb->nx * pb->ny * pb->nz;
-    size_t bytes = tiled_le_offset(pb, n_parts);
-    if (is_xterm_shape(shape_id))
-        bytes += ((size_t)pb->n_atlas * N * sizeof(f32x2) + 255) & ~(size_t)255;
-    return bytes;
+    return ((size_t)pb->n_atlas * N * sizeof(f32x2) + 255) & ~(size_t)255;
+}
+
+size_t tiled_ws_bytes(const pct_problem* pb, int n_slots, int shape_id) {
+    return tiled_le_offset(pb, n_slots) + (is_xterm_shape(shape_id) ? pairs_bytes(pb) : 0);
+}
+
+// Workspace that the configuration `choose` takes can run in: the partial sums of
+// whole windows, and the pairs where the model may pick a cross-term shape.  It
+// depends on the problem alone (not on what the model picks, nor on the device),
+// grows with every extent and the atlases, and touches no GPU.
+static size_t least_ws_bytes(const pct_problem* pb) {
+    Config c;
+    if (!fixed_config(pb, &c))
+        return tiled_le_offset(pb, pb->n_atlas) + (may_take_xterm(pb) ? pairs_bytes(pb) : 0);
+    TileGeometry g;
+    if (!make_geometry(pb, c.shape_id, c.group, &g)) return 0;
+    return tiled_ws_bytes(pb, g.n_groups, c.shape_id);
+}
+
+// Lets the geometry keep as many partial sums as fit `bytes`; false where not one does.
+static bool fit_slots(const pct_problem* pb, int shape_id, size_t bytes, TileGeometry* g) {
+    g->slots = 0;
+    if (tiled_ws_bytes(pb, g->n_parts(), shape_id) <= bytes) return true;
+    const size_t N = (size_t)pb->nx * pb->ny * pb->nz;
+    const size_t fixed = is_xterm_shape(shape_id) ? pairs_bytes(pb) : 0;
+    if (bytes < fixed) return false;
+    // the sums end on a multiple of 256 bytes
+    const size_t most = ((bytes - fixed) & ~(size_t)255) / (8 * N);
+    g->slots = (int)std::min<size_t>(most, (size_t)g->n_parts() - 1);
+    return g->slots > 0;
 }
 
 int launch_atlas_pairs(const pct_problem* pb, const float* atlas, const float* label,
@@ -744,8 +796,10 @@ int launch_finalize(const pct_problem* pb, const TileGeometry& g, const float* w
     const long long N = (long long)pb->nx * pb->ny * pb->nz;
     const dim3 fb(64 * kFinRows),
         fgrid((pb->ny + 63) / 64, (pb->nx + kFinRows - 1) / kFinRows, pb->nz);
-    hipLaunchKernelGGL(fuse_finalize, fgrid, fb, 0, stream, ws, g.n_items > 0 ? g.n_parts() : 0, N,
-                       pb->nx, pb->ny, pb->nz, g.r, out);
+    // parts that ran in rounds are one sum by now
+    const int n = g.n_items <= 0 ? 0 : g.slots ? 1 : g.n_parts();
+    hipLaunchKernelGGL(fuse_finalize, fgrid, fb, 0, stream, ws, n, N, pb->nx, pb->ny, pb->nz, g.r,
+                       out);
     return hipGetLastError() == hipSuccess ? PCT_OK : PCT_ERR_HIP;
 }
 
@@ -768,6 +822,9 @@ TiledArgs make_tiled_args(const pct_problem* pb, const TileGeometry& g, const fl
     a.n_atlas = pb->n_atlas;
     a.group = g.group;
     a.n_split = g.n_split;
+    a.parts = g.n_split;
+    a.first_part = 0;
+    a.add = 0;
     const double div = problem_divisor(pb);
     a.scale = (float)std::sqrt(1.4426950408889634 / div);
     a.only = nullptr;
@@ -826,27 +883,59 @@ TimedLaunch::~TimedLaunch() {
     if (end) (void)hipEventRecord(end, s);
 }
 
+// The items of `a` where the workspace holds fewer partial sums than there are
+// parts: as many consecutive parts a launch (whole groups, or parts of one) as it
+// holds, each round's sums added to the first one, which the next round's first
+// item goes on from.  The partial sums are added one after another in the order of
+// the finalize pass, so the output has the same bits as with all of them in memory.
+// In the least workspace 30x34x22, n = 2, NH = 7 takes 95 us (15 with all 14 parts in
+// memory), 60x60x60, n = 1, NH = 15 473 us (127), 96x96x64, n = 4, NH = 11 629 us; items of
+// whole windows in the same memory took 83, 498 and 799.
+static int launch_rounds(const TiledArgs& all, const TileGeometry& g, int shape_id,
+                         hipStream_t stream) {
+    const int groups = std::max(1, g.slots / g.n_split);   // a launch
+    const int parts = std::min(g.slots, g.n_split);
+    for (int g0 = 0; g0 < g.n_groups; g0 += groups)
+        for (int first = 0; first < g.n_split; first += parts) {
+            const int ng = std::min(groups, g.n_groups - g0);
+            const int a0 = g0 * g.group, a1 = std::min(all.n_atlas, (g0 + ng) * g.group);
+            TiledArgs a = all;
+            a.atlas += (long long)a0 * a.N;
+            a.label += (long long)a0 * a.N;
+            if (a.le) a.le += (long long)a0 * a.N;
+            a.n_atlas = a1 - a0;
+            a.first_part = first;
+            a.parts = std::min(parts, g.n_split - first);
+            a.add = g0 > 0 || first > 0;
+            a.n_items = (int)(g.n_tiles * ng * a.parts);
+            const int rc = launch_tiled_items(a, shape_id, g.hw, stream);
+            if (rc) return rc;
+            if (ng * a.parts > 1) {
+                hipLaunchKernelGGL(fold_partials, dim3((unsigned)((2 * a.N + 255) / 256)),
+                                   dim3(256), 0, stream, a.ws, ng * a.parts - 1, 2 * a.N);
+                if (hipGetLastError() != hipSuccess) return PCT_ERR_HIP;
+            }
+        }
+    return PCT_OK;
+}
+
 static int launch_tiled(const pct_problem* pb, const float* img, const float* atlas,
                         const float* label, float* out, void* ws, size_t ws_bytes,
                         int shape_id, const TileGeometry& g, hipStream_t stream) {
-    const TiledEntry* e = find_entry(shape_id, g.hw);
-    if (!e) return PCT_ERR_UNSUPPORTED;
-    if (ws_bytes < tiled_ws_bytes(pb, g.n_parts(), shape_id)) return PCT_ERR_INVALID;
+    if (ws_bytes < tiled_ws_bytes(pb, g.n_slots(), shape_id)) return PCT_ERR_INVALID;
     TiledArgs a = make_tiled_args(pb, g, img, atlas, label, static_cast<float*>(ws));
     if (is_xterm_shape(shape_id) && g.n_items > 0) {
         f32x2* le = reinterpret_cast<f32x2*>(static_cast<char*>(ws) +
-                                             tiled_le_offset(pb, g.n_parts()));
+                                             tiled_le_offset(pb, g.n_slots()));
         const int rc = launch_atlas_pairs(pb, atlas, label, pb->n_atlas, a.scale, le, stream);
         if (rc) return rc;
         a.le = le;
     }
     if (g.n_items > 0) {
-        void* kargs[] = {&a};
         TimedLaunch timed(stream);
-        if (hipLaunchKernel(reinterpret_cast<const void*>(e->fn), dim3((unsigned)g.n_items),
-                            dim3(e->shape.waves * 64), kargs, (size_t)e->lds_bytes,
-                            stream) != hipSuccess)
-            return PCT_ERR_HIP;
+        const int rc = g.slots ? launch_rounds(a, g, shape_id, stream)
+                               : launch_tiled_items(a, shape_id, g.hw, stream);
+        if (rc) return rc;
     }
     return launch_finalize(pb, g, static_cast<const float*>(ws), out, stream);
 }
@@ -929,13 +1018,10 @@ extern "C" int pct_normalize_labels_dev(float* d_label, size_t n, pct_stream_t s
 extern "C" size_t pct_fuse_workspace_size(const pct_problem* pb, int choice) {
     if (validate_problem(pb) != PCT_OK) return 0;
     if (!is_tiled_choice(pb, choice)) return 0;
-    // the choice depends on the kernels' occupancy: known from here on, so that the
-    // call that follows chooses the same
-    (void)check_device(nullptr);
     int sid = 0;
     TileGeometry g;
     if (!choose(pb, &sid, nullptr, &g)) return 0;
-    return tiled_ws_bytes(pb, g.n_parts(), sid);
+    return least_ws_bytes(pb);
 }
 
 static int fuse_dev_impl(const pct_problem* pb, const float* img, const float* atlas,
@@ -952,18 +1038,18 @@ static int fuse_dev_impl(const pct_problem* pb, const float* img, const float* a
     int sid = 0;
     TileGeometry g;
     if (!choose(pb, &sid, nullptr, &g)) return PCT_ERR_UNSUPPORTED;
-    size_t need = tiled_ws_bytes(pb, g.n_parts(), sid);
     if (own_ws) {
-        rc = ensure_workspace(dev, need, &ws);
-        if (rc == PCT_ERR_NO_MEMORY && g.n_split > 1 && make_geometry(pb, sid, g.group, &g, 1)) {
-            need = tiled_ws_bytes(pb, g.n_parts(), sid);   // the partial sums of a whole window
-            rc = ensure_workspace(dev, need, &ws);
+        ws_bytes = tiled_ws_bytes(pb, g.n_parts(), sid);
+        rc = ensure_workspace(dev, ws_bytes, &ws);
+        if (rc == PCT_ERR_NO_MEMORY && g.n_split > 1) {
+            ws_bytes = tiled_ws_bytes(pb, g.n_groups, sid);   // of whole windows
+            rc = ensure_workspace(dev, ws_bytes, &ws);
         }
         if (rc) return rc;
-        ws_bytes = need;
-    } else if (!ws || ws_bytes < need || (reinterpret_cast<uintptr_t>(ws) & 255)) {
+    } else if (!ws || ws_bytes < least_ws_bytes(pb) || (reinterpret_cast<uintptr_t>(ws) & 255)) {
         return PCT_ERR_INVALID;
     }
+    if (!fit_slots(pb, sid, ws_bytes, &g)) return PCT_ERR_INVALID;
     return launch_tiled(pb, img, atlas, label, out, ws, ws_bytes, sid, g, stream);
 }
 
@@ -1265,21 +1351,23 @@ static int fuse_host_impl(const pct_problem* pb, const float* img, const float* 
         const size_t post_need =
             std::max<size_t>(post ? postprocess_ws_bytes(pb->nh, pb->nx, pb->ny, pb->nz) : 0, 256);
         auto need = [&]() {
-            return tiled ? std::max(post_need, tiled_ws_bytes(pb, g.n_parts(), sid)) : post_need;
+            return tiled ? std::max(post_need, tiled_ws_bytes(pb, g.n_slots(), sid)) : post_need;
         };
         rc = host_workspace(st, need(), &ws);
-        if (rc == PCT_ERR_NO_MEMORY && tiled && g.n_split > 1 &&
-            make_geometry(pb, sid, g.group, &g, 1))
-            rc = host_workspace(st, need(), &ws);   // the partial sums of a whole window
+        if (rc == PCT_ERR_NO_MEMORY && tiled && g.n_split > 1) {
+            g.slots = g.n_groups;   // the partial sums of whole windows
+            rc = host_workspace(st, need(), &ws);
+        }
     }
     f32x2* le = tiled && is_xterm_shape(sid)
                     ? reinterpret_cast<f32x2*>(static_cast<char*>(ws) +
-                                               tiled_le_offset(pb, g.n_parts()))
+                                               tiled_le_offset(pb, g.n_slots()))
                     : nullptr;
     // cu:1687-1699: host->device copies
     if (!rc) rc = stage_h2d(st, st.img, img, N * 4, cs);
     if (!rc && tiled) {
-        const int chunks = std::min(g.n_groups, kCopyChunks);
+        // rounds go through all atlases in order, so they wait for all copies
+        const int chunks = g.slots ? 1 : std::min(g.n_groups, kCopyChunks);
         for (int c = 0; c < chunks && !rc; ++c) {
             const int g0 = (int)((long long)c * g.n_groups / chunks);
             const int g1 = (int)((long long)(c + 1) * g.n_groups / chunks);
@@ -1305,7 +1393,9 @@ static int fuse_host_impl(const pct_problem* pb, const float* img, const float* 
                                         le + off, cstream);
                 a.le = le + off;
             }
-            if (!rc) rc = launch_tiled_items(a, sid, g.hw, cstream);
+            if (!rc)
+                rc = g.slots ? launch_rounds(a, g, sid, cstream)
+                             : launch_tiled_items(a, sid, g.hw, cstream);
         }
         if (!rc && (hipEventRecord(st.join, st.compute2) != hipSuccess ||
                     hipStreamWaitEvent(s, st.join, 0) != hipSuccess))

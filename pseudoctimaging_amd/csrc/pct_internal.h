@@ -27,11 +27,14 @@ struct TileGeometry {
     int tiles_y = 0, tiles_x = 0, tiles_z = 0;
     int group = 1, n_groups = 1;   // atlases per group, groups
     int n_split = 1;               // parts the window is split into
+    int slots = 0;                 // where the workspace is too small for all partial sums,
+                                   // how many it holds; 0: all
     long long n_tiles = 0, n_items = 0;
     int lds_bytes = 0;
     int wg_per_cu = 0;
     // partial sums per voxel: one per group and part of the window
     int n_parts() const { return n_groups * n_split; }
+    int n_slots() const { return slots ? slots : n_parts(); }   // of them in memory at a time
 };
 
 // Problem validation shared by every entry point.

@@ -74,7 +74,7 @@ struct TiledArgs {
     const float* img;
     const float* atlas;
     const float* label;
-    float* ws;        // [n_groups * n_split][2][N]
+    float* ws;        // [n_groups * parts][2][N]
     long long N;      // nx*ny*nz
     int nx, ny, nz;
     int r;            // hw + 1
@@ -83,6 +83,9 @@ struct TiledArgs {
     int n_items;
     int n_atlas, group;
     int n_split;      // parts of the window (see WindowPart), each an item of its own
+    // this launch runs the parts first_part .. first_part + parts - 1 of every group;
+    // add: the first item's sums are added to those in memory (see launch_rounds)
+    int parts, first_part, add;
     float scale;      // sqrt(log2(e)/div)
     // optional item filter: when set, items whose byte is 0 are skipped
     const unsigned char* only;
@@ -526,6 +529,18 @@ struct WindowPart {
     int dz_begin, dz_end;   // -HW .. HW + 1
     int dy_first, dy_count;
 };
+// Stores an output's sums, or adds them to those in memory.
+__device__ __forceinline__ void store_sums(float* p, float* s, bool add, float P, float S) {
+    if (add) {   // uniform
+        // rounded before they are added, as in the finalize pass
+        asm volatile("" : "+v"(P), "+v"(S));
+        P = *p + P;
+        S = *s + S;
+    }
+    *p = P;
+    *s = S;
+}
+
 template <int HW>
 __device__ __forceinline__ WindowPart window_part(int sp, int n_split) {
     constexpr int K = 2 * HW + 1;
@@ -542,7 +557,7 @@ __device__ __forceinline__ void tiled_item(const TiledArgs& args, int item,
                                            float* __restrict__ lds) {
     using C = TiledCfg<W, BX, BZ, NW, HW>;
     const int part = item / args.n_tiles;   // (atlas group, part of the window)
-    const int g = part / args.n_split, sp = part - g * args.n_split;
+    const int g = part / args.parts, sp = args.first_part + part - g * args.parts;
     int t = item - part * args.n_tiles;
     const int ty = t % args.tiles_y;
     t /= args.tiles_y;
@@ -606,6 +621,7 @@ __device__ __forceinline__ void tiled_item(const TiledArgs& args, int item,
 
     // Store the group's partial sums for the lane's valid outputs.
     if (ly >= 1 && ly <= W - 2 && y < ny - r) {
+        const bool add = args.add && part == 0;
         float* __restrict__ wsP = args.ws + (long long)(2 * part) * args.N;
         float* __restrict__ wsS = wsP + args.N;
 #pragma unroll
@@ -615,8 +631,7 @@ __device__ __forceinline__ void tiled_item(const TiledArgs& args, int item,
                 const int z = z0 + j, x = xb + i;
                 if (z < nz - r && x < nx - r) {
                     const long long idx = z * plane + (long long)x * ny + y;
-                    wsP[idx] = P[j][i];
-                    wsS[idx] = S[j][i];
+                    store_sums(wsP + idx, wsS + idx, add, P[j][i], S[j][i]);
                 }
             }
     }
@@ -1138,7 +1153,7 @@ __device__ __forceinline__ void tiled_item_xt(const TiledArgs& args, int item,
     using C = TiledCfg<W, BX, BZ, NW, HW>;
     using X = XtCfg<C>;
     const int part = item / args.n_tiles;   // (atlas group, part of the window)
-    const int g = part / args.n_split, sp = part - g * args.n_split;
+    const int g = part / args.parts, sp = args.first_part + part - g * args.parts;
     int t = item - part * args.n_tiles;
     const int ty = t % args.tiles_y;
     t /= args.tiles_y;
@@ -1301,6 +1316,7 @@ __device__ __forceinline__ void tiled_item_xt(const TiledArgs& args, int item,
     }
 
     if (ly >= 1 && ly <= W - 2 && y < ny - r) {
+        const bool add = args.add && part == 0;
         float* __restrict__ wsP = args.ws + (long long)(2 * part) * args.N;
         float* __restrict__ wsS = wsP + args.N;
 #pragma unroll
@@ -1310,8 +1326,8 @@ __device__ __forceinline__ void tiled_item_xt(const TiledArgs& args, int item,
                 const int z = z0 + j, x = xb + i;
                 if (z < nz - r && x < nx - r) {
                     const long long idx = z * plane + (long long)x * ny + y;
-                    wsP[idx] = P[j][i] * f[j][i];
-                    wsS[idx] = S[j][i] * f[j][i];
+                    store_sums(wsP + idx, wsS + idx, add, P[j][i] * f[j][i],
+                               S[j][i] * f[j][i]);
                 }
             }
     }
@@ -1360,11 +1376,11 @@ int check_device(int* dev_out);
 // The library's per-device workspace, grown to at least `bytes`.
 int ensure_workspace(int dev, size_t bytes, void** ptr);
 
-// Bytes of workspace a tiled run of `shape_id` with `n_parts` partial sums per
+// Bytes of workspace a tiled run of `shape_id` with `n_slots` partial sums per
 // voxel needs: the partial sums, then for a cross-term shape the (L * 2^-AA, 2^-AA)
 // pair of every atlas voxel (at tiled_le_offset).
-size_t tiled_ws_bytes(const pct_problem* pb, int n_parts, int shape_id);
-size_t tiled_le_offset(const pct_problem* pb, int n_parts);
+size_t tiled_ws_bytes(const pct_problem* pb, int n_slots, int shape_id);
+size_t tiled_le_offset(const pct_problem* pb, int n_slots);
 
 // Bytes of workspace the device post chain needs for a volume, and the chain
 // itself on a caller's workspace of at least that size (pct_post.hip).

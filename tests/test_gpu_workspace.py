@@ -1,0 +1,76 @@
+"""A window split over work items has a partial sum per part.  With a workspace that
+does not hold them all the parts run in rounds, and every output keeps its bits:
+the least workspace, one slot more, all but one, and all of them, for splits by dz and
+by dy, both forms of the kernel, and slabs out of the cross-term range in a part."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle
+import pseudoctimaging_amd as pct
+from pseudoctimaging_amd import _lib
+from parity import compare
+
+pytestmark = pytest.mark.gpu
+
+
+def _split(shape, n, nh, sigma):
+    """The form and the number of parts of the configuration in use."""
+    c = _lib.TileConfig()
+    pb = pct.problem(shape, n, nh, sigma, 1.0)
+    assert _lib.lib().pct_tile_config_choose(ctypes.byref(pb), ctypes.byref(c)) == 0
+    c = c.as_dict()
+    r = (nh - 1) // 2 + 1
+    iz, ix, iy = (m - 2 * r for m in shape)
+    tiles = -(-iz // c["bz"]) * -(-ix // (c["waves"] * (64 // c["seg_width"]) * c["bx"])) * \
+        -(-iy // (c["seg_width"] - 2))
+    assert c["items"] % (tiles * n) == 0
+    return c["form"], c["items"] // (tiles * n)
+
+
+# volume (z, x, y), atlases, NH, sigma, form, whether dy is split too
+CASES = [((24, 31, 12), 4, 9, 0.3, 0, False), ((13, 16, 23), 1, 7, 2.5, 0, True),
+         ((44, 25, 23), 1, 15, 2.5, 0, True), ((33, 82, 18), 9, 8, 2.5, 1, False),
+         ((71, 73, 19), 2, 9, 2.5, 1, False), ((88, 46, 20), 2, 11, 2.5, 1, False),
+         ((94, 40, 16), 1, 14, 2.5, 1, False), ((53, 33, 48), 1, 15, 2.5, 1, False)]
+
+
+@pytest.mark.parametrize("spike", [False, True])
+@pytest.mark.parametrize("shape,n,nh,sigma,form,dy", CASES)
+def test_any_accepted_workspace_gives_the_same_bits(gpu, shape, n, nh, sigma, form, dy, spike):
+    import torch
+    used, parts = _split(shape, n, nh, sigma)
+    assert used == form and parts > 1 and (parts > nh // 2 * 2 + 1) == dy
+    nz, nx, ny = shape
+    img, amri, lab = pct.synth_tissue(nx, ny, nz, n, 2, False, nh)
+    pct.normalize_labels(lab)
+    if spike:   # values out of the cross-term range: a few of an atlas, one of the target
+        amri[n - 1, nz // 2, nx // 2 - 1:nx // 2 + 2, ny // 2] = 40.0
+        img[nz // 2 - 2, nx - nx // 3, ny // 2] = 9.0
+    d = [torch.from_numpy(a).cuda() for a in (img, amri, lab)]
+    out = torch.full_like(d[0], -1.0)
+    pct.fuse_device(*d, out, nh, sigma)
+    compare(out.cpu().numpy(), oracle.fuse(img, amri, lab, nh, sigma, 1.0))
+
+    L = _lib.lib()
+    pb = pct.problem(shape, n, nh, sigma, 1.0)
+    least = L.pct_fuse_workspace_size(ctypes.byref(pb), pct.CHOICE_SM)
+    slot = 8 * n * img.size
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def run(nbytes):
+        ws = torch.full((nbytes // 4 + 64,), float("nan"), device="cuda")
+        got = torch.full_like(out, -2.0)
+        rc = L.pct_fuse_dev_ws(ctypes.byref(pb), *(ctypes.c_void_p(t.data_ptr()) for t in d),
+                               ctypes.c_void_p(got.data_ptr()), pct.CHOICE_SM,
+                               ctypes.c_void_p(ws.data_ptr()), nbytes, stream)
+        torch.cuda.synchronize()
+        return rc, got
+
+    for more in sorted({0, 1, 2, parts // 2, parts - 2, parts - 1, parts, 4 * parts}):
+        rc, got = run(least + more * (slot + 256) // 256 * 256)
+        assert rc == 0
+        assert torch.equal(got.view(torch.int32), out.view(torch.int32)), more
+    rc, got = run(least - 256)
+    assert rc == _lib.PCT_ERR_INVALID and bool((got == -2.0).all())
