@@ -120,7 +120,9 @@ int pct_pseudo_ct_host(const pct_problem* pb, const float* img, const float* atl
 /* Device-pointer variant: inputs already resident in HBM, enqueued on
  * `stream`, asynchronous.  Uses a per-device workspace owned by the library
  * (grown on demand; calls that overlap on one device must be ordered on one
- * stream).  No host synchronisation unless the workspace has to grow. */
+ * stream).  No host synchronisation unless the workspace has to grow, which
+ * it cannot while `stream` is recorded into a graph: run the problem, or one
+ * that needs at least pct_fuse_workspace_size() bytes, before. */
 int pct_fuse_dev(const pct_problem* pb, const float* d_img, const float* d_atlas,
                  const float* d_atlas_label_norm, float* d_out, int choice,
                  pct_stream_t stream);

@@ -661,6 +661,8 @@ struct DeviceState {
     bool ok = false;
     void* ws = nullptr;
     size_t ws_bytes = 0;
+    bool recorded = false;       // a graph runs in `ws` in rounds (see fuse_workspace)
+    std::vector<void*> kept;     // such workspaces since outgrown
 };
 
 static std::mutex g_dev_mutex;
@@ -702,7 +704,11 @@ int ensure_workspace(int dev, size_t bytes, void** ptr) {
     if (st.ws_bytes < bytes) {
         if (st.ws) {
             if (hipDeviceSynchronize() != hipSuccess) return PCT_ERR_HIP;
-            (void)hipFree(st.ws);
+            if (st.recorded)
+                st.kept.push_back(st.ws);
+            else
+                (void)hipFree(st.ws);
+            st.recorded = false;
             st.ws = nullptr;
             st.ws_bytes = 0;
         }
@@ -714,6 +720,36 @@ int ensure_workspace(int dev, size_t bytes, void** ptr) {
     }
     *ptr = st.ws;
     return PCT_OK;
+}
+
+// The library's workspace for a fusion that runs in `least` bytes and best in
+// `want`: grown to `want`, or to `least` when that is out of memory.  Nothing grows
+// while the stream is recorded into a graph, so a workspace that earlier calls left
+// between the two is used as it is; it is then kept for the graph when a later call
+// outgrows it, until pct_release.
+static int fuse_workspace(int dev, size_t least, size_t want, hipStream_t stream, void** ptr,
+                          size_t* bytes) {
+    {
+        std::lock_guard<std::mutex> lk(g_dev_mutex);
+        DeviceState& st = g_dev[dev];
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        if (st.ws_bytes >= least && st.ws_bytes < want) {
+            if (hipStreamIsCapturing(stream, &status) != hipSuccess) (void)hipGetLastError();
+            if (status == hipStreamCaptureStatusActive) {
+                st.recorded = true;
+                *ptr = st.ws;
+                *bytes = st.ws_bytes;
+                return PCT_OK;
+            }
+        }
+    }
+    *bytes = want;
+    int rc = ensure_workspace(dev, want, ptr);
+    if (rc == PCT_ERR_NO_MEMORY && least < want) {
+        *bytes = least;
+        rc = ensure_workspace(dev, least, ptr);
+    }
+    return rc;
 }
 
 bool is_xterm_shape(int shape_id) {
@@ -1039,12 +1075,9 @@ static int fuse_dev_impl(const pct_problem* pb, const float* img, const float* a
     TileGeometry g;
     if (!choose(pb, &sid, nullptr, &g)) return PCT_ERR_UNSUPPORTED;
     if (own_ws) {
-        ws_bytes = tiled_ws_bytes(pb, g.n_parts(), sid);
-        rc = ensure_workspace(dev, ws_bytes, &ws);
-        if (rc == PCT_ERR_NO_MEMORY && g.n_split > 1) {
-            ws_bytes = tiled_ws_bytes(pb, g.n_groups, sid);   // of whole windows
-            rc = ensure_workspace(dev, ws_bytes, &ws);
-        }
+        // the partial sums of whole windows at least
+        rc = fuse_workspace(dev, tiled_ws_bytes(pb, g.n_groups, sid),
+                            tiled_ws_bytes(pb, g.n_parts(), sid), stream, &ws, &ws_bytes);
         if (rc) return rc;
     } else if (!ws || ws_bytes < least_ws_bytes(pb) || (reinterpret_cast<uintptr_t>(ws) & 255)) {
         return PCT_ERR_INVALID;
@@ -1581,15 +1614,19 @@ extern "C" void pct_release(void) {
     release_host_buffers();
     std::lock_guard<std::mutex> lk(g_dev_mutex);
     for (auto& kv : g_dev) {
-        if (kv.second.ws) {
+        DeviceState& st = kv.second;
+        if (st.ws) st.kept.push_back(st.ws);
+        if (!st.kept.empty()) {
             int cur = 0;
             (void)hipGetDevice(&cur);
             (void)hipSetDevice(kv.first);
             (void)hipDeviceSynchronize();
-            (void)hipFree(kv.second.ws);
+            for (void* p : st.kept) (void)hipFree(p);
             (void)hipSetDevice(cur);
-            kv.second.ws = nullptr;
-            kv.second.ws_bytes = 0;
         }
+        st.kept.clear();
+        st.ws = nullptr;
+        st.ws_bytes = 0;
+        st.recorded = false;
     }
 }

@@ -74,3 +74,49 @@ def test_any_accepted_workspace_gives_the_same_bits(gpu, shape, n, nh, sigma, fo
         assert torch.equal(got.view(torch.int32), out.view(torch.int32)), more
     rc, got = run(least - 256)
     assert rc == _lib.PCT_ERR_INVALID and bool((got == -2.0).all())
+
+
+def test_graph_in_a_workspace_too_small_for_all_parts(gpu):
+    """A recorded call cannot grow the library's workspace: it runs in what an earlier
+    call left.  Later calls that outgrow it leave the graph its memory."""
+    import torch
+
+    def inputs(shape, n, nh):
+        img, amri, lab = pct.synth_tissue(shape[1], shape[2], shape[0], n, 2, False, nh)
+        pct.normalize_labels(lab)
+        d = [torch.from_numpy(a).cuda() for a in (img, amri, lab)]
+        return d, torch.full_like(d[0], -1.0)
+
+    first, recorded = ((48, 80, 96), 4, 3), ((60, 60, 60), 1, 15)
+    size = [_split(*c, 2.5)[1] * 8 * c[1] * np.prod(c[0]) for c in (first, recorded)]
+    assert _split(*recorded, 2.5)[0] == 1 and 16 * 60 ** 3 <= size[0] < size[1]
+    d1, o1 = inputs(*first)
+    d2, o2 = inputs(*recorded)
+    # the recorded problem's output, in a workspace of the test's own
+    L = _lib.lib()
+    pb = pct.problem(recorded[0], 1, 15, 2.5, 1.0)
+    nbytes = L.pct_fuse_workspace_size(ctypes.byref(pb), pct.CHOICE_SM)
+    ws = torch.empty(nbytes // 4 + 64, device="cuda")
+    want = torch.full_like(o2, -3.0)
+    assert L.pct_fuse_dev_ws(ctypes.byref(pb), *(ctypes.c_void_p(t.data_ptr()) for t in d2),
+                             ctypes.c_void_p(want.data_ptr()), pct.CHOICE_SM,
+                             ctypes.c_void_p(ws.data_ptr()), nbytes,
+                             ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    pct.release()
+    pct.fuse_device(*d1, o1, first[2], 2.5)   # leaves a workspace between the two sizes
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        pct.fuse_device(*d2, o2, recorded[2], 2.5)
+    for replay in range(4):
+        o2.fill_(-2.0)
+        if replay == 2:   # outgrows the workspace; the next calls use the new one
+            grown = torch.full_like(o2, -4.0)
+            pct.fuse_device(*d2, grown, recorded[2], 2.5)
+            pct.fuse_device(*d1, o1, first[2], 2.5)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o2.view(torch.int32), want.view(torch.int32)), replay
+    assert torch.equal(grown.view(torch.int32), want.view(torch.int32))
+    del graph
+    pct.release()
