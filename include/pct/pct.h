@@ -218,7 +218,8 @@ typedef struct pct_subject {
  * uses the library's per-device workspace. */
 int pct_fuse_batch_dev(const pct_subject* subjects, int n_subjects, pct_stream_t stream);
 
-/* Bytes of workspace pct_fuse_batch_dev_ws needs. */
+/* Bytes of workspace pct_fuse_batch_dev_ws needs at most (exactly, for a choice
+ * that was set or autotuned).  No GPU work. */
 size_t pct_fuse_batch_workspace_size(const pct_subject* subjects, int n_subjects);
 
 /* pct_fuse_batch_dev with a caller-provided workspace (256-byte aligned). */

@@ -394,6 +394,11 @@ static std::vector<int> class_groups(const pct_subject* s, int n, int hw) {
     return g;
 }
 
+// Whether the model may give a class a cross-term shape: not at NH 3, where the
+// candidates are too few to pay for the pairs.  Written down because the size of a
+// caller's workspace depends on it.
+static bool may_take_xterm(int hw) { return hw >= 2; }
+
 // Cost model choice per class: the shape with the least pooled time over the
 // subjects of the class, groups of one atlas.  The classes run one after
 // another: on MI355X concurrent class kernels measured slower (six subjects of
@@ -408,6 +413,7 @@ static pct_batch_choice model_choice(const pct_subject* s, int n) {
         if (pbs.empty()) continue;
         double best = -1;
         for (const auto& bk : batch_kernels()) {
+            if (is_xterm_shape(bk.shape_id) && !may_take_xterm(hw)) continue;
             const double cost = model_class_cost(pbs, bk.shape_id, 1);
             if (cost >= 0 && (best < 0 || cost < best * 0.999)) {
                 best = cost;
@@ -419,13 +425,17 @@ static pct_batch_choice model_choice(const pct_subject* s, int n) {
     return ch;
 }
 
+static bool tuned_choice(const pct_subject* s, int n, pct_batch_choice* ch) {
+    std::lock_guard<std::mutex> lk(g_batch_mutex);
+    const auto it = g_batch_tuned.find(shape_signature(s, n));
+    if (it == g_batch_tuned.end()) return false;
+    *ch = it->second;
+    return true;
+}
+
 static pct_batch_choice choose_batch(const pct_subject* s, int n) {
-    {
-        std::lock_guard<std::mutex> lk(g_batch_mutex);
-        auto it = g_batch_tuned.find(shape_signature(s, n));
-        if (it != g_batch_tuned.end()) return it->second;
-    }
-    return model_choice(s, n);
+    pct_batch_choice ch;
+    return tuned_choice(s, n, &ch) ? ch : model_choice(s, n);
 }
 
 static void destroy_graph(CachedGraph& g) {
@@ -537,10 +547,22 @@ using namespace pct;
 
 extern "C" size_t pct_fuse_batch_workspace_size(const pct_subject* subjects, int n_subjects) {
     if (validate_batch(subjects, n_subjects)) return 0;
-    (void)check_device(nullptr);   // so that the call that follows chooses the same
     BatchPlan p;
-    if (!plan_batch(subjects, n_subjects, choose_batch(subjects, n_subjects), &p)) return 0;
-    return p.ws_bytes;
+    pct_batch_choice ch;
+    const bool tuned = tuned_choice(subjects, n_subjects, &ch);
+    if (!tuned) ch = model_choice(subjects, n_subjects);
+    if (!plan_batch(subjects, n_subjects, ch, &p)) return 0;
+    if (tuned) return p.ws_bytes;
+    // What the model picks depends on the device (the kernels' occupancy): enough
+    // for either form, without touching one.
+    size_t bytes = kQueueBytes;
+    for (int i = 0; i < n_subjects; ++i) {
+        const pct_problem& pb = subjects[i].pb;
+        if (!tiled_window(pb)) continue;
+        const size_t sums = tiled_le_offset(&pb, pb.n_atlas);   // as many bytes as pairs
+        bytes += may_take_xterm(class_of(pb)) ? 2 * sums : sums;
+    }
+    return bytes;
 }
 
 extern "C" int pct_fuse_batch_dev(const pct_subject* subjects, int n_subjects,

@@ -54,6 +54,11 @@ assert L.pct_device_count() == 0 and shim.hip_calls() == 1   # the stand-ins are
 for choice in (0, 1, 2):
     assert L.pct_fuse_workspace_size(ctypes.byref(pb), choice) >= 0
 assert L.pct_fuse_workspace_size(ctypes.byref(pb), 2) > 0
+subjects = (_lib.Subject * 2)()
+for s, nh in zip(subjects, (5, 9)):
+    s.pb = _lib.Problem(nx=40, ny=50, nz=30, n_atlas=2, nh=nh, patch=3, sigma=2.5, beta=1.0, div=0.0)
+    s.d_img = s.d_atlas = s.d_atlas_label_norm = s.d_out = 256
+assert L.pct_fuse_batch_workspace_size(subjects, 2) > 0
 print("calls", shim.hip_calls() - 1)
 """
 
