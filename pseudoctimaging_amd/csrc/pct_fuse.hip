@@ -722,18 +722,18 @@ int ensure_workspace(int dev, size_t bytes, void** ptr) {
     return PCT_OK;
 }
 
-// The library's workspace for a fusion that runs in `least` bytes and best in
-// `want`: grown to `want`, or to `least` when that is out of memory.  Nothing grows
-// while the stream is recorded into a graph, so a workspace that earlier calls left
+// The library's workspace for a fusion that runs in sizes.back() bytes and best in
+// sizes[0]: grown to the first of them that there is memory for.  Nothing grows while
+// the stream is recorded into a graph, so a workspace that earlier calls left
 // between the two is used as it is; it is then kept for the graph when a later call
 // outgrows it, until pct_release.
-static int fuse_workspace(int dev, size_t least, size_t want, hipStream_t stream, void** ptr,
-                          size_t* bytes) {
+static int fuse_workspace(int dev, const std::vector<size_t>& sizes, hipStream_t stream,
+                          void** ptr, size_t* bytes) {
     {
         std::lock_guard<std::mutex> lk(g_dev_mutex);
         DeviceState& st = g_dev[dev];
         hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-        if (st.ws_bytes >= least && st.ws_bytes < want) {
+        if (st.ws_bytes >= sizes.back() && st.ws_bytes < sizes[0]) {
             if (hipStreamIsCapturing(stream, &status) != hipSuccess) (void)hipGetLastError();
             if (status == hipStreamCaptureStatusActive) {
                 st.recorded = true;
@@ -743,11 +743,10 @@ static int fuse_workspace(int dev, size_t least, size_t want, hipStream_t stream
             }
         }
     }
-    *bytes = want;
-    int rc = ensure_workspace(dev, want, ptr);
-    if (rc == PCT_ERR_NO_MEMORY && least < want) {
-        *bytes = least;
-        rc = ensure_workspace(dev, least, ptr);
+    int rc = PCT_ERR_NO_MEMORY;
+    for (size_t k = 0; k < sizes.size() && rc == PCT_ERR_NO_MEMORY; ++k) {
+        *bytes = sizes[k];
+        rc = ensure_workspace(dev, sizes[k], ptr);
     }
     return rc;
 }
@@ -781,6 +780,18 @@ static size_t least_ws_bytes(const pct_problem* pb) {
     TileGeometry g;
     if (!make_geometry(pb, c.shape_id, c.group, &g)) return 0;
     return tiled_ws_bytes(pb, g.n_groups, c.shape_id);
+}
+
+// Workspaces that the geometry can run in: with all partial sums in memory, with
+// those of whole windows, with one.
+static std::vector<size_t> workspace_sizes(const pct_problem* pb, int shape_id,
+                                           const TileGeometry& g) {
+    std::vector<size_t> v;
+    for (int slots : {g.n_parts(), g.n_groups, 1}) {
+        const size_t bytes = tiled_ws_bytes(pb, slots, shape_id);
+        if (v.empty() || bytes < v.back()) v.push_back(bytes);
+    }
+    return v;
 }
 
 // Lets the geometry keep as many partial sums as fit `bytes`; false where not one does.
@@ -1075,9 +1086,7 @@ static int fuse_dev_impl(const pct_problem* pb, const float* img, const float* a
     TileGeometry g;
     if (!choose(pb, &sid, nullptr, &g)) return PCT_ERR_UNSUPPORTED;
     if (own_ws) {
-        // the partial sums of whole windows at least
-        rc = fuse_workspace(dev, tiled_ws_bytes(pb, g.n_groups, sid),
-                            tiled_ws_bytes(pb, g.n_parts(), sid), stream, &ws, &ws_bytes);
+        rc = fuse_workspace(dev, workspace_sizes(pb, sid, g), stream, &ws, &ws_bytes);
         if (rc) return rc;
     } else if (!ws || ws_bytes < least_ws_bytes(pb) || (reinterpret_cast<uintptr_t>(ws) & 255)) {
         return PCT_ERR_INVALID;
@@ -1383,13 +1392,12 @@ static int fuse_host_impl(const pct_problem* pb, const float* img, const float* 
     {
         const size_t post_need =
             std::max<size_t>(post ? postprocess_ws_bytes(pb->nh, pb->nx, pb->ny, pb->nz) : 0, 256);
-        auto need = [&]() {
-            return tiled ? std::max(post_need, tiled_ws_bytes(pb, g.n_slots(), sid)) : post_need;
-        };
-        rc = host_workspace(st, need(), &ws);
-        if (rc == PCT_ERR_NO_MEMORY && tiled && g.n_split > 1) {
-            g.slots = g.n_groups;   // the partial sums of whole windows
-            rc = host_workspace(st, need(), &ws);
+        std::vector<size_t> sizes = {post_need};
+        if (tiled) sizes = workspace_sizes(pb, sid, g);
+        rc = PCT_ERR_NO_MEMORY;
+        for (size_t k = 0; k < sizes.size() && rc == PCT_ERR_NO_MEMORY; ++k) {
+            rc = host_workspace(st, std::max(post_need, sizes[k]), &ws);
+            if (!rc && tiled) fit_slots(pb, sid, sizes[k], &g);
         }
     }
     f32x2* le = tiled && is_xterm_shape(sid)
@@ -1569,6 +1577,10 @@ extern "C" int pct_autotune(const pct_problem* pb, const float* d_img, const flo
             void* ws = nullptr;
             const size_t need = tiled_ws_bytes(pb, g.n_parts(), sid);
             rc = ensure_workspace(dev, need, &ws);
+            if (rc == PCT_ERR_NO_MEMORY && t.split > 1) {
+                rc = PCT_OK;   // the shape's other candidates need less
+                continue;
+            }
             if (rc) break;
             // warm-up
             rc = launch_tiled(pb, d_img, d_atlas, d_label, d_out, ws, need, sid, g, s);

@@ -25,6 +25,8 @@ def _split(shape, n, nh, sigma):
     iz, ix, iy = (m - 2 * r for m in shape)
     tiles = -(-iz // c["bz"]) * -(-ix // (c["waves"] * (64 // c["seg_width"]) * c["bx"])) * \
         -(-iy // (c["seg_width"] - 2))
+    if tiles <= 0:   # no interior
+        return c["form"], 1
     assert c["items"] % (tiles * n) == 0
     return c["form"], c["items"] // (tiles * n)
 
@@ -76,7 +78,11 @@ def test_any_accepted_workspace_gives_the_same_bits(gpu, shape, n, nh, sigma, fo
     assert rc == _lib.PCT_ERR_INVALID and bool((got == -2.0).all())
 
 
-def test_graph_in_a_workspace_too_small_for_all_parts(gpu):
+# volume, atlases, NH of a call, and of one that is recorded in the workspace it left:
+# more than whole windows' sums of the second, and less (but more than one sum)
+@pytest.mark.parametrize("first,recorded", [(((48, 80, 96), 4, 3), ((60, 60, 60), 1, 15)),
+                                            (((4, 60, 60), 1, 3), ((24, 31, 12), 4, 9))])
+def test_graph_in_a_workspace_too_small_for_all_parts(gpu, first, recorded):
     """A recorded call cannot grow the library's workspace: it runs in what an earlier
     call left.  Later calls that outgrow it leave the graph its memory."""
     import torch
@@ -87,14 +93,17 @@ def test_graph_in_a_workspace_too_small_for_all_parts(gpu):
         d = [torch.from_numpy(a).cuda() for a in (img, amri, lab)]
         return d, torch.full_like(d[0], -1.0)
 
-    first, recorded = ((48, 80, 96), 4, 3), ((60, 60, 60), 1, 15)
-    size = [_split(*c, 2.5)[1] * 8 * c[1] * np.prod(c[0]) for c in (first, recorded)]
-    assert _split(*recorded, 2.5)[0] == 1 and 16 * 60 ** 3 <= size[0] < size[1]
+    assert _split(*first, 2.5) == (0, 1)
+    left = 8 * first[1] * int(np.prod(first[0]))
+    form, parts = _split(*recorded, 2.5)
+    volume = 8 * int(np.prod(recorded[0]))
+    pairs = form * recorded[1] * volume
+    assert volume + pairs < left < parts * recorded[1] * volume + pairs
     d1, o1 = inputs(*first)
     d2, o2 = inputs(*recorded)
     # the recorded problem's output, in a workspace of the test's own
     L = _lib.lib()
-    pb = pct.problem(recorded[0], 1, 15, 2.5, 1.0)
+    pb = pct.problem(*recorded, 2.5, 1.0)
     nbytes = L.pct_fuse_workspace_size(ctypes.byref(pb), pct.CHOICE_SM)
     ws = torch.empty(nbytes // 4 + 64, device="cuda")
     want = torch.full_like(o2, -3.0)
