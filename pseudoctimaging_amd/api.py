@@ -171,9 +171,10 @@ def normalize_labels_device(label, stream=None) -> None:
           "pct_normalize_labels_dev")
 
 
-def tile_config(shape, n_atlas: int, nh: int) -> dict:
-    """The tiled-kernel configuration the library would use (no GPU work)."""
-    pb = problem(shape, n_atlas, nh)
+def tile_config(shape, n_atlas: int, nh: int, sigma: float = 1.0, beta: float = 1.0) -> dict:
+    """The tiled-kernel configuration the library would use at this sigma and
+    beta (a small divisor rules the cross-term kernels out); no GPU work."""
+    pb = problem(shape, n_atlas, nh, sigma, beta)
     cfg = TileConfig()
     check(lib().pct_tile_config_choose(byref(pb), byref(cfg)), "pct_tile_config_choose")
     return cfg.as_dict()

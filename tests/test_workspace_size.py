@@ -37,6 +37,12 @@ def test_size_grows_with_the_problem(nh, sigma):
         assert s <= 16 * voxels + 512
 
 
+def test_configuration_depends_on_the_divisor():
+    shape = (112, 222, 222)
+    forms = [pct.tile_config(shape, 10, 11, *s)["form"] for s in ((), (2.5, 1.0), (0.3, 1.0))]
+    assert forms == [1, 1, 0]
+
+
 SHIM = """
 static int calls;
 int hipGetDevice(int* d) { ++calls; *d = 0; return 100; }
