@@ -936,8 +936,8 @@ TimedLaunch::~TimedLaunch() {
 // item goes on from.  The partial sums are added one after another in the order of
 // the finalize pass, so the output has the same bits as with all of them in memory.
 // In the least workspace 30x34x22, n = 2, NH = 7 takes 95 us (15 with all 14 parts in
-// memory), 60x60x60, n = 1, NH = 15 473 us (127), 96x96x64, n = 4, NH = 11 629 us; items of
-// whole windows in the same memory took 83, 498 and 799.
+// memory), 60x60x60, n = 1, NH = 15 473 us (127) and 40x66x30, n = 3, NH = 9 129 us (45);
+// items of whole windows in the same memory took 83, 498 and 151.
 static int launch_rounds(const TiledArgs& all, const TileGeometry& g, int shape_id,
                          hipStream_t stream) {
     const int groups = std::max(1, g.slots / g.n_split);   // a launch

@@ -157,14 +157,17 @@ __device__ __forceinline__ float neighbourhood_median(const float* arr, int id, 
 // workgroup barrier after each.  A tile is handed out only after all tiles it
 // waits for, to workgroups that are already running, so every wait ends.
 //
-// What bounds it is the chain of levels a value travels through (1108 at
-// 222x222x112) and, per tile on that chain, one hand-over between workgroups
-// (flag, LDS copy).  Hence small tiles, eight lanes to a voxel (about 130
-// instructions to a median instead of 900 for one lane sorting 27 values), and
-// an LDS copy that starts before the wait with what no tile before it changes.
-// A level takes about 810 cycles, the copy after the wait 1900, the release
-// 1700.  222x222x112 with 4.2e6 NaN voxels: 48.2 ms for the one-workgroup sweep
-// (46 us a level), 1.56 ms here, 1.52 of it in fill_tiles_kernel.  Tiles of
+// What bounds it is the chain of tiles: a tile starts when all levels of the ones
+// before it are done, so its kTileLevels levels and one hand-over between workgroups
+// (flag, LDS copy) come once per diagonal (at 222x222x112, NH = 3: 107 diagonals of
+// up to 213 tiles, 2782 levels in a row where the volume has 1080).  Hence small
+// tiles, eight lanes to a voxel (about 130 instructions to a median instead of 900
+// for one lane sorting 27 values), and an LDS copy that starts before the wait with
+// what no tile before it changes.  222x222x112 with 4.2e6 NaN voxels: 48.2 ms for
+// the one-workgroup sweep (45 us a level), 1.53 ms here, 1.50 of it in
+// fill_tiles_kernel: 14 us a diagonal.  Of those 34000 cycles the levels take 21000
+// (810 each), the copy after the wait 1900 and the release 1700; what the other
+// 9000 go to has not been measured.  Tiles of
 // {4, 8, 32} took 2.7 ms (before the early copy), {4, 8, 8} 2.04, {8, 8, 8}
 // 2.22, {4, 16, 8} 2.56; 512 workgroups 1.70.  Polling with acquire loads,
 // which invalidate the caches each time, took 4.6-6.2 ms.
