@@ -612,9 +612,8 @@ static Config model_choice(const pct_problem* pb, bool xt, bool* known) {
     return best;
 }
 
-// The forced or tuned configuration of a problem, if there is one.
+// The forced or tuned configuration of a problem, if there is one (g_cfg_mutex held).
 static bool fixed_config(const pct_problem* pb, Config* c) {
-    std::lock_guard<std::mutex> lk(g_cfg_mutex);
     if (g_forced_id >= 0) {
         *c = Config{g_forced_id, g_forced_group > 0 ? g_forced_group : 1, 1};
         return true;
@@ -628,20 +627,22 @@ static bool fixed_config(const pct_problem* pb, Config* c) {
 // The configuration of a problem: forced, tuned, or the model's.
 static bool choose(const pct_problem* pb, int* shape_id, double* cost, TileGeometry* geo) {
     Config c;
-    if (!fixed_config(pb, &c)) {
-        const bool xt = may_take_xterm(pb);
-        const auto key =
-            std::make_pair(ShapeKey{pb->nx, pb->ny, pb->nz, pb->n_atlas, pb->nh}, xt);
+    {
         std::lock_guard<std::mutex> lk(g_cfg_mutex);
-        const auto pl = g_planned.find(key);
-        if (pl != g_planned.end()) {
-            c = pl->second;
-        } else {
-            bool known = false;   // whether a device's occupancy went into it
-            c = model_choice(pb, xt, &known);
-            if (known) {
-                if (g_planned.size() >= kPlanned) g_planned.clear();
-                g_planned.emplace(key, c);
+        if (!fixed_config(pb, &c)) {
+            const bool xt = may_take_xterm(pb);
+            const auto key =
+                std::make_pair(ShapeKey{pb->nx, pb->ny, pb->nz, pb->n_atlas, pb->nh}, xt);
+            const auto pl = g_planned.find(key);
+            if (pl != g_planned.end()) {
+                c = pl->second;
+            } else {
+                bool known = false;   // whether a device's occupancy went into it
+                c = model_choice(pb, xt, &known);
+                if (known) {
+                    if (g_planned.size() >= kPlanned) g_planned.clear();
+                    g_planned.emplace(key, c);
+                }
             }
         }
     }
@@ -722,35 +723,6 @@ int ensure_workspace(int dev, size_t bytes, void** ptr) {
     return PCT_OK;
 }
 
-// The library's workspace for a fusion that runs in sizes.back() bytes and best in
-// sizes[0]: grown to the first of them that there is memory for.  Nothing grows while
-// the stream is recorded into a graph, so a workspace that earlier calls left
-// between the two is used as it is; it is then kept for the graph when a later call
-// outgrows it, until pct_release.
-static int fuse_workspace(int dev, const std::vector<size_t>& sizes, hipStream_t stream,
-                          void** ptr, size_t* bytes) {
-    {
-        std::lock_guard<std::mutex> lk(g_dev_mutex);
-        DeviceState& st = g_dev[dev];
-        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-        if (st.ws_bytes >= sizes.back() && st.ws_bytes < sizes[0]) {
-            if (hipStreamIsCapturing(stream, &status) != hipSuccess) (void)hipGetLastError();
-            if (status == hipStreamCaptureStatusActive) {
-                st.recorded = true;
-                *ptr = st.ws;
-                *bytes = st.ws_bytes;
-                return PCT_OK;
-            }
-        }
-    }
-    int rc = PCT_ERR_NO_MEMORY;
-    for (size_t k = 0; k < sizes.size() && rc == PCT_ERR_NO_MEMORY; ++k) {
-        *bytes = sizes[k];
-        rc = ensure_workspace(dev, sizes[k], ptr);
-    }
-    return rc;
-}
-
 bool is_xterm_shape(int shape_id) {
     return shape_id >= 0 && shape_id < (int)shapes().size() && shapes()[shape_id].form == 1;
 }
@@ -775,7 +747,10 @@ size_t tiled_ws_bytes(const pct_problem* pb, int n_slots, int shape_id) {
 // grows with every extent and the atlases, and touches no GPU.
 static size_t least_ws_bytes(const pct_problem* pb) {
     Config c;
-    if (!fixed_config(pb, &c))
+    std::unique_lock<std::mutex> lk(g_cfg_mutex);
+    const bool fixed = fixed_config(pb, &c);
+    lk.unlock();
+    if (!fixed)
         return tiled_le_offset(pb, pb->n_atlas) + (may_take_xterm(pb) ? pairs_bytes(pb) : 0);
     TileGeometry g;
     if (!make_geometry(pb, c.shape_id, c.group, &g)) return 0;
@@ -792,6 +767,37 @@ static std::vector<size_t> workspace_sizes(const pct_problem* pb, int shape_id,
         if (v.empty() || bytes < v.back()) v.push_back(bytes);
     }
     return v;
+}
+
+// The library's workspace for a fusion: grown to the first of workspace_sizes that
+// there is memory for.  Nothing grows while the stream is recorded into a graph, so a
+// workspace that earlier calls left between them is used as it is; it is then kept
+// for the graph when a later call outgrows it, until pct_release.
+static int fuse_workspace(int dev, const pct_problem* pb, int shape_id, const TileGeometry& g,
+                          hipStream_t stream, void** ptr, size_t* bytes) {
+    std::vector<size_t> sizes;
+    {
+        std::lock_guard<std::mutex> lk(g_dev_mutex);
+        DeviceState& st = g_dev[dev];
+        *ptr = st.ws;
+        *bytes = st.ws_bytes;
+        if (st.ws_bytes >= tiled_ws_bytes(pb, g.n_parts(), shape_id)) return PCT_OK;
+        sizes = workspace_sizes(pb, shape_id, g);
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        if (st.ws_bytes >= sizes.back()) {
+            if (hipStreamIsCapturing(stream, &status) != hipSuccess) (void)hipGetLastError();
+            if (status == hipStreamCaptureStatusActive) {
+                st.recorded = true;
+                return PCT_OK;
+            }
+        }
+    }
+    int rc = PCT_ERR_NO_MEMORY;
+    for (size_t k = 0; k < sizes.size() && rc == PCT_ERR_NO_MEMORY; ++k) {
+        *bytes = sizes[k];
+        rc = ensure_workspace(dev, sizes[k], ptr);
+    }
+    return rc;
 }
 
 // Lets the geometry keep as many partial sums as fit `bytes`; false where not one does.
@@ -1086,7 +1092,7 @@ static int fuse_dev_impl(const pct_problem* pb, const float* img, const float* a
     TileGeometry g;
     if (!choose(pb, &sid, nullptr, &g)) return PCT_ERR_UNSUPPORTED;
     if (own_ws) {
-        rc = fuse_workspace(dev, workspace_sizes(pb, sid, g), stream, &ws, &ws_bytes);
+        rc = fuse_workspace(dev, pb, sid, g, stream, &ws, &ws_bytes);
         if (rc) return rc;
     } else if (!ws || ws_bytes < least_ws_bytes(pb) || (reinterpret_cast<uintptr_t>(ws) & 255)) {
         return PCT_ERR_INVALID;
