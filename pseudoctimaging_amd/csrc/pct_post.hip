@@ -164,8 +164,8 @@ __device__ __forceinline__ float neighbourhood_median(const float* arr, int id, 
 // tiles, eight lanes to a voxel (about 130 instructions to a median instead of 900
 // for one lane sorting 27 values), and an LDS copy that starts before the wait with
 // what no tile before it changes.  222x222x112 with 4.2e6 NaN voxels: 48.2 ms for
-// the one-workgroup sweep (45 us a level), 1.53 ms here, 1.50 of it in
-// fill_tiles_kernel: 14 us a diagonal.  Of those 34000 cycles the levels take 21000
+// the one-workgroup sweep (45 us a level), 1.53 ms here, 1.48 of it in
+// fill_tiles_kernel: 14 us a diagonal.  Of those 33000 cycles the levels take 21000
 // (810 each), the copy after the wait 1900 and the release 1700; what the other
 // 9000 go to has not been measured.  Tiles of
 // {4, 8, 32} took 2.7 ms (before the early copy), {4, 8, 8} 2.04, {8, 8, 8}
